@@ -115,6 +115,8 @@ struct FitHost {
   size_t o_pcur, o_chi2c, o_pstp, o_ncnt, o_nacpt, o_nhist, o_nexch, o_sumh, o_tcur, o_flag, o_ptent, o_ptentn;
   size_t o_pout, o_tout, o_chi2, o_datm, o_chi2m, o_mc;
   size_t o_pcur_b = 0, o_chi2c_b = 0, o_tcur_b = 0;   // second state set (xfused)
+  int ulanes = 0;                // model.cuh path: lanes per chain (user_lanes)
+  bool useq = false;             // model.cuh path: whole sequences per wave (k_iter_user)
   bool xfused = false;           // exchange inside the next step launch (FitDesc::xfused)
   bool hwphase = false;          // FitDesc::hwphase
   bool has_datm = false;
@@ -432,6 +434,42 @@ bool eht_xfused(const FitHost& h, const MhreOptions& o) {
   return (h.kind == K_SGRA9 || h.kind == K_SGRA13) && h.s.nbeta <= 64 && o.exchange_launch == 0;
 }
 
+// The model.cuh path's split of a fit over lanes (FitHost::ulanes, useq).
+//
+// k_iter_user keeps a whole ladder of at most 64 rungs in a wave, so a chain
+// has at most 64 / xlanes lanes there, for its data and its nprm random draws;
+// it saves both launches of every iteration.  It is taken while a lane has at
+// most USER_SEQ_DATA data.  Beyond that, and for longer ladders, k_step_user
+// gives a chain up to 256 lanes: as many as it has data, but no more waves
+// than fill the chip several times over (a wave of fewer chains repeats their
+// bookkeeping on more lanes).
+constexpr int USER_SEQ_DATA = 4;
+constexpr long long USER_WAVES = 8192;
+constexpr int USER_SEQ_LDS = 32 << 10;
+
+int pow2_at_least(int n) {
+  int p = 1;
+  while (p < n) p <<= 1;
+  return p;
+}
+
+void user_lanes(FitHost& h) {
+  const MhreFitSpec& s = h.s;
+  h.useq = false;
+  if (s.nbeta <= 64) {
+    int n = 64 / exchange_lanes(s.nbeta);
+    n = std::min(n, pow2_at_least(std::max(s.ndat, s.nprm)));
+    if (s.ndat <= USER_SEQ_DATA * n && 64 / n * user_slot_bytes(s.nprm, s.nptot) <= USER_SEQ_LDS) {
+      h.useq = true;
+      h.ulanes = n;
+      return;
+    }
+  }
+  int n = std::max(8, std::min(256, pow2_at_least(s.ndat)));
+  while (n > 8 && (long long)s.nbeta * s.nseq * n > 64 * USER_WAVES) n >>= 1;
+  h.ulanes = n;
+}
+
 // Most concurrent sequence groups (streams) of a session.
 constexpr int MAX_GROUPS = 8;
 
@@ -473,8 +511,11 @@ void unpack_hist(const std::vector<uint32_t>& bits, int nadj, int P, int C, int*
 struct KindWork {
   int kind;
   int quad_n;
-  bool fused = false;   // quadratic systems: step and exchange in one launch, items (fit, first sequence)
+  bool fused = false;   // step and exchange of whole sequences in one launch, items (fit, first sequence)
   bool rows = false;    // fused quadratic systems: every fit has single-coordinate update rows
+  bool one = false;     // fused model.cuh fits: no chain has more data than lanes
+  int ulanes = 0;       // model.cuh path: lanes per chain
+  int max_prm = 0, max_tot = 0;   // model.cuh path: largest nprm, nptot
   std::vector<WorkItem> step, eval;
   XcdRanges xr{};   // wave-per-chain kinds: step list dealt into per-XCD ranges
   WorkItem* d_step = nullptr;
@@ -711,6 +752,10 @@ StepLaunch make_launch(Session* S, const Group& g, const KindWork& k, int it_off
   L.qslot = k.qslot;
   L.waves_per_simd = S->waves_per_simd;
   L.lds_per_cu = S->lds_per_cu;
+  L.iters = 1;
+  L.ulanes = k.ulanes;
+  L.max_prm = k.max_prm;
+  L.max_tot = k.max_tot;
   L.tr_dec = S->d_tr_dec;
   L.tr_chi2 = S->d_tr_chi2;
   L.tr_ex = S->d_tr_ex;
@@ -732,11 +777,24 @@ StepLaunch exchange_launch(Session* S, const Group& g, int it_off, int close_k) 
   return L;
 }
 
-// The step launches of group g at offset i of its segment.
-int launch_steps(Session* S, const Group& g, int i) {
+// Most iterations of one launch of whole sequences: long enough to hide the
+// launch, short enough that the waves of a session of many fits, which take
+// several rounds of the chip, do not drift far apart.
+constexpr int SEQ_ITERS = 64;
+
+// The step launches of group g at offset i of its segment.  Kinds whose
+// launches hold whole sequences run iterations i .. i + n - 1 (n = 0: none,
+// an earlier launch has them).
+int launch_steps(Session* S, const Group& g, int i, int n) {
   for (const KindWork& k : g.kinds) {
-    const StepLaunch L = make_launch(S, g, k, i);
+    StepLaunch L = make_launch(S, g, k, i);
     hipError_t e = hipSuccess;
+    if (k.kind == K_USER && k.fused) {
+      if (n == 0) continue;
+      L.iters = n;
+      HIPCHK(launch_iter_user(k.one, L, g.stream));
+      continue;
+    }
     if (k.kind == K_SGRA9) e = launch_step_eht(MODEL_SGRA9, L, g.stream);
     else if (k.kind == K_SGRA13) e = launch_step_eht(MODEL_SGRA13, L, g.stream);
     else if (k.kind == K_QUAD && k.fused) e = launch_iter_quad(k.quad_n, k.rows, L, g.stream);
@@ -754,10 +812,10 @@ int launch_group_exchange(Session* S, const Group& g, int i) {
   return MHRE_OK;
 }
 
-// Offset i of group g's segment on its stream: the step launches, then the
-// exchange launch of the sequences that need one.
-int launch_iteration(Session* S, const Group& g, int i) {
-  CHK(launch_steps(S, g, i));
+// Offset i of group g's segment of K iterations on its stream: the step
+// launches, then the exchange launch of the sequences that need one.
+int launch_iteration(Session* S, const Group& g, int i, int K) {
+  CHK(launch_steps(S, g, i, i % SEQ_ITERS == 0 ? std::min(SEQ_ITERS, K - i) : 0));
   return launch_group_exchange(S, g, i);
 }
 
@@ -771,7 +829,7 @@ int close_segment(Session* S, const Group& g, int K) {
 // A segment of K iterations of every group, the groups' launches interleaved.
 int launch_segment(Session* S, int K) {
   for (int i = 0; i < K; ++i)
-    for (const Group& g : S->groups) CHK(launch_iteration(S, g, i));
+    for (const Group& g : S->groups) CHK(launch_iteration(S, g, i, K));
   for (const Group& g : S->groups) CHK(close_segment(S, g, K));
   return MHRE_OK;
 }
@@ -819,7 +877,7 @@ int time_kernels(Session* S, int niter, double* step_ms, double* exch_ms) {
         const Group& g = S->groups[gi];
         hipEvent_t* e = &ev[(size_t)3 * (i * G + gi)];
         HIPCHK(hipEventRecord(e[0], g.stream));
-        CHK(launch_steps(S, g, i));
+        CHK(launch_steps(S, g, i, 1));
         HIPCHK(hipEventRecord(e[1], g.stream));
         CHK(launch_group_exchange(S, g, i));
         HIPCHK(hipEventRecord(e[2], g.stream));
@@ -963,6 +1021,7 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
     if (h.kind == K_SGRA9 || h.kind == K_SGRA13) CHK(pack_eht(h, i));
     if (h.kind == K_QUAD) CHK(pack_quad(h, i));
     if (h.kind == K_USER && h.s.npass <= 0) FAIL(MHRE_EINVAL, "fit %d: npass must be positive", i);
+    if (h.kind == K_USER) user_lanes(h);
     const MhreFitSpec& s = h.s;
     const size_t C = (size_t)h.nchain, P = (size_t)s.nprm, N = (size_t)s.nptot;
     h.o_vis = A.reserve<float>(h.vis.size());
@@ -1080,6 +1139,7 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
     d.n_cnt = at<int>(S, h.o_ncnt); d.n_acpt = at<int>(S, h.o_nacpt); d.hbits = at<uint32_t>(S, h.o_nhist);
     d.hwords = hist_words(s.nadj);
     d.xlanes = exchange_lanes(s.nbeta);
+    d.ulanes = h.ulanes;
     d.n_exch = at<int>(S, h.o_nexch); d.sumh = at<int>(S, h.o_sumh); d.tcur = at<int>(S, h.o_tcur);
     d.flag = at<int>(S, h.o_flag); d.ptent = at<float>(S, h.o_ptent); d.ptentn = at<int>(S, h.o_ptentn);
     d.xfused = h.xfused ? 1 : 0;
@@ -1265,18 +1325,47 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
         }
         continue;
       }
+      if (kk == K_USER) {
+        // model.cuh path: one launch per number of lanes per chain; whole
+        // sequences (items: the fit and the wave's first sequence), or single
+        // chains, every wave holding chains of one fit
+        for (bool fused : {true, false}) {
+          for (int n = 1; n <= 256; n <<= 1) {
+            KindWork kone, kw;
+            kone.kind = kw.kind = kk;
+            kone.ulanes = kw.ulanes = n;
+            kone.fused = kw.fused = fused;
+            kone.one = true;
+            for (int i : idx) {
+              const FitHost& h = S->fits[i];
+              if (h.useq != fused || h.ulanes != n) continue;
+              KindWork& k = fused && h.s.ndat <= n ? kone : kw;
+              k.max_prm = std::max(k.max_prm, h.s.nprm);
+              k.max_tot = std::max(k.max_tot, h.s.nptot);
+              if (fused) {
+                int s0, s1;
+                seq_range(i, g, &s0, &s1);
+                const int per = 64 / (exchange_lanes(h.s.nbeta) * n);
+                for (int q = s0; q < s1; q += per) k.step.push_back({i, q});
+                continue;
+              }
+              const size_t before = k.step.size();
+              chains(i, k.step);
+              if (k.step.size() > before)
+                while (n < 64 && k.step.size() % (64 / n)) k.step.push_back({i, -1});
+            }
+            if (!kone.step.empty()) grp.kinds.push_back(std::move(kone));
+            if (!kw.step.empty()) grp.kinds.push_back(std::move(kw));
+          }
+        }
+        continue;
+      }
       KindWork kw;
       kw.kind = kk;
       kw.qslot = qslot++;
-      for (int i : idx) {
-        const size_t before = kw.step.size();
-        chains(i, kw.step);
-        // lane-per-chain kernels: every wave holds chains of one fit
-        if (kk == K_USER && kw.step.size() > before)
-          while (kw.step.size() % 64) kw.step.push_back({i, -1});
-      }
+      for (int i : idx) chains(i, kw.step);
       if (kw.step.empty()) continue;
-      if (kk != K_USER) kw.xr = deal_xcd(kw.step, fit_cost);
+      kw.xr = deal_xcd(kw.step, fit_cost);
       grp.kinds.push_back(std::move(kw));
     }
     // exchange lists, heaviest fits first, dealt like the step lists; one
@@ -1285,7 +1374,7 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
     // xfused sequences (their segment's closing launch finishes them).
     std::vector<WorkItem> xw, xc;
     for (int i : xorder) {
-      if (quad_fused(S->fits[i])) continue;   // exchanged inside its step launch
+      if (quad_fused(S->fits[i]) || S->fits[i].useq) continue;   // exchanged inside its step launch
       const int per = 64 / exchange_lanes(S->fits[i].s.nbeta);
       int s0, s1;
       seq_range(i, g, &s0, &s1);
@@ -1396,7 +1485,7 @@ int run(Session* S, int niter) {
       if (grp.gexec) continue;
       HIPCHK(hipStreamBeginCapture(grp.stream, hipStreamCaptureModeThreadLocal));
       int rc = MHRE_OK;
-      for (int i = 0; i < G && rc == MHRE_OK; ++i) rc = launch_iteration(S, grp, i);
+      for (int i = 0; i < G && rc == MHRE_OK; ++i) rc = launch_iteration(S, grp, i, G);
       if (rc == MHRE_OK) rc = close_segment(S, grp, G);
       hipGraph_t g = nullptr;
       const hipError_t ec = hipStreamEndCapture(grp.stream, &g);
@@ -1845,7 +1934,7 @@ int mhre_session_fit_info(const void* session, int fit, int* info, int ninfo) {
   if (fit < 0 || fit >= (int)S->fits.size()) FAIL(MHRE_EINVAL, "mhre_session_fit_info: no fit %d", fit);
   const FitHost& h = S->fits[fit];
   info[0] = h.kind;
-  info[1] = (h.xfused || quad_fused(h)) ? 1 : 0;
+  info[1] = (h.xfused || quad_fused(h) || h.useq) ? 1 : 0;
   info[2] = h.hwphase ? 1 : 0;
   info[3] = (int)S->groups.size();
   if (ninfo >= 5) info[4] = h.qrow.empty() ? 0 : 1;

@@ -66,6 +66,9 @@ struct StepLaunch {
   int qslot;             // RunClock::qhead slot of the persistent form
   int waves_per_simd;    // > 0: cap on resident waves per SIMD (LDS reserved per work-group)
   int lds_per_cu;        // bytes of LDS per compute unit
+  int iters;             // launches that hold whole sequences: iterations it_off .. it_off + iters - 1
+  int ulanes;            // model.cuh path: lanes per chain of the list's fits
+  int max_prm, max_tot;  // model.cuh path: largest nprm and nptot of the list's fits
   int* tr_dec; float* tr_chi2; int* tr_ex; int tr_it0; int tr_nit;   // optional decision trace
 };
 
@@ -89,6 +92,12 @@ hipError_t launch_exchange(const StepLaunch& L, const WorkItem* xwork, const Xcd
 hipError_t launch_eval_user(const FitDesc* fits, const WorkItem* work, int nwork, int model_only,
                             int respect_flag, hipStream_t s);
 hipError_t launch_step_user(const StepLaunch& L, hipStream_t s);
+// L.iters iterations of whole sequences, exchange included; items are (fit,
+// first sequence of the wave); one: no fit has more data than lanes per chain
+hipError_t launch_iter_user(bool one, const StepLaunch& L, hipStream_t s);
+// LDS bytes of one chain's state in these kernels, for launches whose fits
+// have at most nprm varied and nptot parameters
+constexpr int user_slot_bytes(int nprm, int nptot) { return (2 * 8 * nprm + 7 * 4 * nprm + 2 * 4 * nptot + 7) / 8 * 8; }
 const char* user_model_name();
 
 }  // namespace mhre

@@ -29,23 +29,6 @@
 
 namespace mhre {
 
-// ------------------------------------------------------------------ helpers
-
-__device__ inline int pick_with_retry(uint32_t w0, int n, uint32_t c0, uint32_t c1, uint32_t c2,
-                                      uint32_t c3base, uint32_t k0, uint32_t k1) {
-  int k = pick_index(w0, n);
-  for (int r = 1; k >= n && r <= RNG_MAX_RETRY; ++r)
-    k = pick_index(philox4x32_10(c0, c1, c2, c3base + (uint32_t)r, k0, k1).x, n);
-  return k >= n ? n - 1 : k;
-}
-
-// Box-Muller in float64 (same formula as the oracle, so proposals round to
-// the same fp32 value).
-__device__ inline double normal64(uint32_t w1, uint32_t w2) {
-  const double u1 = (double)u01(w1), u2 = (double)u01(w2);
-  return sqrt(-2.0 * log(u1)) * cos(6.283185307179586 * u2);
-}
-
 // ------------------------------------------------------------- init chains
 
 __global__ void k_init_chains(const FitDesc* fits, const WorkItem* work, int nwork) {

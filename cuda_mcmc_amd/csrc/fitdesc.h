@@ -69,6 +69,7 @@ struct FitDesc {
   int hwords;            // words per acceptance history: ceil(nadj / 32)
   int xlanes;            // exchange: lanes per sequence (a power of two >= nbeta, or 64),
                          // so one wave swaps 64 / xlanes sequences side by side
+  int ulanes;            // model.cuh path: lanes per chain (a power of two)
   int hwphase;           // ring+Gaussian step kernel: every shift phase (revolutions) is
                          // bounded by 64 over the prior box, the chains' values and the
                          // data's baselines, so the hardware sine needs no reduction

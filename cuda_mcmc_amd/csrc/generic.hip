@@ -5,9 +5,16 @@
 // results in mc->datm[imd], return 0/1/2/-1.  The kernels here fuse what the
 // reference splits into calc_chi2_terms (src/gpu_mcmc.cu:273-325),
 // calc_chi2 (:331-350), gen_proposal (:361-411), spmp_mcmc (:426-474) and
-// adjust_steps (:480-526): one thread per chain runs every pass over every
-// datum in order, so pass p+1 may read what pass p stored in datm exactly as
-// in the reference, and the chain's whole iteration is one launch.
+// adjust_steps (:480-526).  As in the reference, where the data of one pass
+// are threads of one launch (:754), the data of a pass run side by side: a
+// chain has 1 to 256 lanes, datum id on lane id % lanes, and between two
+// passes its lanes wait for each other, so pass p+1 may read what pass p
+// stored in datm.
+//
+//   k_iter_user  fits with few data: a sequence's whole ladder in one wave,
+//                many iterations with their replica exchange in one launch
+//   k_step_user  the others: one iteration a launch, up to 4 waves a chain
+//                (the exchange has a launch of its own, k_exchange)
 #include <hip/hip_runtime.h>
 #include "mhre_device.h"
 #include "fitdesc.h"
@@ -21,159 +28,528 @@
 
 namespace mhre {
 
-// chi^2 of chain ch from the user's model (all passes), written to chi2m.
-// Returns the sum over all ndat terms (the reference sums every chi2m entry
-// of the chain, including entries no pass rewrote).  Sets *err on iret < 0.
-__device__ inline double user_chi2(const FitDesc& f, int ch, int* err) {
-  CCalcModel* mc = f.mc;
+// Orders the global and LDS accesses of a chain's lanes: what one stored
+// before is read by the others afterwards.  NW = 1: the lanes share a wave
+// (its memory operations keep their order); else they are a work-group.
+template <int NW>
+__device__ inline void chain_fence() {
+  if (NW == 1) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  } else {
+    __syncthreads();
+  }
+}
+
+// The lanes of one chain.
+template <int NW>
+struct ChainLanes {
+  int n;          // lanes of the chain (a power of two; 64 NW for NW > 1)
+  int j;          // this lane's place among them
+  double* xs;     // NW > 1: work-group LDS, 2 NW doubles
+  int flip;
+
+  // Sum over the chain's lanes, the same on each of them.  NW > 1: the waves'
+  // sums meet in xs, whose two halves take turns, so that one barrier does.
+  __device__ double sum(double v) {
+    if (NW == 1) {
+      if (n == 64) return wave_sum(v);
+      for (int m = n >> 1; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+      return v;
+    }
+    v = wave_sum(v);
+    double* x = xs + flip * NW;
+    flip ^= 1;
+    if (lane_id() == 0) x[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double s = x[0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) s += x[w];
+    return s;
+  }
+};
+
+// The fit's CCalcModel as a local object.  Its fields come from scalar loads
+// and its pointers are known to be global, so once model() is inlined no
+// field is read again per datum and its arrays take global instead of flat
+// accesses.
+__device__ inline CCalcModel user_model_args(const FitDesc& f) {
+  const CONSTANT CCalcModel* c = wave_const(f.mc);
+  CCalcModel m;
+  m.imodel = c->imodel; m.ncoor = c->ncoor; m.ndat = c->ndat; m.nicoor = c->nicoor; m.nidat = c->nidat;
+  m.ndatm = c->ndatm; m.nptot = c->nptot; m.nbeta = c->nbeta; m.nseq = c->nseq; m.nchi2m = c->nchi2m;
+  m.coor = (float*)gptr(c->coor); m.dat = (float*)gptr(c->dat); m.std2r = (float*)gptr(c->std2r);
+  m.icoor = (int*)gptr(c->icoor); m.idat = (int*)gptr(c->idat);
+  m.datm = (float*)gptr(c->datm); m.chi2m = (float*)gptr(c->chi2m);
+  m.pcur = (float*)gptr(c->pcur); m.flag = (int*)gptr(c->flag); m.chi2c = (float*)gptr(c->chi2c);
+  return m;
+}
+
+// One pass of datum id of chain ch: true and the new chi^2 term, or false if
+// the pass gives this datum no result.
+__device__ inline bool user_term(const FitDesc& f, CCalcModel* mc, int ch, int id, int ipass, float* term, int* err) {
+  const int imd = ch * f.ndat + id;
+  const int iret = model(mc, id, ch * f.nptot, imd, ipass);
+  if (iret == 0) return false;
+  if (iret < 0) { *err = iret; return false; }
+  float dif = gptr(f.dat)[id] - gptr(f.datm)[imd];
+  if (iret == 2) dif = atan2f(sinf(dif), cosf(dif));
+  *term = (dif * dif) * gptr(f.std2r)[id];
+  gptr(f.chi2m)[imd] = *term;
+  return true;
+}
+
+// chi^2 of chain ch from the user's model (all passes), its terms in chi2m:
+// the sum over all ndat terms (the reference sums every chi2m entry of the
+// chain, including entries no pass rewrote), in float64.  ONE: the chain has
+// at most one datum a lane, whose chi2m entry the lane keeps in term, so that
+// the sum needs no load behind the store.
+template <int NW, bool ONE>
+__device__ inline double user_chi2(const FitDesc& f, CCalcModel* mc, ChainLanes<NW>& cl, int ch, float* term,
+                                   int* err) {
   const int ndat = f.ndat;
-  const int ipt = ch * f.nptot;
-  const size_t base = (size_t)ch * ndat;
   for (int ipass = 0; ipass < f.npass; ++ipass) {
-    for (int id = 0; id < ndat; ++id) {
-      const int imd = (int)(base + id);
-      const int iret = model(mc, id, ipt, imd, ipass);
-      if (iret == 0) continue;
-      if (iret < 0) { *err = iret; continue; }
-      float dif = f.dat[id] - f.datm[imd];
-      if (iret == 2) dif = atan2f(sinf(dif), cosf(dif));
-      f.chi2m[imd] = (dif * dif) * f.std2r[id];
+    if (ipass) chain_fence<NW>();
+    if (ONE) {
+      if (cl.j < ndat) user_term(f, mc, ch, cl.j, ipass, term, err);
+    } else {
+      float t;
+      for (int id = cl.j; id < ndat; id += cl.n) user_term(f, mc, ch, id, ipass, &t, err);
     }
   }
   double s = 0.0;
-  for (int id = 0; id < ndat; ++id) s += (double)f.chi2m[base + id];
-  return s;
+  if (ONE) {
+    if (cl.j < ndat) s = (double)*term;
+  } else {
+    const GLOBAL float* c = gptr(f.chi2m) + (size_t)ch * ndat;
+    for (int id = cl.j; id < ndat; id += cl.n) s += (double)c[id];
+  }
+  return cl.sum(s);
 }
 
+// Model data and chi^2 of every chain of the list, one wave per chain.
 __global__ void __launch_bounds__(64) k_eval_user(const FitDesc* fits, const WorkItem* work, int nwork,
                                                   int model_only, int respect_flag) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= nwork) return;
-  const WorkItem w = work[g];
-  const FitDesc& f = fits[w.fit];
-  const int ch = w.idx;
+  const WorkItem w = work[blockIdx.x];
+  const FitDesc& f = wave_fit(fits, w.fit);
+  const int ch = __builtin_amdgcn_readfirstlane(w.idx);
+  CCalcModel mc = user_model_args(f);
+  ChainLanes<1> cl{64, lane_id(), nullptr, 0};
   int err = 0;
   if (model_only) {
     // calc_model (src/gpu_mcmc.cu:633-658): pass 0 only, no chi^2
-    for (int id = 0; id < f.ndat; ++id) {
-      const int iret = model(f.mc, id, ch * f.nptot, ch * f.ndat + id, 0);
+    for (int id = cl.j; id < f.ndat; id += 64) {
+      const int iret = model(&mc, id, ch * f.nptot, ch * f.ndat + id, 0);
       if (iret < 0) err = iret;
     }
   } else {
     double s;
     if (respect_flag && f.flag[ch] == 0) {
       s = 0.0;
-      for (int id = 0; id < f.ndat; ++id) s += (double)f.chi2m[(size_t)ch * f.ndat + id];
+      for (int id = cl.j; id < f.ndat; id += 64) s += (double)f.chi2m[(size_t)ch * f.ndat + id];
+      s = cl.sum(s);
     } else {
-      s = user_chi2(f, ch, &err);
+      float t;
+      s = user_chi2<1, false>(f, &mc, cl, ch, &t, &err);
     }
-    f.chi2c[ch] = (float)s;
+    if (cl.j == 0) f.chi2c[ch] = (float)s;
   }
   if (err && f.errflag) atomicExch(f.errflag, err);
 }
 
-// The chain's nprm proposals of this iteration (one lane); returns the
-// chi^2 evaluations performed.
-__device__ unsigned user_one_chain(const FitDesc& f, int ch, int it, const TraceBuf& tr) {
+// A chain's state in LDS for the launch, one copy per wave (the waves of a
+// chain compute the same, so no wave waits for another's bookkeeping): P
+// entries of each array, then two rows of N parameters (k_iter_user's
+// exchange writes the one that the iteration did not use).
+struct UserSlot {
+  double *z, *lu;        // this iteration's Gaussian steps and log u
+  float* stp;
+  int *cnt, *nac, *sh;
+  uint32_t* hw;          // the history word holding entry cnt % nadj ...
+  int* hwi;              // ... and its index
+  int* k;                // this iteration's coordinate picks
+  float* row;
+};
+__device__ inline UserSlot user_slot(char* lds, int P) {
+  UserSlot u;
+  u.z = reinterpret_cast<double*>(lds);
+  u.lu = u.z + P;
+  u.stp = reinterpret_cast<float*>(u.lu + P);
+  u.cnt = reinterpret_cast<int*>(u.stp + P);
+  u.nac = u.cnt + P;
+  u.sh = u.nac + P;
+  u.hw = reinterpret_cast<uint32_t*>(u.sh + P);
+  u.hwi = reinterpret_cast<int*>(u.hw + P);
+  u.k = u.hwi + P;
+  u.row = reinterpret_cast<float*>(u.k + P);
+  return u;
+}
+
+// Place and number of a wave's lanes of a chain, for work that every wave of
+// the chain does by itself.
+template <int NW>
+__device__ inline int own_j(const ChainLanes<NW>& cl) { return NW == 1 ? cl.j : lane_id(); }
+template <int NW>
+__device__ inline int own_n(const ChainLanes<NW>& cl) { return NW == 1 ? cl.n : 64; }
+
+// The wave's LDS copy of the chain's state; hist: the launch has burn-in
+// iterations.
+template <int NW>
+__device__ inline void user_load(const FitDesc& f, const ChainLanes<NW>& cl, int ch, const UserSlot& u, bool hist) {
   const int C = f.nchain, P = f.nprm, N = f.nptot;
-  const int ibeta = ch / f.nseq;
-  const bool burn = it < f.nburn;
-  const double beta = (double)f.beta[ibeta];
-  float chi2c = f.chi2c[ch];
-  int flag = 0, tlast = 0, err = 0;
-  float told = 0.0f;
-  unsigned nev = 0;
-  for (int s = 0; s < P; ++s) {
-    const U4 r = philox4x32_10((uint32_t)ch, (uint32_t)it, (uint32_t)s, 0u, f.key0, f.key1);
-    int k = pick_index(r.x, P);
-    for (int rr = 1; k >= P && rr <= RNG_MAX_RETRY; ++rr)
-      k = pick_index(philox4x32_10((uint32_t)ch, (uint32_t)it, (uint32_t)s, (uint32_t)rr, f.key0, f.key1).x, P);
-    if (k >= P) k = P - 1;
-    const int t = f.ivar[k];
+  for (int k = own_j(cl); k < P; k += own_n(cl)) {
     const size_t pk = (size_t)k * C + ch;
-    float* pt = f.pcur + (size_t)ch * N + t;
-    const float old = *pt;
-    const double u1 = (double)u01(r.y), u2 = (double)u01(r.z);
-    double pd = (double)old + (double)f.pstp[pk] * (sqrt(-2.0 * log(u1)) * cos(6.283185307179586 * u2));
-    if (f.pdescr[t] == 2) pd = pd - 6.283185307179586 * rint(pd / 6.283185307179586);
+    u.stp[k] = gptr(f.pstp)[pk];
+    u.nac[k] = gptr(f.n_acpt)[pk];
+    const int cnt = gptr(f.n_cnt)[pk];
+    u.cnt[k] = cnt;
+    if (hist) {
+      const int wi = (cnt % f.nadj) >> 5;
+      u.sh[k] = gptr(f.sumh)[pk];
+      u.hwi[k] = wi;
+      u.hw[k] = gptr(f.hbits)[((size_t)ch * f.hwords + wi) * P + k];
+    }
+  }
+  for (int i = own_j(cl); i < N; i += own_n(cl)) u.row[i] = gptr(f.pcur)[(size_t)ch * N + i];
+}
+
+template <int NW>
+__device__ inline void user_store(const FitDesc& f, const ChainLanes<NW>& cl, int ch, const UserSlot& u, bool hist) {
+  const int C = f.nchain, P = f.nprm;
+  for (int k = cl.j; k < P; k += cl.n) {
+    const size_t pk = (size_t)k * C + ch;
+    gptr(f.n_acpt)[pk] = u.nac[k];
+    if (hist) {
+      gptr(f.pstp)[pk] = u.stp[k];
+      gptr(f.n_cnt)[pk] = u.cnt[k];
+      gptr(f.sumh)[pk] = u.sh[k];
+      gptr(f.hbits)[((size_t)ch * f.hwords + u.hwi[k]) * P + k] = u.hw[k];
+    }
+  }
+}
+
+// What the chain's last proposal leaves in flag, ptent and ptentn.
+struct LastProposal {
+  int flag, t;
+  float told;
+};
+
+// The chain's nprm proposals of iteration it on the state in u and chi2c;
+// returns the chi^2 evaluations performed.  Every lane of the chain follows
+// the same decisions; the data of a chi^2 are split among them.  row: the
+// current half of u.row.
+template <int NW, bool ONE>
+__device__ unsigned user_substeps(const FitDesc& f, CCalcModel* mc, ChainLanes<NW>& cl, int ch, int it,
+                                  const TraceBuf& tr, const UserSlot& u, float* row, float& chi2c, float* term,
+                                  LastProposal& last, int* err) {
+  const int C = f.nchain, P = f.nprm, N = f.nptot;
+  const bool burn = it < f.nburn;
+  const double beta = (double)gptr(f.beta)[ch / f.nseq];
+  const int nadj = f.nadj;
+  const float rnadj = 1.0f / (float)nadj;
+  GLOBAL float* prow = gptr(f.pcur) + (size_t)ch * N;
+  unsigned nev = 0;
+  // the draws of substep s on the chain's lane s (modulo its lanes)
+  for (int s = own_j(cl); s < P; s += own_n(cl)) {
+    const U4 r = philox4x32_10((uint32_t)ch, (uint32_t)it, (uint32_t)s, 0u, f.key0, f.key1);
+    u.k[s] = pick_with_retry(r.x, P, (uint32_t)ch, (uint32_t)it, (uint32_t)s, 0u, f.key0, f.key1);
+    u.z[s] = normal64(r.y, r.z);
+    u.lu[s] = log((double)u01(r.w));
+  }
+  wave_sync_lds();
+  for (int s = 0; s < P; ++s) {
+    const int k = u.k[s];
+    const int t = gptr(f.ivar)[k];
+    const float old = row[t], sd = u.stp[k];
+    double pd = (double)old + (double)sd * u.z[s];
+    if (gptr(f.pdescr)[t] == 2) pd = pd - 6.283185307179586 * rint(pd / 6.283185307179586);
     const float pn = (float)pd;
-    const bool inprior = !(pn < f.pmint[t] || pn > f.pmaxt[t]);
+    const bool inprior = !(pn < gptr(f.pmint)[t] || pn > gptr(f.pmaxt)[t]);
+    wave_sync_lds();   // every lane has read its row and step size
     int acc = 0;
     double c2 = 0.0;
     if (inprior) {
-      *pt = pn;
-      c2 = user_chi2(f, ch, &err);
+      if (cl.j == 0) prow[t] = pn;
+      chain_fence<NW>();   // the chain's lanes read the proposal through mc->pcur
+      c2 = user_chi2<NW, ONE>(f, mc, cl, ch, term, err);
       ++nev;
       const double x = -0.5 * beta * (c2 - (double)chi2c);
-      if (log((double)u01(r.w)) <= x) {
+      if (u.lu[s] <= x) {
         acc = 1;
         chi2c = (float)c2;
-        f.n_acpt[pk] += 1;
-      } else {
-        *pt = old;
+        if (own_j(cl) == 0) {
+          u.nac[k] += 1;
+          row[t] = pn;
+        }
+      } else if (cl.j == 0) {
+        prow[t] = old;   // every lane has used the rejected value: the sum took its term
       }
     }
-    flag = acc;
-    told = old;
-    tlast = t;
-    if (tr.dec && it >= tr.it0 && it < tr.it0 + tr.nit) {
+    last = LastProposal{acc, t, old};
+    if (tr.dec && it >= tr.it0 && it < tr.it0 + tr.nit && cl.j == 0) {
       const size_t ti = (size_t)f.tr_dec + ((size_t)(it - tr.it0) * P + s) * C + ch;
       tr.dec[ti] = k | ((inprior ? 1 : 0) << 8) | (acc << 9);
       tr.chi2[ti] = inprior ? (float)c2 : 0.0f;
     }
     if (burn) {
-      const int cnt = f.n_cnt[pk];
-      const int a = cnt % f.nadj;   // oldest history entry, replaced by this outcome
-      uint32_t* hw = f.hbits + ((size_t)ch * f.hwords + (a >> 5)) * P + k;
-      const uint32_t word = *hw, bit = 1u << (a & 31);
-      const int hold = (word & bit) ? 1 : 0;
-      *hw = acc ? (word | bit) : (word & ~bit);
-      const int sh = f.sumh[pk] + acc - hold;
-      f.sumh[pk] = sh;
-      const int den = cnt < f.nadj ? cnt : f.nadj;
-      const float rate = (float)sh / (float)den;
-      const float st = f.pstp[pk];
-      f.pstp[pk] = rate < f.adapt_target ? (float)((double)st / 1.01) : (float)((double)st * 1.01);
-      f.n_cnt[pk] = cnt + 1;
+      // history entry cnt % nadj: the oldest one, replaced by this outcome
+      // (the division-free forms of mhre_device.h give the reference's bits)
+      const int cnt = u.cnt[k], wi = u.hwi[k];
+      const int w2 = mod_small(cnt + 1, nadj, rnadj) >> 5;
+      if (own_j(cl) == 0) {
+        const uint32_t bit = 1u << (mod_small(cnt, nadj, rnadj) & 31);
+        const uint32_t word = u.hw[k];
+        const int sh = u.sh[k] + acc - ((word & bit) ? 1 : 0);
+        u.hw[k] = acc ? (word | bit) : (word & ~bit);
+        u.sh[k] = sh;
+        const int den = cnt < nadj ? cnt : nadj;
+        u.stp[k] = rate_below(sh, den, f.adapt_mid, f.adapt_tie) ? step_shrink(sd) : step_grow(sd);
+        u.cnt[k] = cnt + 1;
+      }
+      if (w2 != wi) {
+        // the word is full: on to the next one, which an earlier proposal of
+        // this launch may have written (short rings), hence the fences
+        GLOBAL uint32_t* h = gptr(f.hbits) + (size_t)ch * f.hwords * P + k;
+        chain_fence<NW>();
+        if (cl.j == 0) h[(size_t)wi * P] = u.hw[k];
+        chain_fence<NW>();
+        if (own_j(cl) == 0) {
+          u.hw[k] = h[(size_t)w2 * P];
+          u.hwi[k] = w2;
+        }
+      }
     }
+    wave_sync_lds();
   }
-  f.chi2c[ch] = chi2c;
-  f.flag[ch] = flag;
-  f.ptent[ch] = told;
-  f.ptentn[ch] = tlast;
-  if (err && f.errflag) atomicExch(f.errflag, err);
   return nev;
 }
 
-// One lane per chain; every fit's chain list is padded to whole waves, so a
-// wave's lanes share one fit and its counters take one atomic per wave.
-__global__ void __launch_bounds__(64) k_step_user(const FitDesc* fits, const WorkItem* work, int nwork,
-                                                  RunClock* clk, TraceBuf tr, int it_off) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (__builtin_amdgcn_readfirstlane(g) >= nwork) return;
-  const WorkItem w = work[g];
+// One iteration of every chain of the list.  NW = 1: lanes lanes a chain, so
+// 64 / lanes chains a wave (the list is padded to whole waves); NW > 1: one
+// chain a work-group of NW waves.  slot_bytes: LDS of one chain's state
+// (user_slot at maxp parameters).
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) k_step_user(const FitDesc* fits, const WorkItem* work, int nwork,
+                                                       RunClock* clk, TraceBuf tr, int it_off, int lanes,
+                                                       int slot_bytes) {
+  extern __shared__ __align__(16) char lds[];
+  __shared__ double xs[2 * NW];
+  const int lane = lane_id();
+  const int per = NW == 1 ? 64 / lanes : 1;
+  const int c = NW == 1 ? lane / lanes : 0;
+  const WorkItem w = work[blockIdx.x * per + c];
   const FitDesc& f = wave_fit(fits, w.fit);
   pass_clock(clk);
   const int it = __builtin_amdgcn_readfirstlane(load_clock(clk, it_off));
   if (it >= f.nburn + f.niter) return;
-  const bool live = w.idx >= 0;
-  const unsigned nev = live ? user_one_chain(f, w.idx, it, tr) : 0u;
-  wave_count(f, nev, live ? (unsigned)f.nprm : 0u);
+  const int ch = w.idx;
+  const bool live = ch >= 0;   // padding lanes only take part in the counting
+  ChainLanes<NW> cl{NW == 1 ? lanes : 64 * NW, NW == 1 ? lane & (lanes - 1) : (int)threadIdx.x, xs, 0};
+  unsigned nev = 0;
+  if (live) {
+    const int wid = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const UserSlot u = user_slot(lds + (size_t)(wid * per + c) * slot_bytes, f.nprm);
+    const bool hist = it < f.nburn;
+    CCalcModel mc = user_model_args(f);
+    float chi2c = gptr(f.chi2c)[ch], term;
+    LastProposal last{0, 0, 0.0f};
+    int err = 0;
+    user_load(f, cl, ch, u, hist);
+    wave_sync_lds();
+    nev = user_substeps<NW, false>(f, &mc, cl, ch, it, tr, u, u.row, chi2c, &term, last, &err);
+    chain_fence<NW>();   // every wave's state is final and no wave reads the arrays any more
+    user_store(f, cl, ch, u, hist);
+    if (cl.j == 0) {
+      gptr(f.chi2c)[ch] = chi2c;
+      gptr(f.flag)[ch] = last.flag;
+      gptr(f.ptent)[ch] = last.told;
+      gptr(f.ptentn)[ch] = last.t;
+    }
+    if (err && f.errflag) atomicExch(f.errflag, err);
+  }
+  const bool count = live && cl.j == 0;
+  if (NW == 1 || threadIdx.x < 64) wave_count(f, count ? nev : 0u, count ? (unsigned)f.nprm : 0u);
 }
 
-static inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
+// The replica exchange of iteration it among the slots of a k_iter_user wave
+// (reference: gpu_mcmc.cu:548-591, the draws and arithmetic of
+// exchange_wave): slot sl of sequence g of the wave's G is on the n lanes
+// from (sl G + g) n.  Gives each slot the slot that its state started in and
+// its chi^2 and label after the swaps; returns how often its pair swapped.
+// UNIFORM: one sequence, whose attempts take lane reads at scalar indices
+// instead of shuffles.
+template <bool UNIFORM>
+__device__ inline int user_exchange(const FitDesc& f, int iseq, int it, bool live, int sl, int g, int G, int n,
+                                    const TraceBuf& tr, float& c2, int& tc, int& perm) {
+  const int lane = lane_id(), B = f.nbeta, S = f.nseq;
+  const int step = G * n, mine = g * n;   // slot k of this sequence starts at lane k * step + mine
+  int k_l = 0;
+  double lu_l = 0.0, hb_l = 0.0;
+  if (live) {
+    const U4 r = philox4x32_10((uint32_t)iseq, (uint32_t)it, (uint32_t)sl, RNG_EXCH, f.key0, f.key1);
+    k_l = pick_with_retry(r.x, B - 1, (uint32_t)iseq, (uint32_t)it, (uint32_t)sl, RNG_EXCH, f.key0, f.key1);
+    lu_l = log((double)u01(r.y));
+  }
+  if (sl < B - 1) hb_l = -0.5 * ((double)gptr(f.beta)[sl + 1] - (double)gptr(f.beta)[sl]);
+  int nx = 0;
+  perm = sl;
+  const bool trace = tr.ex && it >= tr.it0 && it < tr.it0 + tr.nit;
+  for (int a = 0; a < B; ++a) {   // every lane takes part in every shuffle
+    int k;
+    float ck, ck1;
+    bool acc;
+    if (UNIFORM) {
+      k = bcast(k_l, a * step);
+      ck = bcast(c2, k * step);
+      ck1 = bcast(c2, (k + 1) * step);
+      acc = bcast(lu_l, a * step) <= bcast(hb_l, k * step) * ((double)ck - (double)ck1);
+    } else {
+      k = __shfl(k_l, a * step + mine);
+      ck = __shfl(c2, k * step + mine);
+      ck1 = __shfl(c2, (k + 1) * step + mine);
+      acc = __shfl(lu_l, a * step + mine) <= __shfl(hb_l, k * step + mine) * ((double)ck - (double)ck1);
+    }
+    // perm follows the state that a slot started with, and is turned round below
+    if (acc) {
+      if (sl == k) { c2 = ck1; ++nx; }
+      if (sl == k + 1) c2 = ck;
+      perm = perm == k ? k + 1 : (perm == k + 1 ? k : perm);
+    }
+    if (trace && live && sl == 0 && (lane & (n - 1)) == 0)
+      tr.ex[(size_t)f.tr_ex + ((size_t)(it - tr.it0) * B + a) * S + iseq] = k | ((acc ? 1 : 0) << 16);
+  }
+  const int j = lane & (n - 1);
+  perm = __builtin_amdgcn_ds_permute((perm * step + mine + j) << 2, sl);
+  tc = __shfl(tc, perm * step + mine);
+  return nx;
+}
+
+// Iterations it_off .. it_off + iters - 1 of the segment for whole sequences,
+// replica exchange included: a wave holds the temperature ladders (at most 64
+// rungs) of its sequences, f.ulanes lanes a chain, and nothing couples one
+// sequence to another, so no launch has to end between two iterations.  For
+// problems of few data such a launch is all latency, and so was the exchange
+// launch between two of them.  Items are (fit, first sequence of the wave).
+template <bool ONE>
+__global__ void __launch_bounds__(64) k_iter_user(const FitDesc* fits, const WorkItem* work, int nwork, RunClock* clk,
+                                                  TraceBuf tr, int it_off, int iters, int slot_bytes) {
+  extern __shared__ __align__(16) char lds[];
+  const WorkItem w = work[blockIdx.x];
+  const FitDesc& f = wave_fit(fits, w.fit);
+  pass_clock(clk);
+  const int it0 = __builtin_amdgcn_readfirstlane(load_clock(clk, it_off));
+  const int nit = f.nburn + f.niter;
+  if (it0 >= nit) return;
+  const int lane = lane_id();
+  const int B = f.nbeta, S = f.nseq, P = f.nprm, N = f.nptot, n = f.ulanes;
+  const int G = 64 / (f.xlanes * n);
+  const int c = lane / n, sl = c / G, g = c % G;
+  const int iseq = __builtin_amdgcn_readfirstlane(w.idx) + g;
+  const bool live = iseq < S && sl < B;
+  const int ch = live ? sl * S + iseq : 0;
+  ChainLanes<1> cl{n, lane & (n - 1), nullptr, 0};
+  const UserSlot u = user_slot(lds + (size_t)c * slot_bytes, P);
+  const bool hist = it0 < f.nburn;
+  CCalcModel mc = user_model_args(f);
+  float chi2c = 0.0f, term = 0.0f;
+  int tc = 0, err = 0, nex = 0;
+  unsigned nev = 0, nprop = 0;
+  LastProposal last{0, 0, 0.0f};
+  if (live) {
+    chi2c = gptr(f.chi2c)[ch];
+    tc = gptr(f.tcur)[ch];
+    if (ONE && cl.j < f.ndat) term = gptr(f.chi2m)[(size_t)ch * f.ndat + cl.j];
+    user_load(f, cl, ch, u, hist);
+  }
+  wave_sync_lds();
+  float* row = u.row;
+  float* other = u.row + N;
+  for (int i = 0; i < iters && it0 + i < nit; ++i) {
+    const int it = it0 + i;
+    const bool burn = it < f.nburn;
+    if (live) nev += user_substeps<1, ONE>(f, &mc, cl, ch, it, tr, u, row, chi2c, &term, last, &err);
+    nprop += P;
+    int perm = sl;
+    if (B > 1) {
+      const int nx = G == 1 ? user_exchange<true>(f, iseq, it, live, sl, g, G, n, tr, chi2c, tc, perm)
+                            : user_exchange<false>(f, iseq, it, live, sl, g, G, n, tr, chi2c, tc, perm);
+      if (!burn) nex += nx;
+    }
+    if (live) {
+      // the row that ends up in this slot, from the LDS of the slot it started in
+      const float* src = reinterpret_cast<const float*>(
+          reinterpret_cast<const char*>(row) + (ptrdiff_t)((perm * G + g) - c) * slot_bytes);
+      const bool moved = perm != sl;
+      const bool rec = !burn && f.record;
+      const int itr = it - f.nburn;
+      for (int q = cl.j; q < N; q += n) {
+        const float v = src[q];
+        other[q] = v;
+        if (moved) gptr(f.pcur)[(size_t)ch * N + q] = v;
+        if (rec) {
+          const int ip = gptr(f.invar)[q];
+          if (ip >= 0) gptr(f.pout)[(((size_t)B * ip + sl) * S + iseq) * f.niter + itr] = v;
+        }
+      }
+      if (rec && cl.j == 0) {
+        gptr(f.tout)[(size_t)ch * f.niter + itr] = tc;
+        if (sl == 0) gptr(f.chi2)[(size_t)iseq * f.niter + itr] = chi2c;
+      }
+    }
+    wave_sync_lds();
+    float* sw = row;
+    row = other;
+    other = sw;
+  }
+  if (live) {
+    user_store(f, cl, ch, u, hist);
+    if (cl.j == 0) {
+      gptr(f.chi2c)[ch] = chi2c;
+      gptr(f.tcur)[ch] = tc;
+      if (nex) gptr(f.n_exch)[ch] += nex;
+      gptr(f.flag)[ch] = last.flag;
+      gptr(f.ptent)[ch] = last.told;
+      gptr(f.ptentn)[ch] = last.t;
+    }
+    if (err && f.errflag) atomicExch(f.errflag, err);
+  }
+  const bool count = live && cl.j == 0;
+  wave_count(f, count ? nev : 0u, count ? nprop : 0u);
+}
 
 hipError_t launch_eval_user(const FitDesc* fits, const WorkItem* work, int nwork, int model_only,
                             int respect_flag, hipStream_t s) {
   if (nwork <= 0) return hipSuccess;
-  k_eval_user<<<cdiv(nwork, 64), 64, 0, s>>>(fits, work, nwork, model_only, respect_flag);
+  k_eval_user<<<nwork, 64, 0, s>>>(fits, work, nwork, model_only, respect_flag);
   return hipGetLastError();
 }
 
 hipError_t launch_step_user(const StepLaunch& L, hipStream_t s) {
   if (L.nwork <= 0) return hipSuccess;
   const TraceBuf tr{L.tr_dec, L.tr_chi2, L.tr_ex, L.tr_it0, L.tr_nit};
-  k_step_user<<<cdiv(L.nwork, 64), 64, 0, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off);
+  const int sb = user_slot_bytes(L.max_prm, L.max_tot), n = L.ulanes;
+  switch (n) {
+    case 256:
+      k_step_user<4><<<L.nwork, 256, 4 * sb, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, n, sb);
+      break;
+    case 128:
+      k_step_user<2><<<L.nwork, 128, 2 * sb, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, n, sb);
+      break;
+    default:
+      k_step_user<1><<<L.nwork / (64 / n), 64, (64 / n) * sb, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, n, sb);
+      break;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_iter_user(bool one, const StepLaunch& L, hipStream_t s) {
+  if (L.nwork <= 0) return hipSuccess;
+  const TraceBuf tr{L.tr_dec, L.tr_chi2, L.tr_ex, L.tr_it0, L.tr_nit};
+  const int sb = user_slot_bytes(L.max_prm, L.max_tot);
+  const int dyn = 64 / L.ulanes * sb;
+  if (one) k_iter_user<true><<<L.nwork, 64, dyn, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, L.iters, sb);
+  else k_iter_user<false><<<L.nwork, 64, dyn, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, L.iters, sb);
   return hipGetLastError();
 }
 
