@@ -28,6 +28,22 @@ __device__ inline int load_clock(const RunClock* clk, int it_off) {
   return __atomic_load_n(&clk->it, __ATOMIC_RELAXED) + it_off;
 }
 
+// Attempt a of the replica exchange of iteration it of sequence iseq: its
+// pair's lower slot and log u (B > 1, a < B).
+struct SwapDraw {
+  int k;
+  double lu;
+};
+__device__ inline SwapDraw swap_draw(const FitDesc& f, int iseq, int it, int a) {
+  const U4 r = philox4x32_10((uint32_t)iseq, (uint32_t)it, (uint32_t)a, RNG_EXCH, f.key0, f.key1);
+  return SwapDraw{pick_with_retry(r.x, f.nbeta - 1, (uint32_t)iseq, (uint32_t)it, (uint32_t)a, RNG_EXCH, f.key0, f.key1),
+                  log((double)u01(r.y))};
+}
+// -0.5 (beta[k+1] - beta[k]) of slot k, 0 for the last one.
+__device__ inline double swap_factor(const FitDesc& f, int k) {
+  return k < f.nbeta - 1 ? -0.5 * ((double)gptr(f.beta)[k + 1] - (double)gptr(f.beta)[k]) : 0.0;
+}
+
 // Adds the wave's performed evaluations and proposals to the fit's counters
 // with one atomic each (every lane of the wave, padding included, calls it).
 __device__ inline void wave_count(const FitDesc& f, unsigned nev, unsigned nprop) {

@@ -318,55 +318,37 @@ __global__ void __launch_bounds__(256) k_eval_eht(const FitDesc* fits, const Wor
 // computes it and keeps what its own slot sl needs: the slot whose row ends
 // up in sl, and sl's chi^2 and label after the swaps.  It also does the
 // exchange launch's per-slot writes for sl (n_exch) and, in slot 0's wave,
-// the sequence's trace entries.  Every operand of the attempts is
-// wave-uniform (lane reads; the n_exch count and the accept bits stay in
-// scalar registers); labels move with the rows, so sl's label is the one its
-// row started with.
+// the sequence's trace entries.  Labels move with the rows, so sl's label is
+// the one its row started with.
+static_assert(sizeof(LadderLds) <= sizeof(float2) * RING, "the swaps use the wave's ring");
 struct SlotAfterSwaps {
   int src;
   float c2;
   int tc;
 };
 __device__ inline SlotAfterSwaps seq_exchange(const FitDesc& f, int iseq, int sl, int itp, const float* c2s,
-                                              const int* tcs, const TraceBuf& tr) {
+                                              const int* tcs, const TraceBuf& tr, LadderLds& ladder) {
   const int lane = lane_id();
   const int B = f.nbeta, S = f.nseq;
   const bool burn = itp < f.nburn;
   const bool slot = lane < B;
-  float c2 = slot ? c2s[(size_t)lane * S + iseq] : 0.0f;
+  const float c2 = slot ? c2s[(size_t)lane * S + iseq] : 0.0f;
   const int tc0 = slot ? tcs[(size_t)lane * S + iseq] : 0;
-  int perm = lane;
-  int nx = 0;
-  if (B > 1) {
-    // attempt a's pair pick and log u on lane a, all drawn up front
-    int k_l = 0;
-    double lu_l = 0.0, hb_l = 0.0;
-    if (slot) {
-      const U4 r = philox4x32_10((uint32_t)iseq, (uint32_t)itp, (uint32_t)lane, RNG_EXCH, f.key0, f.key1);
-      k_l = pick_with_retry(r.x, B - 1, (uint32_t)iseq, (uint32_t)itp, (uint32_t)lane, RNG_EXCH, f.key0, f.key1);
-      lu_l = log((double)u01(r.y));
-    }
-    if (lane < B - 1) hb_l = -0.5 * ((double)f.beta[lane + 1] - (double)f.beta[lane]);
-    uint64_t accm = 0;   // bit a: attempt a swapped
-    for (int a = 0; a < B; ++a) {
-      const int k = bcast(k_l, a);
-      const float ck = bcast(c2, k), ck1 = bcast(c2, k + 1);
-      const double x = bcast(hb_l, k) * ((double)ck - (double)ck1);
-      if (bcast(lu_l, a) <= x) {
-        accm |= 1ull << a;
-        const int pk = bcast(perm, k), pk1 = bcast(perm, k + 1);
-        if (lane == k) { c2 = ck1; perm = pk1; }
-        if (lane == k + 1) { c2 = ck; perm = pk; }
-        if (k == sl) ++nx;
-      }
-    }
-    if (tr.ex && sl == 0 && slot && itp >= tr.it0 && itp < tr.it0 + tr.nit)
-      tr.ex[(size_t)f.tr_ex + ((size_t)(itp - tr.it0) * B + lane) * S + iseq] =
-          k_l | ((int)((accm >> lane) & 1ull) << 16);
-  }
+  if (B < 2) return SlotAfterSwaps{sl, bcast(c2, sl), bcast(tc0, sl)};
+  SwapDraw d{0, 0.0};
+  if (slot) d = swap_draw(f, iseq, itp, lane);
+  const double hk = __shfl(swap_factor(f, lane), d.k);
+  ladder.slot[lane] = LadderSlot{c2, lane};
+  ladder.pair[lane] = 0;
+  const unsigned long long swapped = ladder_swaps(ladder, slot, d.k, 1, d.k == 0, d.lu, hk);
+  if (tr.ex && sl == 0 && slot && itp >= tr.it0 && itp < tr.it0 + tr.nit)
+    tr.ex[(size_t)f.tr_ex + ((size_t)(itp - tr.it0) * B + lane) * S + iseq] =
+        d.k | ((int)((swapped >> lane) & 1ull) << 16);
+  const LadderSlot me = ladder.slot[sl];
+  const int nx = __popcll(ladder.pair[sl] & swapped);
   if (!burn && nx && lane == 0) f.n_exch[(size_t)sl * S + iseq] += nx;
-  const int src = bcast(perm, sl);
-  return SlotAfterSwaps{src, bcast(c2, sl), bcast(tc0, src)};
+  const int src = __builtin_amdgcn_readfirstlane(me.src);
+  return SlotAfterSwaps{src, __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(me.c2))), bcast(tc0, src)};
 }
 
 // One MH iteration of chain ch (all nprm single-parameter proposals) by one
@@ -411,7 +393,9 @@ __device__ __attribute__((always_inline)) void step_one_chain(const FitDesc& f, 
       const int iseq = ch - ibeta * f.nseq;
       const float* ps = odd ? f.pcur : f.pcur_b;
       const SlotAfterSwaps x = seq_exchange(f, iseq, ibeta, it - 1, odd ? f.chi2c : f.chi2c_b,
-                                            odd ? f.tcur : f.tcur_b, tr);
+                                            odd ? f.tcur : f.tcur_b, tr,
+                                            *reinterpret_cast<LadderLds*>(ring));   // not yet used by the chi^2
+      ring_fence();
       pl = lane < N ? ps[((size_t)x.src * f.nseq + iseq) * N + lane] : 0.0f;
       chi2c = x.c2;
       tc = x.tc;
@@ -968,12 +952,12 @@ k_step_quad(const FitDesc* fits, const WorkItem* work, int nwork, RunClock* clk,
 // Sequences iseq0 .. iseq0 + 64/W - 1 of the fit, W = f.xlanes lanes each:
 // lane g*W + j holds temperature slot j of sequence iseq0 + g.  The swap
 // attempts of one sequence are sequential (reference: gpu_mcmc.cu:548-624);
-// the groups of a wave run theirs side by side, exchanging values with lane
-// shuffles inside each group.  The state is read from (ps, cs, ts) and
+// the groups of a wave run theirs side by side (ladder_swaps).  The state is read from (ps, cs, ts) and
 // written to (pd, cd, td), which may be the same arrays; with swaps = false
 // the state is only copied (no attempt, no sample, no trace).
 __device__ void exchange_wave(const FitDesc& f, int iseq0, int it, bool swaps, const float* ps, const float* cs,
-                              const int* ts, float* pd, float* cd, int* td, const TraceBuf& tr) {
+                              const int* ts, float* pd, float* cd, int* td, const TraceBuf& tr,
+                              LadderLds& ladder) {
   const int lane = lane_id();
   const int B = f.nbeta, S = f.nseq, N = f.nptot, W = f.xlanes;
   const bool burn = it < f.nburn;
@@ -988,30 +972,20 @@ __device__ void exchange_wave(const FitDesc& f, int iseq0, int it, bool swaps, c
   int perm = sl;
   int nex = 0;
   if (swaps && B > 1) {
-    // attempt a's pair pick and log u on slot a, all drawn up front
-    int k_l = 0;
-    double lu_l = 0.0, hb_l = 0.0;
-    if (slot) {
-      const U4 r = philox4x32_10((uint32_t)iseq, (uint32_t)it, (uint32_t)sl, RNG_EXCH, f.key0, f.key1);
-      k_l = pick_with_retry(r.x, B - 1, (uint32_t)iseq, (uint32_t)it, (uint32_t)sl, RNG_EXCH, f.key0, f.key1);
-      lu_l = log((double)u01(r.y));
-    }
-    // -0.5 (beta[k+1] - beta[k]) on slot k
-    if (sl < B - 1) hb_l = -0.5 * ((double)f.beta[sl + 1] - (double)f.beta[sl]);
-    for (int a = 0; a < B; ++a) {   // every lane takes part in every shuffle
-      const int k = __shfl(k_l, gb + a);
-      const float ck = __shfl(c2, gb + k), ck1 = __shfl(c2, gb + k + 1);
-      const double x = __shfl(hb_l, gb + k) * ((double)ck - (double)ck1);
-      const bool acc = __shfl(lu_l, gb + a) <= x;
-      const int tk = __shfl(tc, gb + k), tk1 = __shfl(tc, gb + k + 1);
-      const int pk = __shfl(perm, gb + k), pk1 = __shfl(perm, gb + k + 1);
-      if (acc) {
-        if (sl == k) { c2 = ck1; tc = tk1; perm = pk1; if (!burn) ++nex; }
-        if (sl == k + 1) { c2 = ck; tc = tk; perm = pk; }
-      }
-      if (tr.ex && sl == 0 && seq_ok && it >= tr.it0 && it < tr.it0 + tr.nit)
-        tr.ex[(size_t)f.tr_ex + ((size_t)(it - tr.it0) * B + a) * S + iseq] = k | ((acc ? 1 : 0) << 16);
-    }
+    // attempt sl on slot sl's lane
+    SwapDraw d{0, 0.0};
+    if (slot) d = swap_draw(f, iseq, it, sl);
+    const double hk = __shfl(swap_factor(f, sl), gb + d.k);
+    ladder.slot[lane] = LadderSlot{c2, sl};
+    ladder.pair[lane] = 0;
+    const unsigned long long swapped = ladder_swaps(ladder, slot, gb + d.k, 1, d.k == 0, d.lu, hk);
+    c2 = ladder.slot[lane].c2;
+    perm = ladder.slot[lane].src;
+    tc = __shfl(tc, gb + perm);
+    if (!burn) nex = __popcll(ladder.pair[lane] & swapped);
+    if (tr.ex && slot && it >= tr.it0 && it < tr.it0 + tr.nit)
+      tr.ex[(size_t)f.tr_ex + ((size_t)(it - tr.it0) * B + sl) * S + iseq] =
+          d.k | ((int)((swapped >> lane) & 1ull) << 16);
   }
   // move parameter rows: slot lane receives the row that started in slot perm
   float row[MAXP];
@@ -1090,6 +1064,7 @@ __device__ void exchange_serial(const FitDesc& f, int iseq, int it, bool burn, c
 // clears the queue heads and moves the clock on.
 __global__ void __launch_bounds__(64) k_exchange(const FitDesc* fits, const WorkItem* xwork, XcdRanges xr,
                                                  RunClock* clk, TraceBuf tr, int it_off, int close_k) {
+  __shared__ LadderLds ladder;
   const int base = close_k > 0 ? __atomic_load_n(&clk->xit, __ATOMIC_RELAXED)
                                : __atomic_load_n(&clk->it, __ATOMIC_RELAXED);
   const int xb = (int)(blockIdx.x % NXCD);
@@ -1101,7 +1076,7 @@ __global__ void __launch_bounds__(64) k_exchange(const FitDesc* fits, const Work
     if (close_k == 0) {
       const int it = base + it_off;
       if (it <= lf) {
-        if (f.nbeta <= 64) exchange_wave(f, w.idx, it, true, f.pcur, f.chi2c, f.tcur, f.pcur, f.chi2c, f.tcur, tr);
+        if (f.nbeta <= 64) exchange_wave(f, w.idx, it, true, f.pcur, f.chi2c, f.tcur, f.pcur, f.chi2c, f.tcur, tr, ladder);
         else exchange_serial(f, w.idx, it, it < f.nburn, tr);
       }
     } else if (lf >= base) {
@@ -1110,7 +1085,7 @@ __global__ void __launch_bounds__(64) k_exchange(const FitDesc* fits, const Work
       const bool odd = (at & 1) != 0;
       if (lf >= last || odd)
         exchange_wave(f, w.idx, last, lf >= last, odd ? f.pcur_b : f.pcur, odd ? f.chi2c_b : f.chi2c,
-                      odd ? f.tcur_b : f.tcur, f.pcur, f.chi2c, f.tcur, tr);
+                      odd ? f.tcur_b : f.tcur, f.pcur, f.chi2c, f.tcur, tr, ladder);
     }
   }
   if (close_k > 0 && blockIdx.x == 0 && threadIdx.x == 0) {
@@ -1140,7 +1115,8 @@ __global__ void __launch_bounds__(64) k_exchange(const FitDesc* fits, const Work
 // (2 * NQ * 64 words), and with ROWS (fits that have update rows) qlds the
 // wave's LDS for the rows (QROW_LDS floats).
 template <int NQ, bool ROWS>
-__device__ void iter_quad_wave(const FitDesc& f, int iseq0, int it, const TraceBuf& tr, float* qlds, float* stage) {
+__device__ void iter_quad_wave(const FitDesc& f, int iseq0, int it, const TraceBuf& tr, float* qlds, float* stage,
+                               LadderLds& ladder) {
   const int lane = lane_id();
   const int B = f.nbeta, S = f.nseq, W = f.xlanes;
   const int lg = 6 - __builtin_ctz((unsigned)W);   // log2 G
@@ -1174,39 +1150,23 @@ __device__ void iter_quad_wave(const FitDesc& f, int iseq0, int it, const TraceB
   const unsigned nev = slot ? quad_substeps<NQ, true, ROWS>(f, ch, it, tr, x, c2, qlds, stage) : 0u;
   wave_count(f, nev, slot ? (unsigned)f.nprm : 0u);
 
-  // exchange: as exchange_wave, with the partner of slot k at lane k * G + g.
-  // Each lane follows where its starting state goes (pos: no shuffle per
-  // attempt); afterwards one forward permute gives every slot the slot its
-  // state started in (perm), and the labels follow from it.
-  int pos = sl;
+  // exchange: as exchange_wave, with slot k of the sequence at lane k * G + g
+  int perm = sl;
   int nex = 0;
   if (B > 1) {
-    int k_l = 0;
-    double lu_l = 0.0, hb_l = 0.0;
-    if (slot) {
-      const U4 r = philox4x32_10((uint32_t)iseq, (uint32_t)it, (uint32_t)sl, RNG_EXCH, f.key0, f.key1);
-      k_l = pick_with_retry(r.x, B - 1, (uint32_t)iseq, (uint32_t)it, (uint32_t)sl, RNG_EXCH, f.key0, f.key1);
-      lu_l = log((double)u01(r.y));
-    }
-    if (sl < B - 1) hb_l = -0.5 * ((double)f.beta[sl + 1] - (double)f.beta[sl]);
-    for (int a = 0; a < B; ++a) {   // every lane takes part in every shuffle
-      const int k = __shfl(k_l, (a << lg) + g);
-      const int lk = (k << lg) + g, lk1 = lk + G;
-      const float ck = __shfl(c2, lk), ck1 = __shfl(c2, lk1);
-      const double xx = __shfl(hb_l, lk) * ((double)ck - (double)ck1);
-      const bool acc = __shfl(lu_l, (a << lg) + g) <= xx;
-      if (acc) {
-        if (sl == k) { c2 = ck1; if (!burn) ++nex; }
-        if (sl == k + 1) c2 = ck;
-        pos = pos == k ? k + 1 : (pos == k + 1 ? k : pos);
-      }
-      if (tr.ex && sl == 0 && seq_ok && it >= tr.it0 && it < tr.it0 + tr.nit)
-        tr.ex[(size_t)f.tr_ex + ((size_t)(it - tr.it0) * B + a) * S + iseq] = k | ((acc ? 1 : 0) << 16);
-    }
+    SwapDraw d{0, 0.0};
+    if (slot) d = swap_draw(f, iseq, it, sl);
+    const double hk = __shfl(swap_factor(f, sl), (d.k << lg) + g);
+    ladder.slot[lane] = LadderSlot{c2, sl};
+    ladder.pair[lane] = 0;
+    const unsigned long long swapped = ladder_swaps(ladder, slot, (d.k << lg) + g, G, d.k == 0, d.lu, hk);
+    c2 = ladder.slot[lane].c2;
+    perm = ladder.slot[lane].src;
+    if (!burn) nex = __popcll(ladder.pair[lane] & swapped);
+    if (tr.ex && slot && it >= tr.it0 && it < tr.it0 + tr.nit)
+      tr.ex[(size_t)f.tr_ex + ((size_t)(it - tr.it0) * B + sl) * S + iseq] =
+          d.k | ((int)((swapped >> lane) & 1ull) << 16);
   }
-  // pos is a permutation of each sequence's slots (lanes past the ladder keep
-  // their own), so the forward permute writes every lane once
-  const int perm = __builtin_amdgcn_ds_permute(((pos << lg) + g) << 2, sl);
   const int src = (perm << lg) + g;
   tc = __shfl(tc, src);
   // slot lane receives the row that started in slot perm
@@ -1249,9 +1209,14 @@ k_iter_quad(const FitDesc* fits, const WorkItem* work, int nwork, RunClock* clk,
   const int it = __builtin_amdgcn_readfirstlane(load_clock(clk, it_off));
   // 256-thread work-groups: 4 waves
   __shared__ __align__(16) float qlds[ROWS ? 4 : 1][ROWS ? QROW_LDS : 4];
-  __shared__ float qstage[4][2 * NQ * 64];
-  if (it < f.nburn + f.niter)
-    iter_quad_wave<NQ, ROWS>(f, w.idx, it, tr, ROWS ? qlds[threadIdx.x >> 6] : nullptr, qstage[threadIdx.x >> 6]);
+  __shared__ __align__(16) float qstage[4][2 * NQ * 64 < (int)sizeof(LadderLds) / 4 ? sizeof(LadderLds) / 4 : 2 * NQ * 64];
+  if (it < f.nburn + f.niter) {
+    // the staged step sizes are written back before the exchange, whose
+    // ladders then take their place
+    float* st = qstage[threadIdx.x >> 6];
+    iter_quad_wave<NQ, ROWS>(f, w.idx, it, tr, ROWS ? qlds[threadIdx.x >> 6] : nullptr, st,
+                             *reinterpret_cast<LadderLds*>(st));
+  }
 }
 
 // ---------------------------------------------------------------- launchers

@@ -372,59 +372,6 @@ __global__ void __launch_bounds__(64 * NW) k_step_user(const FitDesc* fits, cons
   if (NW == 1 || threadIdx.x < 64) wave_count(f, count ? nev : 0u, count ? (unsigned)f.nprm : 0u);
 }
 
-// The replica exchange of iteration it among the slots of a k_iter_user wave
-// (reference: gpu_mcmc.cu:548-591, the draws and arithmetic of
-// exchange_wave): slot sl of sequence g of the wave's G is on the n lanes
-// from (sl G + g) n.  Gives each slot the slot that its state started in and
-// its chi^2 and label after the swaps; returns how often its pair swapped.
-// UNIFORM: one sequence, whose attempts take lane reads at scalar indices
-// instead of shuffles.
-template <bool UNIFORM>
-__device__ inline int user_exchange(const FitDesc& f, int iseq, int it, bool live, int sl, int g, int G, int n,
-                                    const TraceBuf& tr, float& c2, int& tc, int& perm) {
-  const int lane = lane_id(), B = f.nbeta, S = f.nseq;
-  const int step = G * n, mine = g * n;   // slot k of this sequence starts at lane k * step + mine
-  int k_l = 0;
-  double lu_l = 0.0, hb_l = 0.0;
-  if (live) {
-    const U4 r = philox4x32_10((uint32_t)iseq, (uint32_t)it, (uint32_t)sl, RNG_EXCH, f.key0, f.key1);
-    k_l = pick_with_retry(r.x, B - 1, (uint32_t)iseq, (uint32_t)it, (uint32_t)sl, RNG_EXCH, f.key0, f.key1);
-    lu_l = log((double)u01(r.y));
-  }
-  if (sl < B - 1) hb_l = -0.5 * ((double)gptr(f.beta)[sl + 1] - (double)gptr(f.beta)[sl]);
-  int nx = 0;
-  perm = sl;
-  const bool trace = tr.ex && it >= tr.it0 && it < tr.it0 + tr.nit;
-  for (int a = 0; a < B; ++a) {   // every lane takes part in every shuffle
-    int k;
-    float ck, ck1;
-    bool acc;
-    if (UNIFORM) {
-      k = bcast(k_l, a * step);
-      ck = bcast(c2, k * step);
-      ck1 = bcast(c2, (k + 1) * step);
-      acc = bcast(lu_l, a * step) <= bcast(hb_l, k * step) * ((double)ck - (double)ck1);
-    } else {
-      k = __shfl(k_l, a * step + mine);
-      ck = __shfl(c2, k * step + mine);
-      ck1 = __shfl(c2, (k + 1) * step + mine);
-      acc = __shfl(lu_l, a * step + mine) <= __shfl(hb_l, k * step + mine) * ((double)ck - (double)ck1);
-    }
-    // perm follows the state that a slot started with, and is turned round below
-    if (acc) {
-      if (sl == k) { c2 = ck1; ++nx; }
-      if (sl == k + 1) c2 = ck;
-      perm = perm == k ? k + 1 : (perm == k + 1 ? k : perm);
-    }
-    if (trace && live && sl == 0 && (lane & (n - 1)) == 0)
-      tr.ex[(size_t)f.tr_ex + ((size_t)(it - tr.it0) * B + a) * S + iseq] = k | ((acc ? 1 : 0) << 16);
-  }
-  const int j = lane & (n - 1);
-  perm = __builtin_amdgcn_ds_permute((perm * step + mine + j) << 2, sl);
-  tc = __shfl(tc, perm * step + mine);
-  return nx;
-}
-
 // Iterations it_off .. it_off + iters - 1 of the segment for whole sequences,
 // replica exchange included: a wave holds the temperature ladders (at most 64
 // rungs) of its sequences, f.ulanes lanes a chain, and nothing couples one
@@ -435,6 +382,7 @@ template <bool ONE>
 __global__ void __launch_bounds__(64) k_iter_user(const FitDesc* fits, const WorkItem* work, int nwork, RunClock* clk,
                                                   TraceBuf tr, int it_off, int iters, int slot_bytes) {
   extern __shared__ __align__(16) char lds[];
+  __shared__ LadderLds ladder;
   const WorkItem w = work[blockIdx.x];
   const FitDesc& f = wave_fit(fits, w.fit);
   pass_clock(clk);
@@ -462,6 +410,7 @@ __global__ void __launch_bounds__(64) k_iter_user(const FitDesc* fits, const Wor
     if (ONE && cl.j < f.ndat) term = gptr(f.chi2m)[(size_t)ch * f.ndat + cl.j];
     user_load(f, cl, ch, u, hist);
   }
+  const double hb = swap_factor(f, sl);
   wave_sync_lds();
   float* row = u.row;
   float* other = u.row + N;
@@ -472,9 +421,24 @@ __global__ void __launch_bounds__(64) k_iter_user(const FitDesc* fits, const Wor
     nprop += P;
     int perm = sl;
     if (B > 1) {
-      const int nx = G == 1 ? user_exchange<true>(f, iseq, it, live, sl, g, G, n, tr, chi2c, tc, perm)
-                            : user_exchange<false>(f, iseq, it, live, sl, g, G, n, tr, chi2c, tc, perm);
-      if (!burn) nex += nx;
+      // the exchange (reference: gpu_mcmc.cu:548-591): slot sl of sequence g is
+      // entry c of the ladder LDS, and its first lane has attempt sl
+      SwapDraw d{0, 0.0};
+      if (live) d = swap_draw(f, iseq, it, sl);
+      const double hk = __shfl(hb, (d.k * G + g) * n);
+      if (cl.j == 0) {
+        ladder.slot[c] = LadderSlot{chi2c, sl};
+        ladder.pair[c] = 0;
+      }
+      const bool attempt = live && cl.j == 0;
+      const unsigned long long swapped = ladder_swaps(ladder, attempt, d.k * G + g, G, d.k == 0, d.lu, hk);
+      chi2c = ladder.slot[c].c2;
+      perm = ladder.slot[c].src;
+      tc = __shfl(tc, (perm * G + g) * n);
+      if (!burn) nex += __popcll(ladder.pair[c] & swapped);
+      if (tr.ex && attempt && it >= tr.it0 && it < tr.it0 + tr.nit)
+        tr.ex[(size_t)f.tr_ex + ((size_t)(it - tr.it0) * B + sl) * S + iseq] =
+            d.k | ((int)((swapped >> lane) & 1ull) << 16);
     }
     if (live) {
       // the row that ends up in this slot, from the LDS of the slot it started in

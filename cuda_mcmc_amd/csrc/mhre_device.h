@@ -388,4 +388,65 @@ __device__ inline void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// ------------------------------------------------ swaps of a ladder
+
+// One temperature slot during the swaps: its chi^2 and the slot that its
+// state started in.
+struct __align__(8) LadderSlot {
+  float c2;
+  int src;
+};
+
+// A wave's LDS for ladder_swaps: one entry per slot, slot k of a sequence at
+// index base + k * dk.
+struct LadderLds {
+  LadderSlot slot[64];
+  unsigned long long pair[64];   // lanes whose attempt names the pair (k, k + 1)
+};
+
+// The swap attempts of the wave's ladders (reference: gpu_mcmc.cu:548-591).
+// A lane with attempt = true holds one: the pair of slots at k0 and k0 + dk
+// (first: k0 is its sequence's first slot), accepted if
+// lu <= hb (chi^2 of k0 - chi^2 of k0 + dk).  Attempts act in the order of
+// their lanes, but only those that share a slot depend on one another, and
+// which do follows from the draws alone.  So an attempt runs as soon as the
+// earlier ones on its slots are done, all that are ready side by side: a
+// ladder of 32 rungs has 32 attempts in about 6 such steps (at most 11 in
+// 3000 random ladders), each a chain of an LDS read, two float64 operations and an LDS
+// write.  One attempt after the other through lane reads took 0.15 us an attempt.
+// Every lane of the wave calls it, with lds.slot filled and lds.pair zeroed;
+// returns the lanes whose attempts were accepted (lds.pair[k] & it: those of
+// pair k).
+__device__ inline unsigned long long ladder_swaps(LadderLds& lds, bool attempt, int k0, int dk, bool first, double lu,
+                                                  double hb) {
+  const int lane = lane_id();
+  wave_sync_lds();
+  unsigned long long before = 0;
+  if (attempt) atomicOr(&lds.pair[k0], 1ull << lane);
+  wave_sync_lds();
+  if (attempt)
+    before = (lds.pair[k0] | lds.pair[k0 + dk] | (first ? 0ull : lds.pair[k0 - dk])) & ((1ull << lane) - 1ull);
+  unsigned long long done = 0, swapped = 0;
+  bool pending = attempt;
+  for (;;) {
+    const bool ready = pending && (before & ~done) == 0;
+    const unsigned long long m = __ballot(ready);
+    if (m == 0) break;   // the earliest attempt left is always ready, so none is left
+    bool acc = false;
+    if (ready) {
+      const LadderSlot a = lds.slot[k0], b = lds.slot[k0 + dk];
+      acc = lu <= hb * ((double)a.c2 - (double)b.c2);
+      if (acc) {
+        lds.slot[k0] = b;
+        lds.slot[k0 + dk] = a;
+      }
+      pending = false;
+    }
+    swapped |= __ballot(acc);
+    done |= m;
+    wave_sync_lds();
+  }
+  return swapped;
+}
+
 }  // namespace mhre
