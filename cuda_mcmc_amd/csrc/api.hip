@@ -777,11 +777,6 @@ StepLaunch exchange_launch(Session* S, const Group& g, int it_off, int close_k) 
   return L;
 }
 
-// Most iterations of one launch of whole sequences: long enough to hide the
-// launch, short enough that the waves of a session of many fits, which take
-// several rounds of the chip, do not drift far apart.
-constexpr int SEQ_ITERS = 64;
-
 // The step launches of group g at offset i of its segment.  Kinds whose
 // launches hold whole sequences run iterations i .. i + n - 1 (n = 0: none,
 // an earlier launch has them).
@@ -789,15 +784,14 @@ int launch_steps(Session* S, const Group& g, int i, int n) {
   for (const KindWork& k : g.kinds) {
     StepLaunch L = make_launch(S, g, k, i);
     hipError_t e = hipSuccess;
-    if (k.kind == K_USER && k.fused) {
+    if (k.fused) {
       if (n == 0) continue;
       L.iters = n;
-      HIPCHK(launch_iter_user(k.one, L, g.stream));
+      HIPCHK(k.kind == K_USER ? launch_iter_user(k.one, L, g.stream) : launch_iter_quad(k.quad_n, k.rows, L, g.stream));
       continue;
     }
     if (k.kind == K_SGRA9) e = launch_step_eht(MODEL_SGRA9, L, g.stream);
     else if (k.kind == K_SGRA13) e = launch_step_eht(MODEL_SGRA13, L, g.stream);
-    else if (k.kind == K_QUAD && k.fused) e = launch_iter_quad(k.quad_n, k.rows, L, g.stream);
     else if (k.kind == K_QUAD) e = launch_step_quad(k.quad_n, L, g.stream);
     else e = launch_step_user(L, g.stream);
     HIPCHK(e);

@@ -15,6 +15,25 @@ __device__ inline const FitDesc& wave_fit(const FitDesc* fits, int fit) {
   return *(const FitDesc*)wave_const(fits + __builtin_amdgcn_readfirstlane(fit));
 }
 
+// The same descriptor, and the same value, through an address that the compiler
+// cannot follow: what a loop over iterations reads through it, or derives
+// from it, is read and derived again each time (scalar loads and a few
+// instructions) instead of being kept in registers over the whole loop.
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ inline const FitDesc& fit_again(const FitDesc& f) {
+  uint64_t a = (uint64_t)&f;
+  asm volatile("" : "+s"(a));
+  return *(const FitDesc*)(const CONSTANT FitDesc*)a;
+}
+__device__ inline int value_again(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+#else
+__device__ inline const FitDesc& fit_again(const FitDesc& f) { return f; }
+__device__ inline int value_again(int v) { return v; }
+#endif
+
 // Step launches: the first thread of the grid hands the segment's first
 // iteration on to the segment's closing exchange launch (RunClock); every
 // thread reads its iteration with load_clock (clk.it plus the launch's offset
@@ -67,6 +86,11 @@ struct TraceBuf {
   int it0, nit;
 };
 
+// Most iterations of one launch of whole sequences: long enough to hide the
+// launch, short enough that the waves of a session of many fits, which take
+// several rounds of the chip, do not drift far apart.
+constexpr int SEQ_ITERS = 64;
+
 struct StepLaunch {
   const FitDesc* fits;   // device
   const WorkItem* work;  // device, step work list
@@ -94,8 +118,8 @@ hipError_t launch_eval_eht(int model, const FitDesc* fits, const WorkItem* work,
 hipError_t launch_step_eht(int model, const StepLaunch& L, hipStream_t s);
 hipError_t launch_eval_quad(int n, const FitDesc* fits, const WorkItem* work, int nwork, hipStream_t s);
 hipError_t launch_step_quad(int n, const StepLaunch& L, hipStream_t s);
-// step + exchange of whole sequences (ladders of at most 64 rungs); work items
-// are (fit, first sequence of the wave); rows: every fit of the launch has
+// L.iters iterations (step + exchange) of whole sequences (ladders of at most
+// 64 rungs); work items are (fit, first sequence of the wave); rows: every fit of the launch has
 // single-coordinate update rows (FitDesc::qrow)
 hipError_t launch_iter_quad(int n, bool rows, const StepLaunch& L, hipStream_t s);
 // Exchange of the sequences in xwork (items: fit, first sequence of the wave):

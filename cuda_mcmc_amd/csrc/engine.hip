@@ -724,24 +724,80 @@ __global__ void __launch_bounds__(256) k_eval_quad(const FitDesc* fits, const Wo
   f.chi2c[w.idx] = (float)QuadSys<NQ>::chi2(gptr(f.qcoef), f.quad_neq, x);
 }
 
+// What a lane keeps of its chain besides x and chi2c while a launch runs.
+// CACHE (k_iter_quad, many iterations a launch): the adaptation counters n_cnt
+// and sumh of all its parameters, and the accepted proposals of each in 16-bit
+// counts; the step sizes and the current acceptance-history words (the word
+// that holds entry cnt % nadj) sit in the wave's LDS, [NQ][64] each, column =
+// lane.  Lanes pick different parameters, so per-proposal accesses in memory
+// scatter over rows, each lane a cache line of its own; held for the launch,
+// every array moves once per launch instead.
+template <int NQ, bool CACHE>
+struct QuadCarry {
+  int cnt[CACHE ? NQ : 1], sh[CACHE ? NQ : 1];
+  uint32_t nacc[CACHE ? (NQ + 1) / 2 : 1];
+  float* sp;
+  uint32_t* hw;
+  // the last proposal's accept flag, parameter and old value
+  int flag, tlast;
+  float told;
+};
+static_assert(SEQ_ITERS * 8 <= 65535, "a launch's accepted proposals of one parameter fit 16 bits");
+
+// hist: the launch has burn-in iterations.
+template <int NQ>
+__device__ inline void quad_load(const FitDesc& f, int ch, bool hist, QuadCarry<NQ, true>& q) {
+  const int C = f.nchain, P = f.nprm, ln = lane_id();
+#pragma unroll
+  for (int i = 0; i < (NQ + 1) / 2; ++i) q.nacc[i] = 0;
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    q.cnt[i] = q.sh[i] = 0;
+    if (i < P) {
+      q.sp[i * 64 + ln] = gptr(f.pstp)[i * C + ch];
+      if (hist) {
+        q.cnt[i] = gptr(f.n_cnt)[i * C + ch];
+        q.sh[i] = gptr(f.sumh)[i * C + ch];
+      }
+    }
+  }
+  if (hist) {
+#pragma unroll
+    for (int i = 0; i < NQ; ++i)
+      if (i < P) q.hw[i * 64 + ln] = gptr(f.hbits)[(ch * f.hwords + ((q.cnt[i] % f.nadj) >> 5)) * P + i];
+  }
+}
+// Acceptance counts only where a proposal was accepted (a lane left out
+// touches no line).
+template <int NQ>
+__device__ inline void quad_store(const FitDesc& f, int ch, bool hist, const QuadCarry<NQ, true>& q) {
+  const int C = f.nchain, P = f.nprm, ln = lane_id();
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    if (i < P) {
+      const int na = (int)((q.nacc[i / 2] >> (16 * (i & 1))) & 0xffffu);
+      if (na) gptr(f.n_acpt)[i * C + ch] += na;
+      if (hist) {
+        gptr(f.n_cnt)[i * C + ch] = q.cnt[i];
+        gptr(f.sumh)[i * C + ch] = q.sh[i];
+        gptr(f.pstp)[i * C + ch] = q.sp[i * 64 + ln];
+        gptr(f.hbits)[(ch * f.hwords + ((q.cnt[i] % f.nadj) >> 5)) * P + i] = q.hw[i * 64 + ln];
+      }
+    }
+  }
+}
+
 // The chain's nprm proposals of this iteration (one lane) on the state x,
 // chi2c held by the caller; returns the chi^2 evaluations performed.
-// CACHE: in the burn-in stage the adaptation counters n_cnt and sumh of all
-// the chain's parameters are read once (one coalesced row per parameter) and
-// kept in registers for the iteration, instead of one scattered
-// read-modify-write per proposal (lanes pick different parameters); the
-// step sizes and acceptance counts of all its parameters sit in the wave's
-// LDS for the iteration (stage: [NQ][64] floats then [NQ][64] ints, column
-// = lane), read and written back once.  Scattered single-word accesses per
-// proposal had made the launch HBM-bound (every lane a cache line of its own).
+// CACHE: the rest of its state is in q for the launch, else in memory.
 // ROWS: the weighted residual of every equation is evaluated in full once,
 // then kept in registers; a proposal, which moves one coordinate, updates
 // them from its block of the fit's row table in LDS (QROW_* layout) with
 // n + 3 operations per equation instead of n(n+1)/2 + n.  Its chi^2 is the
 // same sum of squares to float rounding (sqrt(w) r)^2 against r^2 w.
 template <int NQ, bool CACHE, bool ROWS = false>
-__device__ unsigned quad_substeps(const FitDesc& f, int ch, int it, const TraceBuf& tr, float (&x)[NQ],
-                                  float& chi2c, const float* rows = nullptr, float* stage = nullptr) {
+__device__ unsigned quad_substeps(const FitDesc& f, int ch, int ibeta, int it, const TraceBuf& tr, float (&x)[NQ],
+                                  float& chi2c, QuadCarry<NQ, CACHE>& q, const float* rows = nullptr) {
   const int C = f.nchain, P = f.nprm;
   const CONSTANT float* qc = wave_const(f.qcoef);
   const int neq = __builtin_amdgcn_readfirstlane(f.quad_neq);
@@ -754,38 +810,14 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, int it, const TraceB
   const CONSTANT int* pdescr = wave_const(f.pdescr);
   const CONSTANT float* pmint = wave_const(f.pmint);
   const CONSTANT float* pmaxt = wave_const(f.pmaxt);
-  const int ibeta = ch / f.nseq;
   const bool burn = it < f.nburn;
   const double beta = (double)gptr(f.beta)[ibeta];
   const int nadj = __builtin_amdgcn_readfirstlane(f.nadj);
   const int hwn = __builtin_amdgcn_readfirstlane(f.hwords);
   const float rnadj = 1.0f / (float)nadj;
-  int cnt_c[NQ], sh_c[NQ];
-  if (CACHE && burn) {
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      cnt_c[i] = i < P ? n_cnt[(size_t)i * C + ch] : 0;
-      sh_c[i] = i < P ? sumh[(size_t)i * C + ch] : 0;
-    }
-  }
   const int ln = lane_id();
-  float* sp = stage;
-  int* sa = reinterpret_cast<int*>(stage + NQ * 64);
-  if (CACHE) {
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      if (i < P) {
-        sp[i * 64 + ln] = pstp[i * C + ch];
-        sa[i * 64 + ln] = n_acpt[i * C + ch];
-      }
-    }
-  }
   float res[QROW_MAXEQ], resn[QROW_MAXEQ];
   if (ROWS) QuadSys<NQ>::residuals(qc, wave_const(f.qrow) + NQ * QROW_TS(NQ), neq, x, res);
-  // CACHE: bit k = a proposal of parameter k was accepted
-  uint32_t chg = 0;
-  int flag = 0, tlast = 0;
-  float told = 0.0f;
   unsigned nev = 0;
   for (int s = 0; s < P; ++s) {
     const U4 r = philox4x32_10((uint32_t)ch, (uint32_t)it, (uint32_t)s, 0u, f.key0, f.key1);
@@ -795,7 +827,7 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, int it, const TraceB
     float old = 0.0f;
 #pragma unroll
     for (int i = 0; i < NQ; ++i) old = (i == t) ? x[i] : old;
-    const float sd = CACHE ? sp[k * 64 + ln] : pstp[pk];
+    const float sd = CACHE ? q.sp[k * 64 + ln] : pstp[pk];
     // burn-in: the acceptance-history word of this outcome's entry
     // cnt % nadj (the oldest one), read before the proposal so that its
     // latency overlaps the chi^2
@@ -805,15 +837,15 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, int it, const TraceB
       if (CACHE) {
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-          cnt = (i == k) ? cnt_c[i] : cnt;
-          sh0 = (i == k) ? sh_c[i] : sh0;
+          cnt = (i == k) ? q.cnt[i] : cnt;
+          sh0 = (i == k) ? q.sh[i] : sh0;
         }
       } else {
         cnt = n_cnt[pk];
         sh0 = sumh[pk];
       }
       ha = mod_small(cnt, nadj, rnadj);
-      hword = hbits[(ch * hwn + (ha >> 5)) * P + k];
+      hword = CACHE ? q.hw[k * 64 + ln] : hbits[(ch * hwn + (ha >> 5)) * P + k];
     }
     // The Gaussian step in fp32 with the hardware log2 and cosine (which takes
     // revolutions, so cos(2 pi u2) is one instruction; its absolute error is
@@ -842,8 +874,9 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, int it, const TraceB
         acc = 1;
         chi2c = (float)c2;
         if (CACHE) {
-          sa[k * 64 + ln] += 1;
-          chg |= 1u << k;
+          const uint32_t one = 1u << (16 * (k & 1));
+#pragma unroll
+          for (int i = 0; i < (NQ + 1) / 2; ++i) q.nacc[i] += (k >> 1) == i ? one : 0u;
         } else {
           n_acpt[pk] += 1;
         }
@@ -858,27 +891,38 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, int it, const TraceB
         for (int i = 0; i < NQ; ++i) x[i] = (i == t) ? old : x[i];
       }
     }
-    flag = acc;
-    told = old;
-    tlast = t;
+    q.flag = acc;
+    q.told = old;
+    q.tlast = t;
     if (burn) {
       const uint32_t bit = 1u << (ha & 31);
       const int hold = (hword & bit) ? 1 : 0;
-      // stored only when the entry changes: the lanes of a wave touch one
-      // history line each, so every lane left out saves a line
-      if (acc != hold) hbits[(ch * hwn + (ha >> 5)) * P + k] = hword ^ bit;
+      const uint32_t nword = acc != hold ? hword ^ bit : hword;
+      if (CACHE) {
+        const int hn = ha + 1 == nadj ? 0 : ha + 1;   // the next proposal's entry
+        uint32_t next = nword;
+        if ((hn >> 5) != (ha >> 5)) {
+          hbits[(ch * hwn + (ha >> 5)) * P + k] = nword;
+          next = hbits[(ch * hwn + (hn >> 5)) * P + k];
+        }
+        q.hw[k * 64 + ln] = next;
+      } else if (nword != hword) {
+        // stored only when the entry changes: the lanes of a wave touch one
+        // history line each, so every lane left out saves a line
+        hbits[(ch * hwn + (ha >> 5)) * P + k] = nword;
+      }
       const int sh = sh0 + acc - hold;
       const int den = cnt < nadj ? cnt : nadj;
       const float nsd = rate_below(sh, den, f.adapt_mid, f.adapt_tie) ? step_shrink(sd) : step_grow(sd);
-      if (CACHE) sp[k * 64 + ln] = nsd;
-      else pstp[pk] = nsd;
       if (CACHE) {
+        q.sp[k * 64 + ln] = nsd;
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-          cnt_c[i] = (i == k) ? cnt + 1 : cnt_c[i];
-          sh_c[i] = (i == k) ? sh : sh_c[i];
+          q.cnt[i] = (i == k) ? cnt + 1 : q.cnt[i];
+          q.sh[i] = (i == k) ? sh : q.sh[i];
         }
       } else {
+        pstp[pk] = nsd;
         sumh[pk] = sh;
         n_cnt[pk] = cnt + 1;
       }
@@ -889,24 +933,6 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, int it, const TraceB
       gptr(tr.chi2)[ti] = inprior ? (float)c2 : 0.0f;
     }
   }
-  // write back; acceptance counts only where a proposal was accepted (a
-  // lane left out touches no line)
-  if (CACHE) {
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      if (i < P) {
-        if (burn) {
-          n_cnt[i * C + ch] = cnt_c[i];
-          sumh[i * C + ch] = sh_c[i];
-          pstp[i * C + ch] = sp[i * 64 + ln];
-        }
-        if ((chg >> i) & 1u) n_acpt[i * C + ch] = sa[i * 64 + ln];
-      }
-    }
-  }
-  gptr(f.flag)[ch] = flag;
-  gptr(f.ptent)[ch] = told;
-  gptr(f.ptentn)[ch] = tlast;
   return nev;
 }
 
@@ -917,13 +943,16 @@ __device__ unsigned quad_one_chain(const FitDesc& f, int ch, int it, const Trace
 #pragma unroll
   for (int i = 0; i < NQ; ++i) x[i] = pcur[(size_t)ch * NQ + i];
   float chi2c = gptr(f.chi2c)[ch];
-  const unsigned nev = quad_substeps<NQ, false>(f, ch, it, tr, x, chi2c);
+  QuadCarry<NQ, false> q;
+  const unsigned nev = quad_substeps<NQ, false>(f, ch, ch / f.nseq, it, tr, x, chi2c, q);
 #pragma unroll
   for (int i = 0; i < NQ; ++i) pcur[(size_t)ch * NQ + i] = x[i];
   gptr(f.chi2c)[ch] = chi2c;
+  gptr(f.flag)[ch] = q.flag;
+  gptr(f.ptent)[ch] = q.told;
+  gptr(f.ptentn)[ch] = q.tlast;
   return nev;
 }
-
 
 // One lane per chain; all chains of a wave belong to one fit (the host pads
 // every fit's chain list to whole waves), so the coefficients are uniform.
@@ -1099,24 +1128,34 @@ __global__ void __launch_bounds__(64) k_exchange(const FitDesc* fits, const Work
 
 // ------------------------------------- quadratic systems: step + exchange
 
-// One whole MH-RE iteration of quadratic-system sequences in one launch: the
+// Whole MH-RE iterations of quadratic-system sequences in one launch: the
 // lane-per-chain proposals of k_step_quad, then the replica exchange of every
 // sequence among the lanes that hold its temperature slots, with the chain
-// states still in registers (parameter rows move by lane shuffles, not through
-// memory).  A wave holds G = 64 / W sequences (W = xlanes, ladders of at most
-// 64 rungs); lane l is temperature slot l / G of sequence iseq0 + l % G, so
-// the G sequences of one slot are adjacent in the state arrays.  The random
-// counters are those of k_step_quad and k_exchange (reference update rule:
-// gpu_mcmc.cu:361-526 then :533-626), so the chains are the same bit for bit.
-// The burn-in counters held in registers (quad_substeps<NQ, true>) take the
-// register cap to 7 waves per SIMD.
-// The body of k_iter_quad for the wave's G sequences from iseq0; stage is
-// the wave's LDS for its chains' step sizes and acceptance counts
-// (2 * NQ * 64 words), and with ROWS (fits that have update rows) qlds the
-// wave's LDS for the rows (QROW_LDS floats).
+// states in registers and LDS from one iteration to the next (parameter rows
+// move by lane shuffles, not through memory).  Nothing couples one sequence to
+// another, so a launch runs many iterations, and the state, counters and
+// acceptance history move through memory once per launch.  A wave holds
+// G = 64 / W sequences (W = xlanes, ladders of at most 64 rungs); lane l is
+// temperature slot l / G of sequence iseq0 + l % G, so the G sequences of one
+// slot are adjacent in the state arrays.  The random counters are those of
+// k_step_quad and k_exchange (reference update rule: gpu_mcmc.cu:361-526 then
+// :533-626), so the chains are the same bit for bit.
+
+// A wave's LDS in k_iter_quad.
 template <int NQ, bool ROWS>
-__device__ void iter_quad_wave(const FitDesc& f, int iseq0, int it, const TraceBuf& tr, float* qlds, float* stage,
-                               LadderLds& ladder) {
+struct __align__(16) QuadLds {
+  float rows[ROWS ? NQ * QROW_TS(NQ) : 4];   // the fit's update rows
+  float sp[NQ * 64];
+  uint32_t hw[NQ * 64];
+  LadderLds ladder;
+};
+
+// The body of k_iter_quad for the wave's G sequences from iseq0: iterations
+// it0 .. it1 - 1.
+template <int NQ, bool ROWS>
+__device__ void iter_quad_wave(const FitDesc& f0, int iseq0, int it0, int it1, const TraceBuf& tr,
+                               QuadLds<NQ, ROWS>& lds) {
+  const FitDesc& f = f0;
   const int lane = lane_id();
   const int B = f.nbeta, S = f.nseq, W = f.xlanes;
   const int lg = 6 - __builtin_ctz((unsigned)W);   // log2 G
@@ -1125,11 +1164,14 @@ __device__ void iter_quad_wave(const FitDesc& f, int iseq0, int it, const TraceB
   const int iseq = __builtin_amdgcn_readfirstlane(iseq0) + g;
   const bool seq_ok = iseq < S;
   const bool slot = seq_ok && sl < B;
-  const int ch = sl * S + iseq;
-  const bool burn = it < f.nburn;
+  const int ch0 = sl * S + iseq, ch = ch0;
+  const bool hist = it0 < f.nburn;
   GLOBAL float* pcur = gptr(f.pcur);
   GLOBAL float* chi2c_a = gptr(f.chi2c);
   GLOBAL int* tcur_a = gptr(f.tcur);
+  QuadCarry<NQ, true> q;
+  q.sp = lds.sp;
+  q.hw = lds.hw;
   float x[NQ];
   float c2 = 0.0f;
   int tc = 0;
@@ -1138,85 +1180,91 @@ __device__ void iter_quad_wave(const FitDesc& f, int iseq0, int it, const TraceB
   if (slot) {
     c2 = chi2c_a[ch];
     tc = tcur_a[ch];
+    quad_load(f, ch, hist, q);
   }
   if (ROWS) {
     // the fit's update rows into this wave's LDS, every lane taking part
     constexpr int n4 = NQ * QROW_TS(NQ) / 4;
     const GLOBAL float4* src = (const GLOBAL float4*)gptr(f.qrow);
-    float4* dst = reinterpret_cast<float4*>(qlds);
+    float4* dst = reinterpret_cast<float4*>(lds.rows);
     for (int i = lane; i < n4; i += 64) dst[i] = src[i];
     ring_fence();
   }
-  const unsigned nev = slot ? quad_substeps<NQ, true, ROWS>(f, ch, it, tr, x, c2, qlds, stage) : 0u;
-  wave_count(f, nev, slot ? (unsigned)f.nprm : 0u);
-
-  // exchange: as exchange_wave, with slot k of the sequence at lane k * G + g
-  int perm = sl;
+  const double hb = swap_factor(f, sl);
+  unsigned nev = 0;
   int nex = 0;
-  if (B > 1) {
-    SwapDraw d{0, 0.0};
-    if (slot) d = swap_draw(f, iseq, it, sl);
-    const double hk = __shfl(swap_factor(f, sl), (d.k << lg) + g);
-    ladder.slot[lane] = LadderSlot{c2, sl};
-    ladder.pair[lane] = 0;
-    const unsigned long long swapped = ladder_swaps(ladder, slot, (d.k << lg) + g, G, d.k == 0, d.lu, hk);
-    c2 = ladder.slot[lane].c2;
-    perm = ladder.slot[lane].src;
-    if (!burn) nex = __popcll(ladder.pair[lane] & swapped);
-    if (tr.ex && slot && it >= tr.it0 && it < tr.it0 + tr.nit)
-      tr.ex[(size_t)f.tr_ex + ((size_t)(it - tr.it0) * B + sl) * S + iseq] =
-          d.k | ((int)((swapped >> lane) & 1ull) << 16);
-  }
-  const int src = (perm << lg) + g;
-  tc = __shfl(tc, src);
-  // slot lane receives the row that started in slot perm
-  float row[NQ];
+  for (int it = it0; it < it1; ++it) {
+    const FitDesc& f = fit_again(f0);
+    const int B = f.nbeta, S = f.nseq, ch = value_again(ch0);
+    const bool burn = it < f.nburn;
+    if (slot) nev += quad_substeps<NQ, true, ROWS>(f, ch, sl, it, tr, x, c2, q, lds.rows);
+
+    // exchange: as exchange_wave, with slot k of the sequence at lane k * G + g
+    if (B > 1) {
+      SwapDraw d{0, 0.0};
+      if (slot) d = swap_draw(f, iseq, it, sl);
+      const double hk = __shfl(hb, (d.k << lg) + g);
+      lds.ladder.slot[lane] = LadderSlot{c2, sl};
+      lds.ladder.pair[lane] = 0;
+      const unsigned long long swapped = ladder_swaps(lds.ladder, slot, (d.k << lg) + g, G, d.k == 0, d.lu, hk);
+      c2 = lds.ladder.slot[lane].c2;
+      const int src = (lds.ladder.slot[lane].src << lg) + g;
+      if (!burn) nex += __popcll(lds.ladder.pair[lane] & swapped);
+      if (tr.ex && slot && it >= tr.it0 && it < tr.it0 + tr.nit)
+        tr.ex[(size_t)f.tr_ex + ((size_t)(it - tr.it0) * B + sl) * S + iseq] =
+            d.k | ((int)((swapped >> lane) & 1ull) << 16);
+      // slot lane receives the row that started in slot src
+      tc = __shfl(tc, src);
 #pragma unroll
-  for (int i = 0; i < NQ; ++i) row[i] = __shfl(x[i], src);
+      for (int i = 0; i < NQ; ++i) x[i] = __shfl(x[i], src);
+    }
+    if (!burn && f.record) {
+      const int itr = it - f.nburn;
+      if (slot) {
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+          const int ip = f.invar[i];
+          if (ip >= 0) gptr(f.pout)[((size_t)f.nchain * ip + ch) * f.niter + itr] = x[i];
+        }
+        f.tout[(size_t)ch * f.niter + itr] = tc;
+      }
+      if (sl == 0 && seq_ok) f.chi2[(size_t)iseq * f.niter + itr] = c2;
+    }
+  }
   if (slot) {
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) pcur[(size_t)ch * NQ + i] = row[i];
+    for (int i = 0; i < NQ; ++i) pcur[(size_t)ch * NQ + i] = x[i];
     chi2c_a[ch] = c2;
     tcur_a[ch] = tc;
-    if (!burn && nex) gptr(f.n_exch)[ch] += nex;
+    if (nex) gptr(f.n_exch)[ch] += nex;
+    gptr(f.flag)[ch] = q.flag;
+    gptr(f.ptent)[ch] = q.told;
+    gptr(f.ptentn)[ch] = q.tlast;
+    quad_store(f, ch, hist, q);
   }
-  if (!burn && f.record) {
-    const int itr = it - f.nburn;
-    if (slot) {
-#pragma unroll
-      for (int i = 0; i < NQ; ++i) {
-        const int ip = f.invar[i];
-        if (ip >= 0) f.pout[(((size_t)B * ip + sl) * S + iseq) * f.niter + itr] = row[i];
-      }
-      f.tout[(size_t)ch * f.niter + itr] = tc;
-    }
-    if (sl == 0 && seq_ok) f.chi2[(size_t)iseq * f.niter + itr] = c2;
-  }
+  wave_count(f, nev, slot ? (unsigned)(f.nprm * (it1 - it0)) : 0u);
 }
 
-// The rows form keeps every equation's residual in registers; its LDS
-// (rows and stage, 27 KB per work-group at NQ = 8) already limits it to 5
-// waves per SIMD, which is also its register cap.  The full form takes 16 KB
-// per work-group and the register cap of 6 waves (at 7 it spills).
+// The rows form keeps every equation's residual in registers: 4 waves per
+// SIMD; the full form 5 (with one wave more each, both spill inside the
+// proposals).  What bounds it is FP32 issue.  512 systems of 8 equations, 16 x 32
+// chains, an iteration per launch against 64: sampling 37.2 -> 28.1 us an
+// iteration, burn-in (whose per-proposal history and counter accesses kept it
+// waiting on memory) 58.0 -> 35.8 us.
 template <int NQ, bool ROWS>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ROWS ? 5 : 6)))
-k_iter_quad(const FitDesc* fits, const WorkItem* work, int nwork, RunClock* clk, TraceBuf tr, int it_off) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ROWS ? 4 : 5)))
+k_iter_quad(const FitDesc* fits, const WorkItem* work, int nwork, RunClock* clk, TraceBuf tr, int it_off, int iters) {
   const int wv = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
   if (wv >= nwork) return;
   pass_clock(clk);
   const WorkItem w = work[wv];
   const FitDesc& f = wave_fit(fits, w.fit);
-  const int it = __builtin_amdgcn_readfirstlane(load_clock(clk, it_off));
+  const int it0 = __builtin_amdgcn_readfirstlane(load_clock(clk, it_off));
   // 256-thread work-groups: 4 waves
-  __shared__ __align__(16) float qlds[ROWS ? 4 : 1][ROWS ? QROW_LDS : 4];
-  __shared__ __align__(16) float qstage[4][2 * NQ * 64 < (int)sizeof(LadderLds) / 4 ? sizeof(LadderLds) / 4 : 2 * NQ * 64];
-  if (it < f.nburn + f.niter) {
-    // the staged step sizes are written back before the exchange, whose
-    // ladders then take their place
-    float* st = qstage[threadIdx.x >> 6];
-    iter_quad_wave<NQ, ROWS>(f, w.idx, it, tr, ROWS ? qlds[threadIdx.x >> 6] : nullptr, st,
-                             *reinterpret_cast<LadderLds*>(st));
-  }
+  __shared__ QuadLds<NQ, ROWS> lds[4];
+  const int end = f.nburn + f.niter;
+  const int it1 = it0 + iters < end ? it0 + iters : end;
+  if (it0 < it1) iter_quad_wave<NQ, ROWS>(f, w.idx, it0, it1, tr, lds[threadIdx.x >> 6]);
 }
 
 // ---------------------------------------------------------------- launchers
@@ -1327,9 +1375,9 @@ static hipError_t launch_iter_quad_form(int n, const StepLaunch& L, hipStream_t 
   const TraceBuf tr{L.tr_dec, L.tr_chi2, L.tr_ex, L.tr_it0, L.tr_nit};
   const int g = cdiv(L.nwork, 4);   // one work item per wave, 4 waves per work-group
   switch (n) {
-    case 2: k_iter_quad<2, ROWS><<<g, 256, 0, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off); break;
-    case 4: k_iter_quad<4, ROWS><<<g, 256, 0, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off); break;
-    case 8: k_iter_quad<8, ROWS><<<g, 256, 0, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off); break;
+    case 2: k_iter_quad<2, ROWS><<<g, 256, 0, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, L.iters); break;
+    case 4: k_iter_quad<4, ROWS><<<g, 256, 0, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, L.iters); break;
+    case 8: k_iter_quad<8, ROWS><<<g, 256, 0, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, L.iters); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -45,7 +45,6 @@ constexpr int TILE = 64;       // visibilities per wave step
 constexpr int QROW_MAXEQ = 8;
 constexpr int QROW_TS(int n) { return (n + 2) * QROW_MAXEQ + 4; }
 constexpr int QROW_FLOATS(int n) { return n * QROW_TS(n) + QROW_MAXEQ; }
-constexpr int QROW_LDS = 8 * QROW_TS(8);   // per wave: the blocks of the largest system
 
 struct FitDesc {
   // ---- sizes and options
