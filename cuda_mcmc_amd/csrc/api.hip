@@ -102,6 +102,8 @@ struct FitHost {
   std::vector<int> clor;         // 4 per closure: ring byte offsets of the legs, datum
   std::vector<float> clow;       // 4 per closure
   std::vector<int> tinfo;        // 2 per tile: first closure, max u^2+v^2 (float bits)
+  std::vector<int> spass;        // 4 per closure pass (FitDesc::spass)
+  std::vector<int> stile;        // ntile + 1 (FitDesc::stile)
   std::vector<int> clr;          // gradient: leg rounds per closure (color_closure_legs)
   int nround = 0;
   bool ring_grad = false;        // the gradient may use the single-pass ring kernel
@@ -110,7 +112,7 @@ struct FitHost {
   std::vector<int> sumh;
   std::vector<uint32_t> hbits;   // packed acceptance history
   // arena offsets
-  size_t o_vis, o_rho2, o_clo, o_clor, o_clow, o_tinfo, o_qcoef, o_qrow;
+  size_t o_vis, o_rho2, o_clo, o_clor, o_clow, o_tinfo, o_spass, o_stile, o_qcoef, o_qrow;
   size_t o_coor, o_dat, o_std2r, o_icoor, o_idat, o_pdescr, o_ivar, o_invar, o_pmint, o_pmaxt, o_beta;
   size_t o_pcur, o_chi2c, o_pstp, o_ncnt, o_nacpt, o_nhist, o_nexch, o_sumh, o_tcur, o_flag, o_ptent, o_ptentn;
   size_t o_pout, o_tout, o_chi2, o_datm, o_chi2m, o_mc;
@@ -323,6 +325,22 @@ int pack_eht(FitHost& h, int idx) {
     mx = std::nextafter(mx * (1.0f + 1e-6f), INFINITY);
     memcpy(&h.tinfo[2 * t + 1], &mx, 4);
   }
+  // The order in which the one-wave step kernel adds a lane's terms: the tiles
+  // in turn, and after every cgroup-th (and the last) one the closures complete
+  // by then, 64 at a time; a block of 8 tiles starts at a multiple of 8 entries.
+  h.spass.clear();
+  h.stile.clear();
+  int entry = 0, c0 = 0, kleft = h.cgroup;
+  for (int t = 0; t < h.ntile; ++t) {
+    if (t % 8 == 0) entry = (entry + 7) / 8 * 8;
+    h.stile.push_back(entry++);
+    if (--kleft != 0 && t + 1 != h.ntile) continue;
+    kleft = h.cgroup;
+    const int c1 = h.tinfo[2 * (t + 1)];
+    for (int c = c0; c < c1; c += TILE) h.spass.insert(h.spass.end(), {c, std::min(c + TILE, c1), entry++, 0});
+    c0 = std::max(c0, c1);
+  }
+  h.stile.push_back((entry + 7) / 8 * 8);
   // The shift phases need no reduction before the hardware sine when they
   // are bounded well inside its input domain (|h| <= 256 revolutions).
   h.hwphase = eht_phase_bound(h) <= 64.0 && !env_flag("MHRE_REDUCE_PHASES");
@@ -470,6 +488,50 @@ void user_lanes(FitHost& h) {
   h.ulanes = n;
 }
 
+// Waves per chain of the ring+Gaussian fits `idx` of a session: 1 (the grid or
+// persistent form), or 4 or 8 (the split form, k_step_eht_split) for sessions
+// whose chains are few enough that a work-group each is resident on the chip
+// at once, or in two rounds where there is enough to share.  Of 4 and 8 the
+// one with fewer rounds, then the wider.  Measured, us an iteration with 1 / 4
+// / 8 waves per chain, 9 parameters, ladders of 32 rungs:
+//   323 visibilities + 319 closures:  512 chains 47.1 / 32.3 / 29.2,
+//     1024: 52.5 / 40.1 / 48.3, 2048: 65.8 / 61.7 / 96.4
+//   2000 + 600:  512: 110.8 / 51.8 / 43.1, 1024: 113 / 94.4 / 78.1, 2048: 125.7 / 187 / 155
+//   1000 + 300, 2048: 85.5 / 74.5 / 111;  192, 512: 27.3 / 27.3 / 27.7;  256: 29.3 / 28.0 / 27.9
+// With 13 parameters, 323 + 319, 2048 chains: 87.1 / 89.0 / 144, hence two
+// rounds only from SPLIT_TWO_ROUNDS terms per lane on.
+constexpr int SPLIT_LDS = 52 << 10;
+constexpr int SPLIT_MIN_TERMS = 4, SPLIT_TWO_ROUNDS = 16;
+constexpr int SPLIT_WAVES_PER_CU = 16;   // its registers allow 4 waves per SIMD
+
+int eht_split_waves(const std::vector<FitHost>& fits, const std::vector<int>& idx, int ncu, int lds_per_cu) {
+  long long chains = 0;
+  int nt = 0, ne = 0, terms = 0;
+  for (int i : idx) {
+    const FitHost& h = fits[i];
+    const int np = (int)h.spass.size() / 4;
+    // closures recomputed from their visibilities; more than a wave has lanes for
+    if ((h.ncph > 0 && !h.ring_ok) || h.ntile > TILE || np > TILE) return 1;
+    chains += h.nchain;
+    nt = std::max(nt, h.ntile);
+    ne = std::max(ne, h.stile.back());
+    terms = std::max(terms, h.ntile + np);
+  }
+  const int lds = eht_split_lds(nt, ne);
+  if (lds > SPLIT_LDS || terms < SPLIT_MIN_TERMS) return 1;
+  int best = 1;
+  long long best_rounds = terms >= SPLIT_TWO_ROUNDS ? 2 : 1;
+  for (int w : {4, 8}) {
+    const long long at_once = (long long)ncu * std::min(lds_per_cu / (lds + EHT_SPLIT_STATIC_LDS), SPLIT_WAVES_PER_CU / w);
+    const long long rounds = at_once > 0 ? (chains + at_once - 1) / at_once : 1000;
+    if (rounds <= best_rounds) {
+      best = w;
+      best_rounds = rounds;
+    }
+  }
+  return best;
+}
+
 // Most concurrent sequence groups (streams) of a session.
 constexpr int MAX_GROUPS = 8;
 
@@ -514,6 +576,8 @@ struct KindWork {
   bool fused = false;   // step and exchange of whole sequences in one launch, items (fit, first sequence)
   bool rows = false;    // fused quadratic systems: every fit has single-coordinate update rows
   bool one = false;     // fused model.cuh fits: no chain has more data than lanes
+  int split = 1;        // ring+Gaussian: waves per chain of the split form, while the session uses it
+  int max_tile = 0, max_entry = 0;
   int ulanes = 0;       // model.cuh path: lanes per chain
   int max_prm = 0, max_tot = 0;   // model.cuh path: largest nprm, nptot
   std::vector<WorkItem> step, eval;
@@ -557,6 +621,7 @@ struct Session {
   std::vector<Group> groups;
   MhreOptions opt{};
   int wpb = 4, persistent = 0, grid = 0, ncu = 1;
+  bool split = false;   // ring+Gaussian kinds of few chains run in the split form (KindWork::split)
   int waves_per_simd = 0, lds_per_cu = 0;   // occupancy cap of the native step launches
   int graph_iters = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -753,6 +818,9 @@ StepLaunch make_launch(Session* S, const Group& g, const KindWork& k, int it_off
   L.waves_per_simd = S->waves_per_simd;
   L.lds_per_cu = S->lds_per_cu;
   L.iters = 1;
+  L.split = S->split ? k.split : 1;
+  L.max_tile = k.max_tile;
+  L.max_entry = k.max_entry;
   L.ulanes = k.ulanes;
   L.max_prm = k.max_prm;
   L.max_tot = k.max_tot;
@@ -942,9 +1010,13 @@ int autotune(Session* S, int iters, int* best_wpb, int* best_persistent, double*
   if (iters <= 0) FAIL(MHRE_EINVAL, "autotune: iters must be positive");
   double best = 1e300;
   int bw = S->wpb, bp = S->persistent;
+  // a session that splits its chains over waves does so in place of the first
+  // candidate, whose work-groups are the widest too
+  const bool split = S->split;
   for (const auto& c : cand) {
     S->wpb = c[0];
     S->persistent = c[1];
+    S->split = split && c[0] == 4 && c[1] == 0;
     S->grid = std::max(1, S->ncu * (16 / S->wpb));
     double t = 0.0;
     CHK(time_iterations(S, iters, &t));
@@ -956,6 +1028,7 @@ int autotune(Session* S, int iters, int* best_wpb, int* best_persistent, double*
   }
   S->wpb = bw;
   S->persistent = bp;
+  S->split = split && bw == 4 && bp == 0;
   S->grid = std::max(1, S->ncu * (16 / S->wpb));
   drop_graph(S);
   if (best_wpb) *best_wpb = bw;
@@ -998,6 +1071,8 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
   S->wpb = S->opt.waves_per_block == 1 || S->opt.waves_per_block == 2 ? S->opt.waves_per_block : 4;
   S->persistent = S->opt.persistent > 0 ? 1 : 0;
   S->waves_per_simd = std::max(0, S->opt.waves_per_simd);
+  // a launch form that the caller names is the one that runs
+  S->split = S->opt.waves_per_block == 0 && !S->persistent && S->waves_per_simd == 0;
 
   const int it0 = specs[0].it0;
   S->fits.resize(nfits);
@@ -1024,6 +1099,8 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
     h.o_clor = A.reserve<int>(h.clor.size());
     h.o_clow = A.reserve<float>(h.clow.size());
     h.o_tinfo = A.reserve<int>(h.tinfo.size());
+    h.o_spass = A.reserve<int>(h.spass.size());
+    h.o_stile = A.reserve<int>(h.stile.size());
     h.o_qcoef = A.reserve<float>(h.qcoef.size());
     h.o_qrow = A.reserve<float>(h.qrow.size());
     h.o_coor = A.reserve<float>(s.coor ? s.ncoor : 0);
@@ -1074,6 +1151,16 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
     h.d.ndatm = (long long)ndatm;
   }
   // all arguments are validated and packed: now the device resources
+  // persistent grid: a few work-groups per CU
+  int dev = 0, ncu = 0;
+  HIPCHK(hipGetDevice(&dev));
+  HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  S->ncu = ncu;
+  S->grid = std::max(1, ncu * (16 / S->wpb));
+  int lds = 0;
+  if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) != hipSuccess || lds <= 0)
+    lds = 160 << 10;
+  S->lds_per_cu = lds;
   HIPCHK(hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking));
   HIPCHK(hipEventCreate(&S->ev0));
   HIPCHK(hipEventCreate(&S->ev1));
@@ -1123,6 +1210,7 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
     d.record = h.record ? 1 : 0;
     d.vis = at<float4>(S, h.o_vis); d.rho2 = at<float>(S, h.o_rho2);
     d.clo = at<int4>(S, h.o_clo); d.clor = at<int4>(S, h.o_clor); d.clow = at<float4>(S, h.o_clow);
+    d.spass = at<int4>(S, h.o_spass); d.stile = at<int>(S, h.o_stile); d.nspass = (int)h.spass.size() / 4;
     d.tinfo = at<int2>(S, h.o_tinfo); d.qcoef = at<float>(S, h.o_qcoef);
     d.qrow = h.qrow.empty() ? nullptr : at<float>(S, h.o_qrow);
     d.coor = at<float>(S, h.o_coor); d.dat = at<float>(S, h.o_dat); d.std2r = at<float>(S, h.o_std2r);
@@ -1157,6 +1245,8 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
     U.add(h.o_clor, h.clor.data(), h.clor.size());
     U.add(h.o_clow, h.clow.data(), h.clow.size());
     U.add(h.o_tinfo, h.tinfo.data(), h.tinfo.size());
+    U.add(h.o_spass, h.spass.data(), h.spass.size());
+    U.add(h.o_stile, h.stile.data(), h.stile.size());
     U.add(h.o_qcoef, h.qcoef.data(), h.qcoef.size());
     U.add(h.o_qrow, h.qrow.data(), h.qrow.size());
     U.add(h.o_coor, s.coor, s.coor ? s.ncoor : 0);
@@ -1359,6 +1449,11 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
       kw.qslot = qslot++;
       for (int i : idx) chains(i, kw.step);
       if (kw.step.empty()) continue;
+      kw.split = eht_split_waves(S->fits, idx, S->ncu, S->lds_per_cu);
+      for (int i : idx) {
+        kw.max_tile = std::max(kw.max_tile, S->fits[i].ntile);
+        kw.max_entry = std::max(kw.max_entry, S->fits[i].stile.back());
+      }
       kw.xr = deal_xcd(kw.step, fit_cost);
       grp.kinds.push_back(std::move(kw));
     }
@@ -1408,17 +1503,6 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
   CHK(dev_alloc(S, &S->d_init, init.size()));
   if (!init.empty())
     HIPCHK(hipMemcpyAsync(S->d_init, init.data(), init.size() * sizeof(WorkItem), hipMemcpyHostToDevice, S->stream));
-
-  // persistent grid: a few work-groups per CU
-  int dev = 0, ncu = 0;
-  HIPCHK(hipGetDevice(&dev));
-  HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  S->ncu = ncu;
-  S->grid = std::max(1, ncu * (16 / S->wpb));
-  int lds = 0;
-  if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) != hipSuccess || lds <= 0)
-    lds = 160 << 10;
-  S->lds_per_cu = lds;
 
   // decision trace of iterations it0 .. it0 + trace_iters - 1
   if (S->opt.trace_iters > 0) {
@@ -1932,6 +2016,12 @@ int mhre_session_fit_info(const void* session, int fit, int* info, int ninfo) {
   info[2] = h.hwphase ? 1 : 0;
   info[3] = (int)S->groups.size();
   if (ninfo >= 5) info[4] = h.qrow.empty() ? 0 : 1;
+  if (ninfo >= 6) {
+    info[5] = h.kind == K_USER ? h.ulanes : 1;
+    if (S->split && !S->groups.empty())
+      for (const KindWork& k : S->groups[0].kinds)
+        if (k.kind == h.kind && h.kind != K_USER) info[5] = k.split;
+  }
   return MHRE_OK;
 }
 

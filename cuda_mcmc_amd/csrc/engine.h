@@ -107,6 +107,8 @@ struct StepLaunch {
   int waves_per_simd;    // > 0: cap on resident waves per SIMD (LDS reserved per work-group)
   int lds_per_cu;        // bytes of LDS per compute unit
   int iters;             // launches that hold whole sequences: iterations it_off .. it_off + iters - 1
+  int split;             // ring+Gaussian: waves per chain (one work-group each) if above 1
+  int max_tile, max_entry;   // split form: most tiles, and chi^2 terms per lane, of the list's fits
   int ulanes;            // model.cuh path: lanes per chain of the list's fits
   int max_prm, max_tot;  // model.cuh path: largest nprm and nptot of the list's fits
   int* tr_dec; float* tr_chi2; int* tr_ex; int tr_it0; int tr_nit;   // optional decision trace
@@ -116,6 +118,9 @@ hipError_t launch_init(const FitDesc* fits, const WorkItem* work, int nwork, hip
 hipError_t launch_eval_eht(int model, const FitDesc* fits, const WorkItem* work, int nwork, int outputs,
                            int respect_flag, hipStream_t s);
 hipError_t launch_step_eht(int model, const StepLaunch& L, hipStream_t s);
+// LDS of the split step form's model visibilities and term factors.
+constexpr int eht_split_lds(int ntile, int nentry) { return (ntile + nentry) * TILE * (int)sizeof(float2); }
+constexpr int EHT_SPLIT_STATIC_LDS = 12 << 10;   // bound of its other LDS (Bessel table, prologue)
 hipError_t launch_eval_quad(int n, const FitDesc* fits, const WorkItem* work, int nwork, hipStream_t s);
 hipError_t launch_step_quad(int n, const StepLaunch& L, hipStream_t s);
 // L.iters iterations (step + exchange) of whole sequences (ladders of at most

@@ -73,6 +73,10 @@ struct EhtView {
   const GLOBAL int4* clor;
   const GLOBAL float4* clow;
   const CONSTANT int2* tinfo;   // per-tile entries: read with scalar loads
+  const GLOBAL int4* spass;
+  const GLOBAL int* stile;
+  const GLOBAL int2* tinfo_g;
+  int nspass;
   GLOBAL float* datm;
   GLOBAL float* chi2m;
   long long ndatm;
@@ -86,6 +90,7 @@ __device__ inline EhtView eht_view(const FitDesc& f) {
   v.datm = gptr(f.datm); v.chi2m = gptr(f.chi2m); v.ndatm = f.ndatm;
   v.nvis = f.nvis; v.ncph = f.ncph; v.ntile = f.ntile; v.ring_ok = f.ring_ok; v.cgroup = f.cgroup;
   v.ndat = f.ndat; v.nchain = f.nchain;
+  v.spass = gptr(f.spass); v.stile = gptr(f.stile); v.tinfo_g = gptr(f.tinfo); v.nspass = f.nspass;
   return v;
 }
 
@@ -98,15 +103,20 @@ __device__ inline void ring_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
-// Closure term from three model visibilities: the residual
+// Closure residual (and its weighted square, closure_term) from three model
+// visibilities:
 // wrap(obs - (pa + pb - pc)) as arg(e^{i obs} conj(a b conj(c))).
-__device__ inline float closure_term(float2 a, float2 b, float2 e, float4 ow, float* model_cph) {
+__device__ inline float closure_resid(float2 a, float2 b, float2 e, float4 ow, float* model_cph) {
   const float abr = a.x * b.x - a.y * b.y, abi = a.x * b.y + a.y * b.x;
   const float br = abr * e.x + abi * e.y, bi = abi * e.x - abr * e.y;   // a b conj(e)
   const float xr = ow.x * br + ow.y * bi;
   const float xi = ow.y * br - ow.x * bi;
   const float dd = atan2_fast(xi, xr);
   if (model_cph) *model_cph = atan2_fast(bi, br);
+  return dd;
+}
+__device__ inline float closure_term(float2 a, float2 b, float2 e, float4 ow, float* model_cph) {
+  const float dd = closure_resid(a, b, e, ow, model_cph);
   return dd * dd * ow.z;
 }
 
@@ -311,32 +321,65 @@ __global__ void __launch_bounds__(256) k_eval_eht(const FitDesc* fits, const Wor
 
 // ------------------------------------------------------------ step kernel
 
+// A wave's LDS before its first chi^2: the random numbers of its iteration,
+// then the ladder of the exchange.
+constexpr int MAX_DRAWS = 64 + 2 * MAXP;
+struct StepPrologue {
+  LadderLds ladder;
+  double v[MAX_DRAWS];
+  int k[MAX_DRAWS];
+};
+
+// The random numbers of a chain's iteration it and of the nB swap attempts of
+// its sequence's exchange before it: entry a < nB the attempt's pair and log u,
+// entry nB + s substep s's coordinate pick and log u, entry nB + nprm + s its
+// Gaussian step.  One entry a lane, so that all of them cost one Philox block, one
+// float64 logarithm and one cosine (a second time beyond 64 entries), with one
+// copy of that code: a launch meets every line of it cold.
+__device__ inline void step_draws(const FitDesc& f, int ch, int iseq, int it, int nB, StepPrologue& pro) {
+  const int P = f.nprm, n = nB + 2 * P;
+#pragma unroll 1
+  for (int e = lane_id(); e < n; e += 64) {
+    const bool swap = e < nB, gauss = e >= nB + P;
+    const uint32_t c0 = swap ? iseq : ch, c1 = swap ? it - 1 : it;
+    const uint32_t c2 = swap ? e : gauss ? e - nB - P : e - nB, c3 = swap ? RNG_EXCH : 0u;
+    const U4 r = philox4x32_10(c0, c1, c2, c3, f.key0, f.key1);
+    // the logarithm's argument: log u of a swap is word 1, of a proposal word
+    // 3; the Gaussian step (normal64) starts from word 1
+    const double lu = log((double)u01(swap || gauss ? r.y : r.w));
+    double v = lu;
+    if (gauss) v = sqrt(-2.0 * lu) * cos(6.283185307179586 * (double)u01(r.z));
+    pro.v[e] = v;
+    if (!gauss) pro.k[e] = pick_with_retry(r.x, swap ? nB - 1 : P, c0, c1, c2, c3, f.key0, f.key1);
+  }
+  wave_sync_lds();
+}
+
 // The replica exchange of iteration itp of sequence iseq (reference:
 // gpu_mcmc.cu:548-624, the same draws and arithmetic as exchange_wave),
 // computed inside one wave whose lane j holds temperature slot j (B <= 64)
-// with chi^2 and labels read from c2s and tcs.  Every wave of the sequence
+// with its chi^2 c2 and label tc0.  Every wave of the sequence
 // computes it and keeps what its own slot sl needs: the slot whose row ends
 // up in sl, and sl's chi^2 and label after the swaps.  It also does the
 // exchange launch's per-slot writes for sl (n_exch) and, in slot 0's wave,
 // the sequence's trace entries.  Labels move with the rows, so sl's label is
 // the one its row started with.
-static_assert(sizeof(LadderLds) <= sizeof(float2) * RING, "the swaps use the wave's ring");
+static_assert(sizeof(StepPrologue) <= sizeof(float2) * RING, "the prologue uses the wave's ring");
 struct SlotAfterSwaps {
   int src;
   float c2;
   int tc;
 };
-__device__ inline SlotAfterSwaps seq_exchange(const FitDesc& f, int iseq, int sl, int itp, const float* c2s,
-                                              const int* tcs, const TraceBuf& tr, LadderLds& ladder) {
+__device__ inline SlotAfterSwaps seq_exchange(const FitDesc& f, int iseq, int sl, int itp, float c2, int tc0,
+                                              const TraceBuf& tr, StepPrologue& pro) {
   const int lane = lane_id();
   const int B = f.nbeta, S = f.nseq;
   const bool burn = itp < f.nburn;
   const bool slot = lane < B;
-  const float c2 = slot ? c2s[(size_t)lane * S + iseq] : 0.0f;
-  const int tc0 = slot ? tcs[(size_t)lane * S + iseq] : 0;
   if (B < 2) return SlotAfterSwaps{sl, bcast(c2, sl), bcast(tc0, sl)};
+  LadderLds& ladder = pro.ladder;
   SwapDraw d{0, 0.0};
-  if (slot) d = swap_draw(f, iseq, itp, lane);
+  if (slot) d = SwapDraw{pro.k[lane], pro.v[lane]};
   const double hk = __shfl(swap_factor(f, lane), d.k);
   ladder.slot[lane] = LadderSlot{c2, lane};
   ladder.pair[lane] = 0;
@@ -351,14 +394,204 @@ __device__ inline SlotAfterSwaps seq_exchange(const FitDesc& f, int iseq, int sl
   return SlotAfterSwaps{src, __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(me.c2))), bcast(tc0, src)};
 }
 
+// chi^2 of a chain's proposals by the one wave that runs it.
+template <class M>
+struct WaveChi2 {
+  const EhtView& v;
+  float2* ring;
+  const BesselTab& bt;
+  int ch;
+  __device__ void setup() {}
+  __device__ StepPrologue& prologue() const { return *reinterpret_cast<StepPrologue*>(ring); }
+  template <bool HW>
+  __device__ double chi2(const typename M::Inv& q) { return eht_chi2_wave<M, false, HW>(v, q, ring, bt, ch); }
+};
+
+// chi^2 of a chain's proposals by the W waves of a work-group, for sessions of
+// few chains: there one wave per chain leaves most of the chip idle and spends
+// most of its own time waiting for its LDS reads and arithmetic.  Wave 0 runs
+// the chain; the others wait at the barrier for the invariants of its next
+// proposal and take their share of the data: wave w models tiles w, w + W, ...
+// into vis, then forms closure passes w, w + W, ....  The terms meet in LDS in
+// the order in which one wave would add them, each as the two factors of a
+// product (r r of a visibility, w dd^2 of a closure), and are added in that
+// order, in fp32 over the blocks of 8 tiles (padded with zero terms to a
+// multiple of 8) and then in fp64, so that the chi^2 has the bits of
+// eht_chi2_wave.  Wave 0 adds them all, or beyond SPLIT_TRIPS blocks every
+// wave its share of the blocks (the fp64 sums are then added in another order,
+// which the chi^2, rounded to fp32, does not show).
+constexpr int SPLIT_TRIPS = 2;
+constexpr int SPLIT_MAXW = 8;
+template <class M>
+struct SplitLds {
+  typename M::Inv q;
+  double xs[SPLIT_MAXW];
+  int go;   // 1: model q, 0: the iteration is over
+};
+template <class M>
+struct SplitChi2 {
+  const EhtView& v;
+  const BesselTab& bt;
+  float2* vis;        // [ntile * TILE] model visibilities
+  float2* term;       // [entries * TILE] factors of the terms
+  SplitLds<M>& sh;
+  StepPrologue* pro;  // wave 0's
+  int wid, W;
+  // the wave's first tile and pass (the same for every proposal), and lane i's
+  // tile i (its term's entry, the bound of its u^2 + v^2) and pass i:
+  // read with lane reads, as a scalar load in flight would hold up every LDS
+  // read behind it
+  float4 d0, ow0;
+  float r20;
+  int4 ix0;
+  int eall, e_l, pc_l, pe_l, pt_l;
+  uint32_t r2max_l;
+
+  __device__ StepPrologue& prologue() const { return *pro; }
+  __device__ int entry(int t) const { return __builtin_amdgcn_readlane(e_l, t); }
+  __device__ uint32_t r2max(int t) const { return (uint32_t)__builtin_amdgcn_readlane((int)r2max_l, t); }
+  __device__ uint32_t first_closure(int p) const { return (uint32_t)__builtin_amdgcn_readlane(pc_l, p); }
+  __device__ void setup() {
+    // past the fit's data: the padding behind the last tile, and pass 0's
+    // closures, neither of which is used
+    const int lane = lane_id();
+    const uint32_t l = (uint32_t)lane;
+    const int nt = v.ntile, np = v.nspass;
+    e_l = lane < nt ? ldg(v.stile, lane) : 0;
+    eall = __builtin_amdgcn_readfirstlane(ldg(v.stile, nt));
+    r2max_l = lane < nt ? (uint32_t)ldg(v.tinfo_g, lane).y : 0u;
+    int4 ps = make_int4(0, 0, 0, 0);
+    if (lane < np) ps = ldg(v.spass, lane);
+    pc_l = ps.x;
+    pe_l = ps.y;
+    pt_l = ps.z;
+    const int t = wid < nt ? wid : nt;
+    const BufRsrc vb = make_buf(v.vis, (uint32_t)(nt + 1) * TILE * 16u);
+    const BufRsrc rb = make_buf(v.rho2, (uint32_t)(nt + 1) * TILE * 4u);
+    d0 = buf_load_f4(vb, l * 16u, (uint32_t)t * 1024u);
+    r20 = buf_load_f(rb, l * 4u, (uint32_t)t * 256u);
+    const uint32_t c = first_closure(wid < np ? wid : 0) * 16u;
+    const BufRsrc cb = make_buf(v.clo, (uint32_t)(v.ncph + TILE) * 16u);
+    const BufRsrc wb = make_buf(v.clow, (uint32_t)(v.ncph + TILE) * 16u);
+    ix0 = buf_load_i4(cb, l * 16u, c);
+    ow0 = buf_load_f4(wb, l * 16u, c);
+  }
+
+  // Waves 1 .. W - 1.
+  template <bool HW>
+  __device__ void work() {
+    setup();
+    for (int i = (int)threadIdx.x - 64; i < eall * TILE; i += 64 * (W - 1)) term[i] = make_float2(0.0f, 0.0f);
+    for (;;) {
+      __syncthreads();
+      if (sh.go == 0) break;
+      const typename M::Inv q = sh.q;
+      share<HW>(q);
+    }
+  }
+  // Wave 0, after its last proposal.
+  __device__ void finish() {
+    if (lane_id() == 0) sh.go = 0;
+    __syncthreads();
+  }
+  template <bool HW>
+  __device__ double chi2(const typename M::Inv& q) {
+    if (lane_id() == 0) {
+      sh.q = q;
+      sh.go = 1;
+    }
+    __syncthreads();
+    return share<HW>(q);
+  }
+
+  // This wave's share; every wave of the work-group passes the same barriers.
+  // Returns the chi^2 on wave 0.
+  template <bool HW>
+  __device__ double share(const typename M::Inv& q) {
+    const int lane = lane_id();
+    const uint32_t l16 = (uint32_t)lane * 16u, l4 = (uint32_t)lane * 4u;
+    const uint32_t r2_thr = __builtin_amdgcn_readfirstlane(q.r.r2thr);
+    const int nt = __builtin_amdgcn_readfirstlane(v.ntile), np = __builtin_amdgcn_readfirstlane(v.nspass);
+    const BufRsrc vb = make_buf(v.vis, (uint32_t)(nt + 1) * TILE * 16u);
+    const BufRsrc rb = make_buf(v.rho2, (uint32_t)(nt + 1) * TILE * 4u);
+    float4 d = d0, dn;
+    float r2 = r20, r2n;
+    for (int t = wid; t < nt;) {
+      // the next one, if there is any: an unused load would be waited for
+      const bool more = t + W < nt;
+      if (more) {
+        dn = buf_load_f4(vb, l16, (uint32_t)(t + W) * 1024u);
+        r2n = buf_load_f(rb, l4, (uint32_t)(t + W) * 256u);
+      }
+      const float2 V = M::template vis<BesselTab, HW>(q, d.x, d.y, r2, r2max(t) > r2_thr, bt);
+      const float r = fmaf(-__builtin_amdgcn_sqrtf(fmaf(V.x, V.x, V.y * V.y)), d.w, d.z);
+      vis[t * TILE + lane] = V;
+      term[entry(t) * TILE + lane] = make_float2(r, r);
+      if (!more) break;
+      d = dn;
+      r2 = r2n;
+      t += W;
+    }
+    __syncthreads();
+    if (np > 0) {
+      const BufRsrc cb = make_buf(v.clo, (uint32_t)(v.ncph + TILE) * 16u);
+      const BufRsrc wb = make_buf(v.clow, (uint32_t)(v.ncph + TILE) * 16u);
+      int4 ix = ix0, ixn;
+      float4 ow = ow0, own;
+      for (int p = wid; p < np;) {
+        const bool more = p + W < np;
+        if (more) {
+          const uint32_t c = first_closure(p + W) * 16u;
+          ixn = buf_load_i4(cb, l16, c);
+          own = buf_load_f4(wb, l16, c);
+        }
+        // closures past the pass's end are not formed yet
+        const bool on = (int)first_closure(p) + lane < __builtin_amdgcn_readlane(pe_l, p);
+        const float dd = closure_resid(vis[ix.x], vis[ix.y], vis[ix.z], ow, nullptr);
+        term[__builtin_amdgcn_readlane(pt_l, p) * TILE + lane] = on ? make_float2(ow.z, dd * dd) : make_float2(0.0f, 0.0f);
+        if (!more) break;
+        ix = ixn;
+        ow = own;
+        p += W;
+      }
+      __syncthreads();
+    }
+    const int ntrip = (nt + 7) / 8;
+    const bool all = ntrip > SPLIT_TRIPS;   // every wave adds its blocks
+    double acc = 0.0;
+    if (all || wid == 0) {
+      for (int k = all ? wid : 0; k < ntrip; k += all ? W : 1) {
+        const int end = 8 * k + 8 < nt ? entry(8 * k + 8) : eall;
+        float part = 0.0f;
+        for (int e = entry(8 * k); e < end; e += 8) {
+          float2 f[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) f[i] = term[(e + i) * TILE + lane];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) part = fmaf(f[i].x, f[i].y, part);
+        }
+        acc += (double)part;
+      }
+      acc = wave_sum(acc);
+    }
+    if (all) {
+      if (lane == 0) sh.xs[wid] = acc;
+      __syncthreads();
+      acc = 0.0;
+      for (int w = 0; w < W; ++w) acc += sh.xs[w];
+    }
+    return acc;
+  }
+};
+
 // One MH iteration of chain ch (all nprm single-parameter proposals) by one
-// wave.  With f.xfused the launch at offset it_off > 0 of its segment first
+// wave (the chi^2 of its proposals by ev).  With f.xfused the launch at offset it_off > 0 of its segment first
 // runs the exchange of iteration it - 1 (the state arrays alternate between
 // the two sets by the parity of it_off); for it past the fit's last iteration
 // only that exchange runs.
-template <class M>
-__device__ __attribute__((always_inline)) void step_one_chain(const FitDesc& f, int ch, int it, int it_off, float2* ring,
-                               typename M::RingPart* rcache, const BesselTab& bt, const TraceBuf& tr) {
+template <class M, class EV>
+__device__ __attribute__((always_inline)) void step_one_chain(const FitDesc& f, int ch, int it, int it_off, EV& ev,
+                               typename M::RingPart* rcache, const TraceBuf& tr) {
   const int lane = lane_id();
   const int C = f.nchain, P = f.nprm, N = f.nptot;
   const int ibeta = ch / f.nseq;
@@ -377,6 +610,31 @@ __device__ __attribute__((always_inline)) void step_one_chain(const FitDesc& f, 
   int sh = (burn && lane < P) ? f.sumh[(size_t)lane * C + ch] : 0;
   const double beta = (double)f.beta[ibeta];
 
+  // the sequence's chi^2 and labels before the exchange, slot j on lane j
+  const int iseq = ch - ibeta * f.nseq;
+  const bool odd = (it_off & 1) != 0;
+  float c2_l = 0.0f;
+  int tc_l = 0;
+  if (f.xfused && it_off > 0 && lane < f.nbeta) {
+    const size_t me = (size_t)lane * f.nseq + iseq;
+    c2_l = (odd ? f.chi2c : f.chi2c_b)[me];
+    tc_l = (odd ? f.tcur : f.tcur_b)[me];
+  }
+
+  // This iteration's random numbers and those of the exchange before it.  They
+  // need none of the chain's state, so they come first and hide the loads above.
+  const bool swaps = f.xfused && it_off > 0 && f.nbeta > 1;
+  const int nB = swaps ? f.nbeta : 0;
+  StepPrologue& pro = ev.prologue();
+  step_draws(f, ch, iseq, it, nB, pro);
+  int k_l = 0;
+  double z_l = 0.0, lu_l = 0.0;
+  if (lane < P) {
+    k_l = pro.k[nB + lane];
+    lu_l = pro.v[nB + lane];
+    z_l = pro.v[nB + P + lane];
+  }
+
   // the chain's state before the step (after the previous exchange), and
   // where the state after the step goes
   float* pdst = f.pcur;
@@ -386,15 +644,11 @@ __device__ __attribute__((always_inline)) void step_one_chain(const FitDesc& f, 
   float chi2c;
   int tc = 0;
   if (f.xfused) {
-    const bool odd = (it_off & 1) != 0;
     if (odd) { pdst = f.pcur_b; cdst = f.chi2c_b; }
     tdst = odd ? f.tcur_b : f.tcur;
     if (it_off > 0) {
-      const int iseq = ch - ibeta * f.nseq;
       const float* ps = odd ? f.pcur : f.pcur_b;
-      const SlotAfterSwaps x = seq_exchange(f, iseq, ibeta, it - 1, odd ? f.chi2c : f.chi2c_b,
-                                            odd ? f.tcur : f.tcur_b, tr,
-                                            *reinterpret_cast<LadderLds*>(ring));   // not yet used by the chi^2
+      const SlotAfterSwaps x = seq_exchange(f, iseq, ibeta, it - 1, c2_l, tc_l, tr, pro);
       ring_fence();
       pl = lane < N ? ps[((size_t)x.src * f.nseq + iseq) * N + lane] : 0.0f;
       chi2c = x.c2;
@@ -429,17 +683,18 @@ __device__ __attribute__((always_inline)) void step_one_chain(const FitDesc& f, 
     chi2c = f.chi2c[ch];
   }
 
-  // lane j keeps the history word holding entry cnt % nadj of parameter j
-  int hw_idx = 0;
+  // lane j keeps the history word holding entry pos = cnt % nadj of parameter j
+  int pos = 0;
   uint32_t hword = 0u;
+  const int nadj = f.nadj;
   if (burn && lane < P) {
-    hw_idx = (cnt % f.nadj) >> 5;
-    hword = f.hbits[(ch * f.hwords + hw_idx) * P + lane];
+    pos = cnt % nadj;
+    hword = f.hbits[(ch * f.hwords + (pos >> 5)) * P + lane];
   }
   int flag = 0, tlast = 0;
   float told = 0.0f;
   unsigned nev = 0;
-  const EhtView view = eht_view(f);
+  ev.setup();
   // the float64 trigonometric invariants of the current state, and its ring
   // group (M::RingPart) in the wave's LDS slot rcache[rci]: a proposal that
   // moves neither recomputes only the cheap rest of the invariants.  A
@@ -453,18 +708,6 @@ __device__ __attribute__((always_inline)) void step_one_chain(const FitDesc& f, 
     gather_params<M>(pl, p);
     tg = M::trig(p);
     rcache[0] = M::ring_part(p, tg);
-  }
-
-  // This iteration's random numbers, substep s on lane s: the coordinate
-  // pick, the Gaussian step and log u of the accept test (drawn for every
-  // substep; counter-based, so unused draws shift nothing).
-  int k_l = 0;
-  double z_l = 0.0, lu_l = 0.0;
-  if (lane < P) {
-    const U4 r = philox4x32_10((uint32_t)ch, (uint32_t)it, (uint32_t)lane, 0u, f.key0, f.key1);
-    k_l = pick_with_retry(r.x, P, (uint32_t)ch, (uint32_t)it, (uint32_t)lane, 0u, f.key0, f.key1);
-    z_l = normal64(r.y, r.z);
-    lu_l = log((double)u01(r.w));
   }
 
   for (int s = 0; s < P; ++s) {
@@ -493,8 +736,7 @@ __device__ __attribute__((always_inline)) void step_one_chain(const FitDesc& f, 
       }
       const typename M::Inv q = M::assemble(p, tn, rp);
       // one copy of the chi^2 loop per phase form (the branch is per wave)
-      c2 = f.hwphase ? eht_chi2_wave<M, false, true>(view, q, ring, bt, ch)
-                     : eht_chi2_wave<M, false, false>(view, q, ring, bt, ch);
+      c2 = f.hwphase ? ev.template chi2<true>(q) : ev.template chi2<false>(q);
       ++nev;
       const double x = -0.5 * beta * (c2 - (double)chi2c);
       if (bcast(lu_l, s) <= x) {
@@ -511,23 +753,21 @@ __device__ __attribute__((always_inline)) void step_one_chain(const FitDesc& f, 
     told = old;
     tlast = t;
     if (burn && lane == k) {
-      // history entry cnt % nadj: the oldest one, replaced by this outcome
+      // history entry pos = cnt % nadj: the oldest one, replaced by this outcome
       // (the division-free forms of mhre_device.h give the reference's bits)
-      const int nadj = f.nadj;
-      const float rnadj = 1.0f / (float)nadj;
-      const uint32_t bit = 1u << (mod_small(cnt, nadj, rnadj) & 31);
+      const uint32_t bit = 1u << (pos & 31);
       const int hold = (hword & bit) ? 1 : 0;
       hword = acc ? (hword | bit) : (hword & ~bit);
       sh += acc - hold;
       const int den = cnt < nadj ? cnt : nadj;
       stp = rate_below(sh, den, f.adapt_mid, f.adapt_tie) ? step_shrink(stp) : step_grow(stp);
       ++cnt;
-      const int w2 = mod_small(cnt, nadj, rnadj) >> 5;
-      if (w2 != hw_idx) {
-        f.hbits[(ch * f.hwords + hw_idx) * P + lane] = hword;
-        hw_idx = w2;
-        hword = f.hbits[(ch * f.hwords + hw_idx) * P + lane];
+      const int next = pos + 1 == nadj ? 0 : pos + 1;
+      if ((next >> 5) != (pos >> 5)) {   // the word is full: on to the next one
+        f.hbits[(ch * f.hwords + (pos >> 5)) * P + lane] = hword;
+        hword = f.hbits[(ch * f.hwords + (next >> 5)) * P + lane];
       }
+      pos = next;
     }
     if (tr.dec && it >= tr.it0 && it < tr.it0 + tr.nit && lane == 0) {
       const size_t ti = (size_t)f.tr_dec + ((size_t)(it - tr.it0) * P + s) * C + ch;
@@ -543,7 +783,7 @@ __device__ __attribute__((always_inline)) void step_one_chain(const FitDesc& f, 
     f.n_acpt[(size_t)lane * C + ch] = nac;
     if (burn) {
       f.sumh[(size_t)lane * C + ch] = sh;
-      f.hbits[(ch * f.hwords + hw_idx) * P + lane] = hword;
+      f.hbits[(ch * f.hwords + (pos >> 5)) * P + lane] = hword;
     }
   }
   if (lane == 0) {
@@ -601,7 +841,10 @@ __global__ void __launch_bounds__(64 * WPB) k_step_eht(const FitDesc* fits, cons
     const WorkItem w = work[wv];
     const FitDesc& f = wave_fit(fits, w.fit);
     if (it > last_busy_it(f, it_off)) return;
-    step_one_chain<M>(f, __builtin_amdgcn_readfirstlane(w.idx), it, it_off, ring, rcache, bt, tr);
+    const int ch = __builtin_amdgcn_readfirstlane(w.idx);
+    const EhtView view = eht_view(f);
+    WaveChi2<M> ev{view, ring, bt, ch};
+    step_one_chain<M>(f, ch, it, it_off, ev, rcache, tr);
   } else {
     const int hs = it_off & 1;
     for (int r = 0; r < NXCD; ++r) {
@@ -611,10 +854,53 @@ __global__ void __launch_bounds__(64 * WPB) k_step_eht(const FitDesc* fits, cons
       for (int j = grab_item(clk, hs, q); j < len; j = grab_item(clk, hs, q)) {
         const WorkItem w = work[base + j];
         const FitDesc& f = wave_fit(fits, w.fit);
-        if (it <= last_busy_it(f, it_off))
-          step_one_chain<M>(f, __builtin_amdgcn_readfirstlane(w.idx), it, it_off, ring, rcache, bt, tr);
+        if (it <= last_busy_it(f, it_off)) {
+          const int ch = __builtin_amdgcn_readfirstlane(w.idx);
+          const EhtView view = eht_view(f);
+          WaveChi2<M> ev{view, ring, bt, ch};
+          step_one_chain<M>(f, ch, it, it_off, ev, rcache, tr);
+        }
       }
     }
+  }
+}
+
+// One work-group of blockDim.x / 64 waves per chain (SplitChi2); work-group b
+// serves the range of XCD b % NXCD.  ntile: the most tiles of the list's fits
+// (the place of the terms in the dynamic LDS).
+template <class M>
+__global__ void __launch_bounds__(64 * SPLIT_MAXW) __attribute__((amdgpu_waves_per_eu(4))) k_step_eht_split(const FitDesc* fits, const WorkItem* work,
+                                                                    XcdRanges xr, RunClock* clk, TraceBuf tr,
+                                                                    int it_off, int ntile) {
+  __shared__ float4 btab[2 * BESSEL_TAB_N];
+  __shared__ typename M::RingPart rcache[2];
+  __shared__ SplitLds<M> sh;
+  __shared__ StepPrologue pro;
+  extern __shared__ __align__(16) char lds[];
+  pass_clock(clk);
+  load_bessel_tab(btab);
+  const BesselTab bt{btab};
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int W = __builtin_amdgcn_readfirstlane((int)(blockDim.x >> 6));
+  const int it = __builtin_amdgcn_readfirstlane(load_clock(clk, it_off));
+  const int xb = (int)(blockIdx.x % NXCD);
+  const int wv = xr.off[xb] + (int)(blockIdx.x / NXCD);
+  if (wv >= xr.off[xb + 1]) return;
+  const WorkItem w = work[wv];
+  const FitDesc& f = wave_fit(fits, w.fit);
+  if (it > last_busy_it(f, it_off)) return;
+  const int ch = __builtin_amdgcn_readfirstlane(w.idx);
+  const EhtView view = eht_view(f);
+  static_assert(sizeof(btab) + sizeof(rcache) + sizeof(sh) + sizeof(pro) <= EHT_SPLIT_STATIC_LDS, "occupancy rule");
+  float2* vis = reinterpret_cast<float2*>(lds);
+  SplitChi2<M> ev{view, bt, vis, vis + ntile * TILE, sh, &pro, wid, W};
+  if (wid == 0) {
+    step_one_chain<M>(f, ch, it, it_off, ev, rcache, tr);
+    ev.finish();
+  } else if (f.hwphase) {
+    ev.template work<true>();
+  } else {
+    ev.template work<false>();
   }
 }
 
@@ -1339,8 +1625,20 @@ static void launch_step_m(const StepLaunch& L, hipStream_t s) {
   }
 }
 
+template <class M>
+static void launch_step_split(const StepLaunch& L, hipStream_t s) {
+  const TraceBuf tr{L.tr_dec, L.tr_chi2, L.tr_ex, L.tr_it0, L.tr_nit};
+  k_step_eht_split<M><<<xcd_grid(L.xr, 1), 64 * L.split, eht_split_lds(L.max_tile, L.max_entry), s>>>(
+      L.fits, L.work, L.xr, L.clk, tr, L.it_off, L.max_tile);
+}
+
 hipError_t launch_step_eht(int model, const StepLaunch& L, hipStream_t s) {
   if (L.nwork <= 0) return hipSuccess;
+  if (L.split > 1) {
+    if (model == MODEL_SGRA9) launch_step_split<Sgra9>(L, s);
+    else launch_step_split<Sgra13>(L, s);
+    return hipGetLastError();
+  }
   if (model == MODEL_SGRA9) launch_step_m<Sgra9>(L, s);
   else launch_step_m<Sgra13>(L, s);
   return hipGetLastError();

@@ -88,6 +88,14 @@ struct FitDesc {
   const int2* tinfo;       // [ntile + 2] per tile t: first closure whose largest index
                            // lies past tile t - 1, and the max u^2+v^2 of tile t's
                            // visibilities (float bits)
+  // Order of a chi^2's terms per lane, for the step kernel that splits a chain
+  // over the waves of a work-group: entry stile[t] is tile t's residual, a
+  // closure pass (at most 64 closures formed together) the entry spass[p].z
+  // behind the tile after which the one-wave kernel forms it.  Every block of 8
+  // tiles starts at a multiple of 8; entries that nothing names are zero.
+  const int4* spass;       // [nspass] first closure, end, entry, 0
+  const int* stile;        // [ntile + 1] entry of each tile, then their number
+  int nspass;
   const int* clr;          // [ncph + TILE] gradient only: round of each closure leg
                            // (4 bits per leg), no two legs of one 64-closure batch
                            // and round naming the same visibility; null elsewhere

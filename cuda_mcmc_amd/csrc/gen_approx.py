@@ -180,7 +180,7 @@ def main():
     print("// 8 floats per interval (B0 B1 B2 C0 C1 C2 0 0); fp32 max abs err B %.2e, C %.2e on [0, 64]"
           % (eb, ec))
     print("static constexpr int BESSEL_TAB_N = %d;" % nq)
-    print("__device__ static constexpr float BESSEL_TAB[%d] = {" % tab.size)
+    print("alignas(16) __device__ static constexpr float BESSEL_TAB[%d] = {" % tab.size)
     for j in range(nq):
         print("    " + " ".join("%.9ef," % v for v in tab[8 * j:8 * j + 8]))
     print("};")
@@ -189,7 +189,7 @@ def main():
     ed = check_piecewise32(td, D, h=0.25)
     tabd = np.concatenate([td, np.zeros((nq, 1))], axis=1).ravel()
     print("// D on the same intervals: D0 D1 D2 0 per interval (gradient kernels); fp32 max abs err %.2e" % ed)
-    print("__device__ static constexpr float BESSEL_TABD[%d] = {" % tabd.size)
+    print("alignas(16) __device__ static constexpr float BESSEL_TABD[%d] = {" % tabd.size)
     for j in range(nq):
         print("    " + " ".join("%.9ef," % v for v in tabd[4 * j:4 * j + 4]))
     print("};")

@@ -274,8 +274,8 @@ struct BesselTab {
 // Copies BESSEL_TAB into the work-group's LDS table (all threads take part;
 // call before any thread of the group leaves).
 __device__ inline void load_bessel_tab(float4* tab) {
-  float* t = reinterpret_cast<float*>(tab);
-  for (int i = (int)threadIdx.x; i < 8 * BESSEL_TAB_N; i += (int)blockDim.x) t[i] = BESSEL_TAB[i];
+  const float4* src = reinterpret_cast<const float4*>(BESSEL_TAB);
+  for (int i = (int)threadIdx.x; i < 2 * BESSEL_TAB_N; i += (int)blockDim.x) tab[i] = src[i];
   __syncthreads();
 }
 

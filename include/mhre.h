@@ -194,7 +194,10 @@ int mhre_session_stats(void *session, MhreStats *stats);
  * info[3] = the session's sequence groups, and with ninfo >= 5 info[4] = 1 if
  * its quadratic-system steps update each equation's residual from a row
  * table when a proposal moves one coordinate, instead of evaluating every
- * equation in full.  ninfo >= 4. */
+ * equation in full.  ninfo >= 4.  With
+ * ninfo >= 6 info[5] = how far one chain is split: its waves on the
+ * ring+Gaussian kernels (1, or 4 or 8 in sessions of few chains), its lanes on
+ * the model.cuh path (1 .. 256), else 1. */
 int mhre_session_fit_info(const void *session, int fit, int *info, int ninfo);
 int mhre_session_destroy(void *session);
 /* create + run(nburn + niter) + download + destroy. */
