@@ -142,7 +142,7 @@ hipError_t launch_step_user(const StepLaunch& L, hipStream_t s);
 hipError_t launch_iter_user(bool one, const StepLaunch& L, hipStream_t s);
 // LDS bytes of one chain's state in these kernels, for launches whose fits
 // have at most nprm varied and nptot parameters
-constexpr int user_slot_bytes(int nprm, int nptot) { return (2 * 8 * nprm + 7 * 4 * nprm + 2 * 4 * nptot + 7) / 8 * 8; }
+constexpr int user_slot_bytes(int nprm, int nptot) { return (4 * 8 * nprm + 8 * 4 * nprm + 2 * 4 * nptot + 7) / 8 * 8; }
 const char* user_model_name();
 
 }  // namespace mhre

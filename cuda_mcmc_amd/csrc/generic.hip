@@ -12,7 +12,8 @@
 // stored in datm.
 //
 //   k_iter_user  fits with few data: a sequence's whole ladder in one wave,
-//                many iterations with their replica exchange in one launch
+//                many iterations with their replica exchange in one launch,
+//                the random numbers from a second wave
 //   k_step_user  the others: one iteration a launch, up to 4 waves a chain
 //                (the exchange has a launch of its own, k_exchange)
 #include <hip/hip_runtime.h>
@@ -29,11 +30,11 @@
 namespace mhre {
 
 // Orders the global and LDS accesses of a chain's lanes: what one stored
-// before is read by the others afterwards.  NW = 1: the lanes share a wave
+// before is read by the others afterwards.  Waves = 1: the lanes share a wave
 // (its memory operations keep their order); else they are a work-group.
-template <int NW>
+template <int Waves>
 __device__ inline void chain_fence() {
-  if (NW == 1) {
+  if (Waves == 1) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -43,29 +44,29 @@ __device__ inline void chain_fence() {
 }
 
 // The lanes of one chain.
-template <int NW>
+template <int Waves>
 struct ChainLanes {
-  int n;          // lanes of the chain (a power of two; 64 NW for NW > 1)
+  int n;          // lanes of the chain (a power of two; 64 Waves for Waves > 1)
   int j;          // this lane's place among them
-  double* xs;     // NW > 1: work-group LDS, 2 NW doubles
+  double* xs;     // Waves > 1: work-group LDS, 2 Waves doubles
   int flip;
 
-  // Sum over the chain's lanes, the same on each of them.  NW > 1: the waves'
+  // Sum over the chain's lanes, the same on each of them.  Waves > 1: the waves'
   // sums meet in xs, whose two halves take turns, so that one barrier does.
   __device__ double sum(double v) {
-    if (NW == 1) {
+    if (Waves == 1) {
       if (n == 64) return wave_sum(v);
       for (int m = n >> 1; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
       return v;
     }
     v = wave_sum(v);
-    double* x = xs + flip * NW;
+    double* x = xs + flip * Waves;
     flip ^= 1;
     if (lane_id() == 0) x[threadIdx.x >> 6] = v;
     __syncthreads();
     double s = x[0];
 #pragma unroll
-    for (int w = 1; w < NW; ++w) s += x[w];
+    for (int w = 1; w < Waves; ++w) s += x[w];
     return s;
   }
 };
@@ -93,25 +94,26 @@ __device__ inline bool user_term(const FitDesc& f, CCalcModel* mc, int ch, int i
   const int iret = model(mc, id, ch * f.nptot, imd, ipass);
   if (iret == 0) return false;
   if (iret < 0) { *err = iret; return false; }
-  float dif = gptr(f.dat)[id] - gptr(f.datm)[imd];
+  // through mc's pointers, as model() stored it: no load has to wait for the store
+  float dif = mc->dat[id] - mc->datm[imd];
   if (iret == 2) dif = atan2f(sinf(dif), cosf(dif));
-  *term = (dif * dif) * gptr(f.std2r)[id];
-  gptr(f.chi2m)[imd] = *term;
+  *term = (dif * dif) * mc->std2r[id];
+  mc->chi2m[imd] = *term;
   return true;
 }
 
 // chi^2 of chain ch from the user's model (all passes), its terms in chi2m:
 // the sum over all ndat terms (the reference sums every chi2m entry of the
-// chain, including entries no pass rewrote), in float64.  ONE: the chain has
+// chain, including entries no pass rewrote), in float64.  OneDatum: the chain has
 // at most one datum a lane, whose chi2m entry the lane keeps in term, so that
 // the sum needs no load behind the store.
-template <int NW, bool ONE>
-__device__ inline double user_chi2(const FitDesc& f, CCalcModel* mc, ChainLanes<NW>& cl, int ch, float* term,
+template <int Waves, bool OneDatum>
+__device__ inline double user_chi2(const FitDesc& f, CCalcModel* mc, ChainLanes<Waves>& cl, int ch, float* term,
                                    int* err) {
   const int ndat = f.ndat;
   for (int ipass = 0; ipass < f.npass; ++ipass) {
-    if (ipass) chain_fence<NW>();
-    if (ONE) {
+    if (ipass) chain_fence<Waves>();
+    if (OneDatum) {
       if (cl.j < ndat) user_term(f, mc, ch, cl.j, ipass, term, err);
     } else {
       float t;
@@ -119,7 +121,7 @@ __device__ inline double user_chi2(const FitDesc& f, CCalcModel* mc, ChainLanes<
     }
   }
   double s = 0.0;
-  if (ONE) {
+  if (OneDatum) {
     if (cl.j < ndat) s = (double)*term;
   } else {
     const GLOBAL float* c = gptr(f.chi2m) + (size_t)ch * ndat;
@@ -158,45 +160,51 @@ __global__ void __launch_bounds__(64) k_eval_user(const FitDesc* fits, const Wor
   if (err && f.errflag) atomicExch(f.errflag, err);
 }
 
+// The random numbers of one iteration of a chain, P entries each.
+struct UserDraws {
+  double *z, *lu;        // Gaussian steps, log u
+  int* k;                // coordinate picks
+};
 // A chain's state in LDS for the launch, one copy per wave (the waves of a
 // chain compute the same, so no wave waits for another's bookkeeping): P
-// entries of each array, then two rows of N parameters (k_iter_user's
-// exchange writes the one that the iteration did not use).
+// entries of each array, the draws of two iterations, then two rows of N
+// parameters (k_iter_user's exchange writes the one that the iteration did not
+// use).
 struct UserSlot {
-  double *z, *lu;        // this iteration's Gaussian steps and log u
+  UserDraws d[2];
   float* stp;
   int *cnt, *nac, *sh;
   uint32_t* hw;          // the history word holding entry cnt % nadj ...
   int* hwi;              // ... and its index
-  int* k;                // this iteration's coordinate picks
   float* row;
 };
 __device__ inline UserSlot user_slot(char* lds, int P) {
   UserSlot u;
-  u.z = reinterpret_cast<double*>(lds);
-  u.lu = u.z + P;
-  u.stp = reinterpret_cast<float*>(u.lu + P);
+  double* z = reinterpret_cast<double*>(lds);
+  int* k = reinterpret_cast<int*>(z + 4 * P);
+  u.d[0] = UserDraws{z, z + P, k};
+  u.d[1] = UserDraws{z + 2 * P, z + 3 * P, k + P};
+  u.stp = reinterpret_cast<float*>(k + 2 * P);
   u.cnt = reinterpret_cast<int*>(u.stp + P);
   u.nac = u.cnt + P;
   u.sh = u.nac + P;
   u.hw = reinterpret_cast<uint32_t*>(u.sh + P);
   u.hwi = reinterpret_cast<int*>(u.hw + P);
-  u.k = u.hwi + P;
-  u.row = reinterpret_cast<float*>(u.k + P);
+  u.row = reinterpret_cast<float*>(u.hwi + P);
   return u;
 }
 
 // Place and number of a wave's lanes of a chain, for work that every wave of
 // the chain does by itself.
-template <int NW>
-__device__ inline int own_j(const ChainLanes<NW>& cl) { return NW == 1 ? cl.j : lane_id(); }
-template <int NW>
-__device__ inline int own_n(const ChainLanes<NW>& cl) { return NW == 1 ? cl.n : 64; }
+template <int Waves>
+__device__ inline int own_j(const ChainLanes<Waves>& cl) { return Waves == 1 ? cl.j : lane_id(); }
+template <int Waves>
+__device__ inline int own_n(const ChainLanes<Waves>& cl) { return Waves == 1 ? cl.n : 64; }
 
 // The wave's LDS copy of the chain's state; hist: the launch has burn-in
 // iterations.
-template <int NW>
-__device__ inline void user_load(const FitDesc& f, const ChainLanes<NW>& cl, int ch, const UserSlot& u, bool hist) {
+template <int Waves>
+__device__ inline void user_load(const FitDesc& f, const ChainLanes<Waves>& cl, int ch, const UserSlot& u, bool hist) {
   const int C = f.nchain, P = f.nprm, N = f.nptot;
   for (int k = own_j(cl); k < P; k += own_n(cl)) {
     const size_t pk = (size_t)k * C + ch;
@@ -214,8 +222,8 @@ __device__ inline void user_load(const FitDesc& f, const ChainLanes<NW>& cl, int
   for (int i = own_j(cl); i < N; i += own_n(cl)) u.row[i] = gptr(f.pcur)[(size_t)ch * N + i];
 }
 
-template <int NW>
-__device__ inline void user_store(const FitDesc& f, const ChainLanes<NW>& cl, int ch, const UserSlot& u, bool hist) {
+template <int Waves>
+__device__ inline void user_store(const FitDesc& f, const ChainLanes<Waves>& cl, int ch, const UserSlot& u, bool hist) {
   const int C = f.nchain, P = f.nprm;
   for (int k = cl.j; k < P; k += cl.n) {
     const size_t pk = (size_t)k * C + ch;
@@ -235,14 +243,26 @@ struct LastProposal {
   float told;
 };
 
-// The chain's nprm proposals of iteration it on the state in u and chi2c;
+// The draws of iteration it, substep s on the chain's lane s (modulo its lanes).
+template <int Waves>
+__device__ inline void user_draw(const FitDesc& f, const ChainLanes<Waves>& cl, int ch, int it, const UserDraws& d) {
+  const int P = f.nprm;
+  for (int s = own_j(cl); s < P; s += own_n(cl)) {
+    const U4 r = philox4x32_10((uint32_t)ch, (uint32_t)it, (uint32_t)s, 0u, f.key0, f.key1);
+    d.k[s] = pick_with_retry(r.x, P, (uint32_t)ch, (uint32_t)it, (uint32_t)s, 0u, f.key0, f.key1);
+    d.z[s] = normal64(r.y, r.z);
+    d.lu[s] = log((double)u01(r.w));
+  }
+}
+
+// The chain's nprm proposals of iteration it on the state in u and chi2c, with its draws d;
 // returns the chi^2 evaluations performed.  Every lane of the chain follows
 // the same decisions; the data of a chi^2 are split among them.  row: the
 // current half of u.row.
-template <int NW, bool ONE>
-__device__ unsigned user_substeps(const FitDesc& f, CCalcModel* mc, ChainLanes<NW>& cl, int ch, int it,
-                                  const TraceBuf& tr, const UserSlot& u, float* row, float& chi2c, float* term,
-                                  LastProposal& last, int* err) {
+template <int Waves, bool OneDatum>
+__device__ unsigned user_substeps(const FitDesc& f, CCalcModel* mc, ChainLanes<Waves>& cl, int ch, int it,
+                                  const TraceBuf& tr, const UserSlot& u, const UserDraws& d, float* row, float& chi2c,
+                                  float* term, LastProposal& last, int* err) {
   const int C = f.nchain, P = f.nprm, N = f.nptot;
   const bool burn = it < f.nburn;
   const double beta = (double)gptr(f.beta)[ch / f.nseq];
@@ -250,19 +270,11 @@ __device__ unsigned user_substeps(const FitDesc& f, CCalcModel* mc, ChainLanes<N
   const float rnadj = 1.0f / (float)nadj;
   GLOBAL float* prow = gptr(f.pcur) + (size_t)ch * N;
   unsigned nev = 0;
-  // the draws of substep s on the chain's lane s (modulo its lanes)
-  for (int s = own_j(cl); s < P; s += own_n(cl)) {
-    const U4 r = philox4x32_10((uint32_t)ch, (uint32_t)it, (uint32_t)s, 0u, f.key0, f.key1);
-    u.k[s] = pick_with_retry(r.x, P, (uint32_t)ch, (uint32_t)it, (uint32_t)s, 0u, f.key0, f.key1);
-    u.z[s] = normal64(r.y, r.z);
-    u.lu[s] = log((double)u01(r.w));
-  }
-  wave_sync_lds();
   for (int s = 0; s < P; ++s) {
-    const int k = u.k[s];
+    const int k = d.k[s];
     const int t = gptr(f.ivar)[k];
     const float old = row[t], sd = u.stp[k];
-    double pd = (double)old + (double)sd * u.z[s];
+    double pd = (double)old + (double)sd * d.z[s];
     if (gptr(f.pdescr)[t] == 2) pd = pd - 6.283185307179586 * rint(pd / 6.283185307179586);
     const float pn = (float)pd;
     const bool inprior = !(pn < gptr(f.pmint)[t] || pn > gptr(f.pmaxt)[t]);
@@ -271,11 +283,11 @@ __device__ unsigned user_substeps(const FitDesc& f, CCalcModel* mc, ChainLanes<N
     double c2 = 0.0;
     if (inprior) {
       if (cl.j == 0) prow[t] = pn;
-      chain_fence<NW>();   // the chain's lanes read the proposal through mc->pcur
-      c2 = user_chi2<NW, ONE>(f, mc, cl, ch, term, err);
+      chain_fence<Waves>();   // the chain's lanes read the proposal through mc->pcur
+      c2 = user_chi2<Waves, OneDatum>(f, mc, cl, ch, term, err);
       ++nev;
       const double x = -0.5 * beta * (c2 - (double)chi2c);
-      if (u.lu[s] <= x) {
+      if (d.lu[s] <= x) {
         acc = 1;
         chi2c = (float)c2;
         if (own_j(cl) == 0) {
@@ -311,9 +323,9 @@ __device__ unsigned user_substeps(const FitDesc& f, CCalcModel* mc, ChainLanes<N
         // the word is full: on to the next one, which an earlier proposal of
         // this launch may have written (short rings), hence the fences
         GLOBAL uint32_t* h = gptr(f.hbits) + (size_t)ch * f.hwords * P + k;
-        chain_fence<NW>();
+        chain_fence<Waves>();
         if (cl.j == 0) h[(size_t)wi * P] = u.hw[k];
-        chain_fence<NW>();
+        chain_fence<Waves>();
         if (own_j(cl) == 0) {
           u.hw[k] = h[(size_t)w2 * P];
           u.hwi[k] = w2;
@@ -325,19 +337,19 @@ __device__ unsigned user_substeps(const FitDesc& f, CCalcModel* mc, ChainLanes<N
   return nev;
 }
 
-// One iteration of every chain of the list.  NW = 1: lanes lanes a chain, so
-// 64 / lanes chains a wave (the list is padded to whole waves); NW > 1: one
-// chain a work-group of NW waves.  slot_bytes: LDS of one chain's state
+// One iteration of every chain of the list.  Waves = 1: lanes lanes a chain, so
+// 64 / lanes chains a wave (the list is padded to whole waves); Waves > 1: one
+// chain a work-group of Waves waves.  slot_bytes: LDS of one chain's state
 // (user_slot at maxp parameters).
-template <int NW>
-__global__ void __launch_bounds__(64 * NW) k_step_user(const FitDesc* fits, const WorkItem* work, int nwork,
+template <int Waves>
+__global__ void __launch_bounds__(64 * Waves) k_step_user(const FitDesc* fits, const WorkItem* work, int nwork,
                                                        RunClock* clk, TraceBuf tr, int it_off, int lanes,
                                                        int slot_bytes) {
   extern __shared__ __align__(16) char lds[];
-  __shared__ double xs[2 * NW];
+  __shared__ double xs[2 * Waves];
   const int lane = lane_id();
-  const int per = NW == 1 ? 64 / lanes : 1;
-  const int c = NW == 1 ? lane / lanes : 0;
+  const int per = Waves == 1 ? 64 / lanes : 1;
+  const int c = Waves == 1 ? lane / lanes : 0;
   const WorkItem w = work[blockIdx.x * per + c];
   const FitDesc& f = wave_fit(fits, w.fit);
   pass_clock(clk);
@@ -345,10 +357,10 @@ __global__ void __launch_bounds__(64 * NW) k_step_user(const FitDesc* fits, cons
   if (it >= f.nburn + f.niter) return;
   const int ch = w.idx;
   const bool live = ch >= 0;   // padding lanes only take part in the counting
-  ChainLanes<NW> cl{NW == 1 ? lanes : 64 * NW, NW == 1 ? lane & (lanes - 1) : (int)threadIdx.x, xs, 0};
+  ChainLanes<Waves> cl{Waves == 1 ? lanes : 64 * Waves, Waves == 1 ? lane & (lanes - 1) : (int)threadIdx.x, xs, 0};
   unsigned nev = 0;
   if (live) {
-    const int wid = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int wid = Waves == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const UserSlot u = user_slot(lds + (size_t)(wid * per + c) * slot_bytes, f.nprm);
     const bool hist = it < f.nburn;
     CCalcModel mc = user_model_args(f);
@@ -356,9 +368,10 @@ __global__ void __launch_bounds__(64 * NW) k_step_user(const FitDesc* fits, cons
     LastProposal last{0, 0, 0.0f};
     int err = 0;
     user_load(f, cl, ch, u, hist);
+    user_draw(f, cl, ch, it, u.d[0]);
     wave_sync_lds();
-    nev = user_substeps<NW, false>(f, &mc, cl, ch, it, tr, u, u.row, chi2c, &term, last, &err);
-    chain_fence<NW>();   // every wave's state is final and no wave reads the arrays any more
+    nev = user_substeps<Waves, false>(f, &mc, cl, ch, it, tr, u, u.d[0], u.row, chi2c, &term, last, &err);
+    chain_fence<Waves>();   // every wave's state is final and no wave reads the arrays any more
     user_store(f, cl, ch, u, hist);
     if (cl.j == 0) {
       gptr(f.chi2c)[ch] = chi2c;
@@ -369,7 +382,7 @@ __global__ void __launch_bounds__(64 * NW) k_step_user(const FitDesc* fits, cons
     if (err && f.errflag) atomicExch(f.errflag, err);
   }
   const bool count = live && cl.j == 0;
-  if (NW == 1 || threadIdx.x < 64) wave_count(f, count ? nev : 0u, count ? (unsigned)f.nprm : 0u);
+  if (Waves == 1 || threadIdx.x < 64) wave_count(f, count ? nev : 0u, count ? (unsigned)f.nprm : 0u);
 }
 
 // Iterations it_off .. it_off + iters - 1 of the segment for whole sequences,
@@ -377,12 +390,16 @@ __global__ void __launch_bounds__(64 * NW) k_step_user(const FitDesc* fits, cons
 // rungs) of its sequences, f.ulanes lanes a chain, and nothing couples one
 // sequence to another, so no launch has to end between two iterations.  For
 // problems of few data such a launch is all latency, and so was the exchange
-// launch between two of them.  Items are (fit, first sequence of the wave).
-template <bool ONE>
-__global__ void __launch_bounds__(64) k_iter_user(const FitDesc* fits, const WorkItem* work, int nwork, RunClock* clk,
+// launch between two of them.  What is left is the latency of one iteration's
+// chain of steps, so a second wave, with the same lanes, draws the random
+// numbers of the next iteration meanwhile: none of them depends on the chains.
+// Items are (fit, first sequence of the work-group).
+template <bool OneDatum>
+__global__ void __launch_bounds__(128) k_iter_user(const FitDesc* fits, const WorkItem* work, int nwork, RunClock* clk,
                                                   TraceBuf tr, int it_off, int iters, int slot_bytes) {
   extern __shared__ __align__(16) char lds[];
   __shared__ LadderLds ladder;
+  __shared__ SwapDraw swap[2][64];
   const WorkItem w = work[blockIdx.x];
   const FitDesc& f = wave_fit(fits, w.fit);
   pass_clock(clk);
@@ -390,15 +407,27 @@ __global__ void __launch_bounds__(64) k_iter_user(const FitDesc* fits, const Wor
   const int nit = f.nburn + f.niter;
   if (it0 >= nit) return;
   const int lane = lane_id();
-  const int B = f.nbeta, S = f.nseq, P = f.nprm, N = f.nptot, n = f.ulanes;
-  const int G = 64 / (f.xlanes * n);
-  const int c = lane / n, sl = c / G, g = c % G;
+  const int nb = f.nbeta, ns = f.nseq, P = f.nprm, N = f.nptot, n = f.ulanes;
+  const int nwseq = 64 / (f.xlanes * n);
+  const int c = lane / n, sl = c / nwseq, g = c % nwseq;
   const int iseq = __builtin_amdgcn_readfirstlane(w.idx) + g;
-  const bool live = iseq < S && sl < B;
-  const int ch = live ? sl * S + iseq : 0;
+  const bool live = iseq < ns && sl < nb;
+  const int ch = live ? sl * ns + iseq : 0;
   ChainLanes<1> cl{n, lane & (n - 1), nullptr, 0};
   const UserSlot u = user_slot(lds + (size_t)c * slot_bytes, P);
   const bool hist = it0 < f.nburn;
+  const int end = nit - it0 < iters ? nit - it0 : iters;
+  if (__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) != 0) {
+    // the second wave: the draws of iteration i, one iteration ahead
+    for (int i = 0; i < end; ++i) {
+      if (live) {
+        user_draw(f, cl, ch, it0 + i, u.d[i & 1]);
+        if (cl.j == 0 && nb > 1) swap[i & 1][c] = swap_draw(f, iseq, it0 + i, sl);
+      }
+      __syncthreads();
+    }
+    return;
+  }
   CCalcModel mc = user_model_args(f);
   float chi2c = 0.0f, term = 0.0f;
   int tc = 0, err = 0, nex = 0;
@@ -407,43 +436,43 @@ __global__ void __launch_bounds__(64) k_iter_user(const FitDesc* fits, const Wor
   if (live) {
     chi2c = gptr(f.chi2c)[ch];
     tc = gptr(f.tcur)[ch];
-    if (ONE && cl.j < f.ndat) term = gptr(f.chi2m)[(size_t)ch * f.ndat + cl.j];
+    if (OneDatum && cl.j < f.ndat) term = gptr(f.chi2m)[(size_t)ch * f.ndat + cl.j];
     user_load(f, cl, ch, u, hist);
   }
   const double hb = swap_factor(f, sl);
   wave_sync_lds();
   float* row = u.row;
   float* other = u.row + N;
-  for (int i = 0; i < iters && it0 + i < nit; ++i) {
+  for (int i = 0; i < end; ++i) {
     const int it = it0 + i;
+    __syncthreads();   // this iteration's draws are there, the one before's are free
     const bool burn = it < f.nburn;
-    if (live) nev += user_substeps<1, ONE>(f, &mc, cl, ch, it, tr, u, row, chi2c, &term, last, &err);
+    if (live) nev += user_substeps<1, OneDatum>(f, &mc, cl, ch, it, tr, u, u.d[i & 1], row, chi2c, &term, last, &err);
     nprop += P;
     int perm = sl;
-    if (B > 1) {
+    if (nb > 1) {
       // the exchange (reference: gpu_mcmc.cu:548-591): slot sl of sequence g is
       // entry c of the ladder LDS, and its first lane has attempt sl
-      SwapDraw d{0, 0.0};
-      if (live) d = swap_draw(f, iseq, it, sl);
-      const double hk = __shfl(hb, (d.k * G + g) * n);
+      const SwapDraw d = live ? swap[i & 1][c] : SwapDraw{0, 0.0};
+      const double hk = __shfl(hb, (d.k * nwseq + g) * n);
       if (cl.j == 0) {
         ladder.slot[c] = LadderSlot{chi2c, sl};
         ladder.pair[c] = 0;
       }
       const bool attempt = live && cl.j == 0;
-      const unsigned long long swapped = ladder_swaps(ladder, attempt, d.k * G + g, G, d.k == 0, d.lu, hk);
+      const unsigned long long swapped = ladder_swaps(ladder, attempt, d.k * nwseq + g, nwseq, d.k == 0, d.lu, hk);
       chi2c = ladder.slot[c].c2;
       perm = ladder.slot[c].src;
-      tc = __shfl(tc, (perm * G + g) * n);
+      tc = __shfl(tc, (perm * nwseq + g) * n);
       if (!burn) nex += __popcll(ladder.pair[c] & swapped);
       if (tr.ex && attempt && it >= tr.it0 && it < tr.it0 + tr.nit)
-        tr.ex[(size_t)f.tr_ex + ((size_t)(it - tr.it0) * B + sl) * S + iseq] =
+        tr.ex[(size_t)f.tr_ex + ((size_t)(it - tr.it0) * nb + sl) * ns + iseq] =
             d.k | ((int)((swapped >> lane) & 1ull) << 16);
     }
     if (live) {
       // the row that ends up in this slot, from the LDS of the slot it started in
       const float* src = reinterpret_cast<const float*>(
-          reinterpret_cast<const char*>(row) + (ptrdiff_t)((perm * G + g) - c) * slot_bytes);
+          reinterpret_cast<const char*>(row) + (ptrdiff_t)((perm * nwseq + g) - c) * slot_bytes);
       const bool moved = perm != sl;
       const bool rec = !burn && f.record;
       const int itr = it - f.nburn;
@@ -453,8 +482,12 @@ __global__ void __launch_bounds__(64) k_iter_user(const FitDesc* fits, const Wor
         if (moved) gptr(f.pcur)[(size_t)ch * N + q] = v;
         if (rec) {
           const int ip = gptr(f.invar)[q];
-          if (ip >= 0) gptr(f.pout)[(((size_t)B * ip + sl) * S + iseq) * f.niter + itr] = v;
+          if (ip >= 0) gptr(f.pout)[(((size_t)nb * ip + sl) * ns + iseq) * f.niter + itr] = v;
         }
+      }
+      if (cl.j == 0) {   // model() may read these
+        gptr(f.chi2c)[ch] = chi2c;
+        gptr(f.flag)[ch] = last.flag;
       }
       if (rec && cl.j == 0) {
         gptr(f.tout)[(size_t)ch * f.niter + itr] = tc;
@@ -469,10 +502,8 @@ __global__ void __launch_bounds__(64) k_iter_user(const FitDesc* fits, const Wor
   if (live) {
     user_store(f, cl, ch, u, hist);
     if (cl.j == 0) {
-      gptr(f.chi2c)[ch] = chi2c;
       gptr(f.tcur)[ch] = tc;
       if (nex) gptr(f.n_exch)[ch] += nex;
-      gptr(f.flag)[ch] = last.flag;
       gptr(f.ptent)[ch] = last.told;
       gptr(f.ptentn)[ch] = last.t;
     }
@@ -512,8 +543,8 @@ hipError_t launch_iter_user(bool one, const StepLaunch& L, hipStream_t s) {
   const TraceBuf tr{L.tr_dec, L.tr_chi2, L.tr_ex, L.tr_it0, L.tr_nit};
   const int sb = user_slot_bytes(L.max_prm, L.max_tot);
   const int dyn = 64 / L.ulanes * sb;
-  if (one) k_iter_user<true><<<L.nwork, 64, dyn, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, L.iters, sb);
-  else k_iter_user<false><<<L.nwork, 64, dyn, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, L.iters, sb);
+  if (one) k_iter_user<true><<<L.nwork, 128, dyn, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, L.iters, sb);
+  else k_iter_user<false><<<L.nwork, 128, dyn, s>>>(L.fits, L.work, L.nwork, L.clk, tr, L.it_off, L.iters, sb);
   return hipGetLastError();
 }
 
