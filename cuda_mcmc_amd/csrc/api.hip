@@ -12,14 +12,19 @@
 //     hipGraph and replayed;
 //   * errors are returned as codes with a message (mhre_last_error).
 #include <hip/hip_runtime.h>
+#include <sched.h>
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #define MHRE_NO_MODEL_MACROS 1
@@ -70,6 +75,41 @@ constexpr int kNativeEht = 0;
 bool env_flag(const char* name) {
   const char* v = getenv(name);
   return v && *v && strcmp(v, "0") != 0;
+}
+
+// ---------------------------------------------------------- host threads
+
+// fn(0) .. fn(n - 1), on several host threads if the work (bytes of host memory
+// it goes through) is worth starting them.  fn must not throw.
+constexpr size_t THREAD_BYTES = 4 << 20;   // per thread: starting one costs about as much as 0.3 MB
+constexpr int MAX_THREADS = 8;
+
+int host_threads() {
+  int n = 1;
+  cpu_set_t set;
+  if (sched_getaffinity(0, sizeof set, &set) == 0) n = CPU_COUNT(&set);
+  const char* e = getenv("OMP_NUM_THREADS");
+  const int omp = e ? atoi(e) : 0;
+  if (omp > 0) n = std::min(n, omp);
+  return std::max(1, std::min(n, MAX_THREADS));
+}
+
+template <class Fn>
+void parallel_for(size_t n, size_t bytes, const Fn& fn) {
+  std::atomic<size_t> next{0};
+  auto work = [&]() {
+    for (size_t i = next.fetch_add(1, std::memory_order_relaxed); i < n; i = next.fetch_add(1, std::memory_order_relaxed))
+      fn(i);
+  };
+  const size_t want = std::min({(size_t)host_threads(), n, bytes / THREAD_BYTES + 1});
+  std::vector<std::thread> t;
+  try {
+    t.reserve(want);
+    while (t.size() + 1 < want) t.emplace_back(work);
+  } catch (const std::exception&) {   // no more threads or memory: those that run do all of it
+  }
+  work();
+  for (std::thread& x : t) x.join();
 }
 
 // ----------------------------------------------------------------- arena
@@ -157,8 +197,9 @@ int validate(const MhreFitSpec& s, int idx) {
   const size_t pc = (size_t)s.nprm * s.nbeta * s.nseq;
   for (size_t q = 0; q < pc; ++q)
     if (s.n_cnt[q] < 0) FAIL(MHRE_EINVAL, "fit %d: n_cnt must be non-negative (reference: ones)", idx);
-  for (size_t q = 0; q < (size_t)s.nadj * pc; ++q)
-    if (s.n_hist[q] != 0 && s.n_hist[q] != 1) FAIL(MHRE_EINVAL, "fit %d: n_hist entries must be 0 or 1", idx);
+  int other = 0;   // any bit but the lowest (no early way out, so that it vectorises)
+  for (size_t q = 0; q < (size_t)s.nadj * pc; ++q) other |= s.n_hist[q] & ~1;
+  if (other) FAIL(MHRE_EINVAL, "fit %d: n_hist entries must be 0 or 1", idx);
   for (int b = 0; b < s.nbeta; ++b)
     if (!(s.beta[b] >= 0.0f)) FAIL(MHRE_EINVAL, "fit %d: beta[%d] must be >= 0", idx, b);
   for (int i = 0; i < s.nptot; ++i)
@@ -535,37 +576,81 @@ int eht_split_waves(const std::vector<FitHost>& fits, const std::vector<int>& id
 // Most concurrent sequence groups (streams) of a session.
 constexpr int MAX_GROUPS = 8;
 
-// n_hist[a][q] (0/1, q = k * nchain + chain) -> bit a % 32 of word [a / 32][q]
-// Packs the 0/1 history n_hist[nadj][npc] into bits and, in the same pass,
-// the running accept sums sum[q] = number of set entries of q.
-// n_hist[a][k][chain] (0/1) <-> bit a % 32 of hbits[chain][a / 32][k]
-// (fitdesc.h), with sum[k][chain] = the set entries of (k, chain).
-void pack_hist(const int* n_hist, int nadj, int P, int C, std::vector<uint32_t>& bits, std::vector<int>& sum) {
-  const int W = hist_words(nadj);
-  const size_t npc = (size_t)P * C;
-  bits.assign((size_t)W * npc, 0u);
-  sum.assign(npc, 0);
-  for (int a = 0; a < nadj; ++a) {
-    const int* h = n_hist + (size_t)a * npc;
-    const uint32_t bit = 1u << (a & 31);
-    for (int k = 0; k < P; ++k)
-      for (int c = 0; c < C; ++c) {
-        const size_t q = (size_t)k * C + c;
-        const int on = h[q] != 0;
-        bits[((size_t)c * W + (a >> 5)) * P + k] |= on ? bit : 0u;
-        sum[q] += on;
-      }
+// Between the caller's 0/1 history n_hist[nadj][nprm][chain] and its bits
+// (fitdesc.h: entry a of (k, chain) is bit a % 32 of hbits[chain][a / 32][k]),
+// with sum[k][chain] = the set entries of (k, chain).  A parameter's words of
+// one index are gathered from (scattered to) the chain-major bits once, and
+// their 32 rows of the history go through memory in order.  The rows of a
+// session of 512 small fits are 840 MB: one entry at a time on one thread took
+// 110 ms to unpack them, this form on 8 threads 15.
+struct HistFit {
+  const int* n_hist;
+  int* n_hist_out;
+  int nadj, P, C;
+  std::vector<uint32_t>* bits;
+  std::vector<int>* sum;
+};
+
+void pack_hists(const std::vector<HistFit>& fits) {
+  std::vector<std::pair<int, int>> jobs;   // fit, parameter
+  size_t bytes = 0;
+  for (size_t i = 0; i < fits.size(); ++i) {
+    const HistFit& h = fits[i];
+    const size_t npc = (size_t)h.P * h.C;
+    h.bits->assign((size_t)hist_words(h.nadj) * npc, 0u);
+    h.sum->assign(npc, 0);
+    bytes += (size_t)h.nadj * npc * sizeof(int);
+    for (int k = 0; k < h.P; ++k) jobs.push_back({(int)i, k});
   }
+  parallel_for(jobs.size(), bytes, [&](size_t j) {
+    constexpr int BLOCK = 512;   // chains at a time
+    const HistFit& h = fits[jobs[j].first];
+    const int k = jobs[j].second, W = hist_words(h.nadj);
+    uint32_t word[BLOCK];
+    for (int c0 = 0; c0 < h.C; c0 += BLOCK) {
+      const int nc = std::min(BLOCK, h.C - c0);
+      int* sum = h.sum->data() + (size_t)k * h.C + c0;
+      for (int w = 0; w < W; ++w) {
+        std::fill(word, word + nc, 0u);
+        for (int a = 32 * w; a < std::min(32 * w + 32, h.nadj); ++a) {
+          const int* row = h.n_hist + ((size_t)a * h.P + k) * h.C + c0;
+          for (int c = 0; c < nc; ++c) {
+            const uint32_t on = row[c] != 0;
+            word[c] |= on << (a & 31);
+            sum[c] += (int)on;
+          }
+        }
+        uint32_t* bits = h.bits->data() + ((size_t)c0 * W + w) * h.P + k;
+        for (int c = 0; c < nc; ++c) bits[(size_t)c * W * h.P] = word[c];
+      }
+    }
+  });
 }
 
-void unpack_hist(const std::vector<uint32_t>& bits, int nadj, int P, int C, int* n_hist) {
-  const int W = hist_words(nadj);
-  const size_t npc = (size_t)P * C;
-  for (int a = 0; a < nadj; ++a)
-    for (int k = 0; k < P; ++k)
-      for (int c = 0; c < C; ++c)
-        n_hist[(size_t)a * npc + (size_t)k * C + c] =
-            (int)((bits[((size_t)c * W + (a >> 5)) * P + k] >> (a & 31)) & 1u);
+void unpack_hists(const std::vector<HistFit>& fits) {
+  std::vector<std::pair<int, int>> jobs;   // fit, parameter
+  size_t bytes = 0;
+  for (size_t i = 0; i < fits.size(); ++i) {
+    bytes += (size_t)fits[i].nadj * fits[i].P * fits[i].C * sizeof(int);
+    for (int k = 0; k < fits[i].P; ++k) jobs.push_back({(int)i, k});
+  }
+  parallel_for(jobs.size(), bytes, [&](size_t j) {
+    constexpr int BLOCK = 512;
+    const HistFit& h = fits[jobs[j].first];
+    const int k = jobs[j].second, W = hist_words(h.nadj);
+    uint32_t word[BLOCK];
+    for (int c0 = 0; c0 < h.C; c0 += BLOCK) {
+      const int nc = std::min(BLOCK, h.C - c0);
+      for (int w = 0; w < W; ++w) {
+        const uint32_t* bits = h.bits->data() + ((size_t)c0 * W + w) * h.P + k;
+        for (int c = 0; c < nc; ++c) word[c] = bits[(size_t)c * W * h.P];
+        for (int a = 32 * w; a < std::min(32 * w + 32, h.nadj); ++a) {
+          int* row = h.n_hist_out + ((size_t)a * h.P + k) * h.C + c0;
+          for (int c = 0; c < nc; ++c) row[c] = (int)((word[c] >> (a & 31)) & 1u);
+        }
+      }
+    }
+  });
 }
 
 // ------------------------------------------------------------- session
@@ -633,6 +718,8 @@ struct Session {
   int tr_nit = 0, tr_it0 = 0;
   size_t tr_dec_total = 0, tr_ex_total = 0;
   std::vector<void*> extra;   // other device allocations
+  std::unique_ptr<unsigned char[]> stage;   // host side of the gathered downloads
+  size_t stage_bytes = 0;
 };
 
 template <class T>
@@ -784,20 +871,29 @@ struct Downloads {
     const auto runs = merge_runs(small);
     size_t total = 0;
     for (auto [a, b] : runs) total += small[b - 1].off + small[b - 1].bytes - small[a].off;
-    std::vector<unsigned char> stage(total);
-    size_t at = 0;
+    // kept by the session: fresh pages would be faulted in and pinned by every
+    // download (24 against 5 ms for 52 MB)
+    if (S->stage_bytes < total) {
+      S->stage.reset();
+      S->stage_bytes = 0;
+      S->stage.reset(new unsigned char[total]);
+      S->stage_bytes = total;
+    }
+    unsigned char* const stage = S->stage.get();
+    size_t at = 0, moved = 0;
+    std::vector<size_t> from(small.size());   // place of each range in the stage
     for (auto [a, b] : runs) {
       const size_t lo = small[a].off, hi = small[b - 1].off + small[b - 1].bytes;
-      HIPCHK(hipMemcpyAsync(stage.data() + at, S->arena + lo, hi - lo, hipMemcpyDeviceToHost, S->stream));
+      HIPCHK(hipMemcpyAsync(stage + at, S->arena + lo, hi - lo, hipMemcpyDeviceToHost, S->stream));
+      for (size_t i = a; i < b; ++i) {
+        from[i] = at + (small[i].off - lo);
+        moved += small[i].bytes;
+      }
       at += hi - lo;
     }
     HIPCHK(hipStreamSynchronize(S->stream));
-    at = 0;
-    for (auto [a, b] : runs) {
-      const size_t lo = small[a].off;
-      for (size_t i = a; i < b; ++i) std::memcpy(small[i].host, stage.data() + at + (small[i].off - lo), small[i].bytes);
-      at += small[b - 1].off + small[b - 1].bytes - lo;
-    }
+    parallel_for(small.size(), moved,
+                 [&](size_t i) { std::memcpy(small[i].host, stage + from[i], small[i].bytes); });
     r.clear();
     return MHRE_OK;
   }
@@ -1187,6 +1283,10 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
   }
 
   std::vector<FitDesc> descs(nfits);
+  std::vector<HistFit> hists;
+  for (FitHost& h : S->fits)
+    hists.push_back({h.s.n_hist, nullptr, h.s.nadj, h.s.nprm, h.nchain, &h.hbits, &h.sumh});
+  pack_hists(hists);
   Uploads U;
   for (int i = 0; i < nfits; ++i) {
     FitHost& h = S->fits[i];
@@ -1267,7 +1367,6 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
     U.add(h.o_nacpt, s.n_acpt, P * C);
     // the history as bits and the running accept sums over its nadj entries
     // (the device keeps sumh[k][chain] equal to the set bits of the chain's ring)
-    pack_hist(s.n_hist, s.nadj, P, C, h.hbits, h.sumh);
     U.add(h.o_nhist, h.hbits.data(), h.hbits.size());
     U.add(h.o_nexch, s.n_exch, C);
     U.add(h.o_tcur, s.tcur, C);
@@ -1612,8 +1711,10 @@ int download(Session* S, int model_data) {
     }
   }
   CHK(D.flush(S));
+  std::vector<HistFit> hists;
   for (FitHost& h : S->fits)
-    unpack_hist(h.hbits, h.s.nadj, h.s.nprm, h.nchain, h.s.n_hist);
+    hists.push_back({nullptr, h.s.n_hist, h.s.nadj, h.s.nprm, h.nchain, &h.hbits, nullptr});
+  unpack_hists(hists);
   if (model_data) {
     // model data and chi^2 terms of each chain's final state; chi2c is
     // recomputed identically and already copied out above
