@@ -159,6 +159,8 @@ def _declare(L):
     L.mhre_eht_chi2_grad.argtypes = [vp, vp, C.c_int, C.c_int, vp, vp, vp]
     L.mhre_eht_gn_system.restype = C.c_int
     L.mhre_eht_gn_system.argtypes = [vp, vp, C.c_int, C.c_int, vp, vp, vp, vp]
+    L.mhre_eht_gn_matrices.restype = C.c_int
+    L.mhre_eht_gn_matrices.argtypes = [vp, vp, C.c_int, C.c_int, vp, vp, vp, vp]
     L.mhre_eht_data_destroy.restype = C.c_int
     L.mhre_eht_data_destroy.argtypes = [vp]
     L.mhre_eht_data_info.restype = C.c_int

@@ -5,7 +5,7 @@ The reference samples without derivatives; this module adds them on the same
 data arrays that ``calc_modchi2`` takes (``src/mcmc.h:23-27``), so that
 ``chi2(P)`` here equals the ``chi2c`` of ``calc_modchi2`` for the same
 parameter rows.  The work runs in the HIP kernels behind the C ABI
-(``mhre_eht_chi2_grad``, ``mhre_eht_gn_system``); torch supplies device
+(``mhre_eht_chi2_grad``, ``mhre_eht_gn_matrices``); torch supplies device
 memory and the stream only.
 
 EhtData            one data set packed on the current GPU.
@@ -26,7 +26,6 @@ from . import _lib
 from ._lib import EngineError
 
 NP9 = 9
-_IU = np.triu_indices(NP9)
 
 
 def _stream(t):
@@ -113,14 +112,10 @@ class EhtData:
         n, ldp = self._rows(P)
         chi = torch.empty(n, dtype=torch.float64, device=P.device)
         jtr = torch.empty((n, NP9), dtype=torch.float64, device=P.device)
-        tri = torch.empty((n, NP9 * (NP9 + 1) // 2), dtype=torch.float64, device=P.device)
-        rc = self.lib.mhre_eht_gn_system(self.handle, _dptr(P), n, ldp, _dptr(chi), _dptr(jtr), _dptr(tri),
-                                         _stream(P))
-        _lib.check(self.lib, rc, "mhre_eht_gn_system")
-        jtj = torch.zeros((n, NP9, NP9), dtype=torch.float64, device=P.device)
-        iu = torch.as_tensor(np.stack(_IU), device=P.device)
-        jtj[:, iu[0], iu[1]] = tri
-        jtj = jtj + jtj.transpose(1, 2) - torch.diag_embed(torch.diagonal(jtj, dim1=1, dim2=2))
+        jtj = torch.empty((n, NP9, NP9), dtype=torch.float64, device=P.device)
+        rc = self.lib.mhre_eht_gn_matrices(self.handle, _dptr(P), n, ldp, _dptr(chi), _dptr(jtr), _dptr(jtj),
+                                           _stream(P))
+        _lib.check(self.lib, rc, "mhre_eht_gn_matrices")
         return chi, jtr, jtj
 
 

@@ -1818,9 +1818,30 @@ static bool ring_grad_disabled() {
 
 struct EhtData {
   FitHost h;
+  size_t split_lds = 0;          // launch_eht_grad9
+  int ncu = 0, lds_per_cu = 0, lds_per_block = 0;
   char* dev = nullptr;
   FitDesc* d_fd = nullptr;
 };
+
+// Waves per point of a gradient call of n points: 1 (a wave per point), or a
+// work-group of 4, 8 or 16 while all points' work-groups are on the chip at
+// once, or of at least 8 in two rounds; 16 only where each wave still has two
+// tiles.  Measured, one wave per point -> split, us a call, 2000 visibilities +
+// 600 closures: 1 to 128 points 47 -> 15, 512: 48 -> 19, 1024: 50 -> 30, but
+// 2048 (two rounds of 4 waves) 56 -> 80; 10000 + 3000: 1 point 198 -> 28, 256:
+// 206 -> 33, 257 (two rounds): 206 -> 63.
+int grad_split_waves(const EhtData* E, int n) {
+  const size_t lds = E->split_lds + GRAD_SPLIT_STATIC_LDS;
+  if (lds > (size_t)E->lds_per_block) return 1;
+  const long long fit = (long long)((size_t)E->lds_per_cu / lds);
+  const int most = E->h.ntile >= 2 * GRAD_SPLIT_MAXW ? GRAD_SPLIT_MAXW : 8;
+  auto at_once = [&](int w) { return E->ncu * std::min<long long>(fit, GRAD_SPLIT_WAVES_PER_CU / w); };
+  for (int rounds = 1; rounds <= 2; ++rounds)
+    for (int w = most; w >= (rounds == 1 ? 4 : 8); w >>= 1)
+      if (n <= rounds * at_once(w)) return w;
+  return 1;
+}
 
 void destroy_eht_data(EhtData* E) {
   if (!E) return;
@@ -1937,6 +1958,24 @@ int eht_data_create(const float* coor, const float* dat, const float* std2r, con
   const size_t o_clow = A.reserve<float>(h.clow.size());
   const size_t o_tinfo = A.reserve<int>(h.tinfo.size());
   const size_t o_clr = A.reserve<int>(h.clr.size());
+  // the closures of each visibility (FitDesc::vcl)
+  std::vector<int> off((size_t)h.ntile * TILE + 1, 0), vcl((size_t)3 * h.ncph);
+  for (int c = 0; c < h.ncph; ++c)
+    for (int m = 0; m < 3; ++m) ++off[h.clo[4 * c + m] + 1];
+  for (size_t j = 1; j < off.size(); ++j) off[j] += off[j - 1];
+  std::vector<int> at(off.begin(), off.end() - 1);
+  for (int c = 0; c < h.ncph; ++c)
+    for (int m = 0; m < 3; ++m) vcl[at[h.clo[4 * c + m]]++] = 2 * c + (m == 2 ? 1 : 0);
+  E->split_lds = eht_grad_split_lds(h.ntile, h.ncph);
+  int dev = 0;
+  HIPCHK(hipGetDevice(&dev));
+  HIPCHK(hipDeviceGetAttribute(&E->ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  HIPCHK(hipDeviceGetAttribute(&E->lds_per_block, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+  if (hipDeviceGetAttribute(&E->lds_per_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) != hipSuccess ||
+      E->lds_per_cu < E->lds_per_block)
+    E->lds_per_cu = E->lds_per_block;
+  const size_t o_off = A.reserve<int>(off.size());
+  const size_t o_vcl = A.reserve<int>(vcl.size());
   const size_t o_fd = A.reserve<FitDesc>(1);
   HIPCHK(hipMalloc((void**)&E->dev, A.bytes));
   FitDesc d{};
@@ -1951,12 +1990,16 @@ int eht_data_create(const float* coor, const float* dat, const float* std2r, con
   d.tinfo = reinterpret_cast<const int2*>(E->dev + o_tinfo);
   d.clr = reinterpret_cast<const int*>(E->dev + o_clr);
   d.nround = h.nround;
+  d.vcl_off = reinterpret_cast<const int*>(E->dev + o_off);
+  d.vcl = reinterpret_cast<const int*>(E->dev + o_vcl);
   E->d_fd = reinterpret_cast<FitDesc*>(E->dev + o_fd);
   HIPCHK(hipMemcpy(E->dev + o_vis, h.vis.data(), h.vis.size() * sizeof(float), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(E->dev + o_clo, h.clo.data(), h.clo.size() * sizeof(int), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(E->dev + o_clow, h.clow.data(), h.clow.size() * sizeof(float), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(E->dev + o_tinfo, h.tinfo.data(), h.tinfo.size() * sizeof(int), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(E->dev + o_clr, h.clr.data(), h.clr.size() * sizeof(int), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(E->dev + o_off, off.data(), off.size() * sizeof(int), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(E->dev + o_vcl, vcl.data(), vcl.size() * sizeof(int), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(E->d_fd, &d, sizeof(d), hipMemcpyHostToDevice));
   h.d = d;
   // the caller's arrays are not referenced after this point
@@ -2281,7 +2324,10 @@ int mhre_eht_chi2_grad(void* handle, const float* params, int n, int ldp, double
   const EhtData* E = static_cast<const EhtData*>(handle);
   CHK(eht_check_batch(E, params, n, ldp, chi2));
   const int ring = E->h.ring_grad && !ring_grad_disabled();
-  HIPCHK(launch_eht_grad9(E->d_fd, params, n, ldp, chi2, grad, ring, static_cast<hipStream_t>(stream)));
+  // the form that MHRE_GRAD_RING=0 asks for runs at every number of points
+  const int split = ring_grad_disabled() ? 1 : grad_split_waves(E, n);
+  HIPCHK(launch_eht_grad9(E->d_fd, params, n, ldp, chi2, grad, ring, split, E->split_lds,
+                          static_cast<hipStream_t>(stream)));
   return MHRE_OK;
 }
 
@@ -2291,7 +2337,17 @@ int mhre_eht_gn_system(void* handle, const float* params, int n, int ldp, double
   const EhtData* E = static_cast<const EhtData*>(handle);
   CHK(eht_check_batch(E, params, n, ldp, chi2));
   if (n > 0 && (!jtr || !jtj)) FAIL(MHRE_EINVAL, "jtr and jtj are required");
-  HIPCHK(launch_eht_gn9(E->d_fd, params, n, ldp, chi2, jtr, jtj, static_cast<hipStream_t>(stream)));
+  HIPCHK(launch_eht_gn9(E->d_fd, params, n, ldp, chi2, jtr, jtj, 0, static_cast<hipStream_t>(stream)));
+  return MHRE_OK;
+}
+
+int mhre_eht_gn_matrices(void* handle, const float* params, int n, int ldp, double* chi2, double* jtr,
+                         double* jtj, void* stream) {
+  (void)hipGetLastError();
+  const EhtData* E = static_cast<const EhtData*>(handle);
+  CHK(eht_check_batch(E, params, n, ldp, chi2));
+  if (n > 0 && (!jtr || !jtj)) FAIL(MHRE_EINVAL, "jtr and jtj are required");
+  HIPCHK(launch_eht_gn9(E->d_fd, params, n, ldp, chi2, jtr, jtj, 1, static_cast<hipStream_t>(stream)));
   return MHRE_OK;
 }
 

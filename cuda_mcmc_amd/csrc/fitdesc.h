@@ -100,6 +100,11 @@ struct FitDesc {
                            // (4 bits per leg), no two legs of one 64-closure batch
                            // and round naming the same visibility; null elsewhere
   int nround;              // rounds per batch (gradient only)
+  // gradient only: the closures that contain visibility j are entries
+  // vcl_off[j] .. vcl_off[j + 1] - 1 of vcl, each 2 * closure (of clo), + 1
+  // where its phase enters with a minus
+  const int* vcl_off;      // [ntile * TILE + 1]
+  const int* vcl;          // [3 * ncph]
   const float* qcoef;      // MODEL_QUADSYS packed coefficients
   const float* qrow;       // MODEL_QUADSYS single-coordinate update rows (QROW_* layout),
                            // null where the step evaluates every equation in full

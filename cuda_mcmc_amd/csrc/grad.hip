@@ -29,6 +29,13 @@ constexpr int NINV = 14;   // cth sth se rq2 kBe kCe kBi kCi kd cr cg gaU gaV kg
 constexpr int NP9 = 9;
 constexpr int NJTJ = NP9 * (NP9 + 1) / 2;
 
+// The parameters that each invariant depends on (bit j: parameter j of Zsp Re
+// rq ecc fade gax aq gq th): 35 of the 126 entries of the invariants' Jacobian.
+// The others are exactly zero.
+constexpr int INV_USES[NINV] = {0x100, 0x100, 0x002, 0x004, 0x01e, 0x01e, 0x01e, 0x01e, 0x00e,
+                                0x081, 0x081, 0x062, 0x022, 0x00e};
+__host__ __device__ constexpr bool inv_uses(int m, int j) { return ((INV_USES[m] >> j) & 1) != 0; }
+
 // ------------------------------------------------- float64 forward mode
 
 struct Dual {
@@ -225,8 +232,10 @@ struct GradArgs {
   double* chi2;        // [n]
   float* grad;         // [n][ldp] or null
   double* jtr;         // [n][9]   (k_eht_gn9)
-  double* jtj;         // [n][45]  (k_eht_gn9), row-major upper triangle
+  double* jtj;         // (k_eht_gn9) [n][45], row-major upper triangle, or with full [n][9][9]
+  int full;
 };
+constexpr int GRAD_MAXW = 8;   // most waves that share a point in k_eht_gn9
 
 // Lane j < 9 computes column j of d(inv)/dp into jac[m * 9 + j] (LDS).
 __device__ inline void inv_jacobian(float pl, double* jac) {
@@ -483,65 +492,188 @@ __global__ void __launch_bounds__(256) k_eht_grad9_ring(GradArgs g) {
   }
 }
 
-// Adds the residual row of one datum: dr/dp = J_inv^T dr/dinv.
-__device__ inline void gn_accumulate(const float* rinv, float r, const double* jac, double* jtr, double* jtj) {
-  float row[NP9];
-#pragma unroll
-  for (int j = 0; j < NP9; ++j) {
-    double s = 0.0;
-#pragma unroll
-    for (int m = 0; m < NINV; ++m) s += (double)rinv[m] * jac[m * NP9 + j];
-    row[j] = (float)s;
-  }
-  int k = 0;
-#pragma unroll
-  for (int i = 0; i < NP9; ++i) {
-    jtr[i] += (double)row[i] * (double)r;
-#pragma unroll
-    for (int j = i; j < NP9; ++j) jtj[k++] += (double)row[i] * (double)row[j];
-  }
-}
-
-__global__ void __launch_bounds__(64) k_eht_gn9(GradArgs g) {
+// Gradient of few points, where one wave per point leaves most of the chip idle:
+// the W waves of a work-group share a point's data.  Same terms as
+// k_eht_grad9_ring, in three steps with the whole point's model visibilities
+// and closure adjoints in LDS: wave w models tiles w, w + W, ...; the closures
+// are formed 64 a wave, each leaving its s = -2 dd w; and tile by tile each
+// visibility gathers S_j from the closures that contain it (FitDesc::vcl, so
+// no two lanes add to one place) and runs its reverse pass.
+// 32 points against 2000 visibilities + 600 closures: 47.4 -> 14.9 us.
+template <bool GRAD>
+__global__ void __launch_bounds__(64 * GRAD_SPLIT_MAXW) k_eht_grad9_split(GradArgs g) {
+  extern __shared__ __align__(16) char lds[];
   __shared__ double jac[NINV * NP9];
+  __shared__ double part[GRAD_SPLIT_MAXW][NINV + 1];
   __shared__ float4 btab[2 * BESSEL_TAB_N];
   __shared__ float4 btabd[BESSEL_TAB_N];
   load_bessel_tabs(btab, btabd);
   const BesselTabBCD bt{btab, btabd};
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int W = __builtin_amdgcn_readfirstlane((int)(blockDim.x >> 6));
   const int w = blockIdx.x;
-  if (w >= g.n) return;
   const int lane = lane_id();
-  const FitDesc& f = *g.fd;
+  const FitDesc& f = *(const FitDesc*)wave_const(g.fd);
+  const int nvr = f.ndat - f.ncph, nvis = f.nvis, ntile = f.ntile, ncph = f.ncph;
+  float2* vis_m = reinterpret_cast<float2*>(lds);                // [ntile * TILE]
+  float* clo_s = reinterpret_cast<float*>(vis_m + ntile * TILE);  // [ncph]
   const float pl = lane < NP9 ? g.P[(size_t)w * g.ldp + lane] : 0.0f;
   float p[NP9];
 #pragma unroll
   for (int j = 0; j < NP9; ++j) p[j] = bcast(pl, j);
   const Sgra9::Inv q = Sgra9::prepare(p);
-  inv_jacobian(pl, jac);
+  const GLOBAL float4* vis = gptr(f.vis);
+  double chi = 0.0;
+  for (int t = wid; t < ntile; t += W) {
+    const int i = t * TILE + lane;
+    const float4 d = vis[i];
+    const Fwd9 fw = sgra9_fwd(q, d.x, d.y, bt);
+    if (i < nvr) {
+      const float r = fmaf(-__builtin_amdgcn_sqrtf(fmaf(fw.Vx, fw.Vx, fw.Vy * fw.Vy)), d.w, d.z);
+      chi += (double)(r * r);
+    }
+    vis_m[i] = make_float2(fw.Vx, fw.Vy);
+  }
+  // the last wave has the fewest tiles
+  if (GRAD && wid == W - 1) inv_jacobian(pl, jac);
+  __syncthreads();
+  for (int c = wid * TILE + lane; c < ncph; c += W * TILE) {
+    const int4 ix = gptr(f.clo)[c];
+    const float4 ow = gptr(f.clow)[c];
+    const float dd = closure_resid_v(vis_m[ix.x], vis_m[ix.y], vis_m[ix.z], ow);
+    chi += (double)(dd * dd * ow.z);
+    clo_s[c] = -2.0f * dd * ow.z;   // dd = obs - pa - pb + pc: d(dd^2 w)/dpa
+  }
+  double a[NINV];
+#pragma unroll
+  for (int m = 0; m < NINV; ++m) a[m] = 0.0;
+  if (GRAD) {
+    __syncthreads();
+    for (int t = wid; t < ntile; t += W) {
+      const int j = t * TILE + lane;
+      if (j < nvis) {
+        const float4 d = vis[j];
+        float S = 0.0f;
+        for (int e = gptr(f.vcl_off)[j]; e < gptr(f.vcl_off)[j + 1]; ++e) {
+          const int v = gptr(f.vcl)[e];   // closure, and whether it enters as -p
+          const float s = clo_s[v >> 1];
+          S += (v & 1) ? -s : s;
+        }
+        const Fwd9 fw = sgra9_fwd(q, d.x, d.y, bt);
+        const float m2 = fmaxf(fmaf(fw.Vx, fw.Vx, fw.Vy * fw.Vy), 1e-30f);
+        const float rs = __builtin_amdgcn_rsqf(m2);   // 1/|V|: |V| = m2 rs, 1/|V|^2 = rs^2
+        float sa = 0.0f;
+        if (j < nvr) sa = -2.0f * fmaf(-m2 * rs, d.w, d.z) * d.w * rs;   // -2 (d - |V|) w / |V|
+        const float k = S * (rs * rs);
+        float af[NINV];
+#pragma unroll
+        for (int m = 0; m < NINV; ++m) af[m] = 0.0f;
+        sgra9_bwd(q, fw, fmaf(sa, fw.Vx, -k * fw.Vy), fmaf(sa, fw.Vy, k * fw.Vx), af);
+#pragma unroll
+        for (int m = 0; m < NINV; ++m) a[m] += (double)af[m];
+      }
+    }
+  }
+  chi = wave_sum(chi);
+  if (lane == 0) part[wid][NINV] = chi;
+  if (GRAD) {
+#pragma unroll
+    for (int m = 0; m < NINV; ++m) {
+      const double s = wave_sum(a[m]);
+      if (lane == 0) part[wid][m] = s;
+    }
+  }
+  __syncthreads();
+  static_assert(sizeof(jac) + sizeof(part) + sizeof(btab) + sizeof(btabd) <= GRAD_SPLIT_STATIC_LDS, "split rule");
+  if (wid != 0) return;
+  if (lane <= NINV) {
+    double s = 0.0;
+    for (int i = 0; i < W; ++i) s += part[i][lane];
+    part[0][lane] = s;
+  }
+  wave_sync_lds();
+  if (lane == 0) g.chi2[w] = part[0][NINV];
+  if (GRAD && lane < g.ldp) {
+    double gj = 0.0;
+    if (lane < NP9) {
+#pragma unroll
+      for (int m = 0; m < NINV; ++m) gj += part[0][m] * jac[m * NP9 + lane];
+    }
+    g.grad[(size_t)w * g.ldp + lane] = (float)gj;
+  }
+}
+
+// Sums of 64 values over the 64 lanes, value l's on lane l: in the step of lane
+// bit b each lane hands the half of its values that its partner keeps over to
+// it, so the 64 sums take 63 additions a lane and not 6 (or 8, wave_sum) each.
+__device__ inline double wave_sums64(double (&v)[64]) {
+  const int lane = lane_id();
+#pragma unroll
+  for (int b = 0; b < 6; ++b) {
+    const bool hi = ((lane >> b) & 1) != 0;
+#pragma unroll
+    for (int i = 0; i < (32 >> b); ++i) {
+      const double keep = hi ? v[2 * i + 1] : v[2 * i], give = hi ? v[2 * i] : v[2 * i + 1];
+      v[i] = keep + (b == 0 ? dpp_double<0xB1>(give) : b == 1 ? dpp_double<0x4E>(give) : __shfl_xor(give, 1 << b, 64));
+    }
+  }
+  return v[0];
+}
+
+// Adds the residual row of one datum, dr/dp = J_inv^T dr/dinv, to s: chi^2,
+// J^T r, then the upper triangle of J^T J by rows.
+__device__ inline void gn_accumulate(const float* rinv, float r, const double* jac, double* s) {
+  float row[NP9];
+#pragma unroll
+  for (int j = 0; j < NP9; ++j) {
+    double t = 0.0;
+#pragma unroll
+    for (int m = 0; m < NINV; ++m)
+      if (inv_uses(m, j)) t += (double)rinv[m] * jac[m * NP9 + j];
+    row[j] = (float)t;
+  }
+  s[0] += (double)r * (double)r;
+  int k = 1 + NP9;
+#pragma unroll
+  for (int i = 0; i < NP9; ++i) {
+    s[1 + i] += (double)row[i] * (double)r;
+#pragma unroll
+    for (int j = i; j < NP9; ++j) s[k++] += (double)row[i] * (double)row[j];
+  }
+}
+
+// J^T J and J^T r of one point a work-group, its data shared by the
+// work-group's 1 to GRAD_MAXW waves (the launch takes as many as few points
+// leave the chip idle).  Bound by float64 arithmetic: per datum 35 products
+// for the row (the nonzero entries of J_inv) and 55 for the sums.
+// 16 points against 2000 visibilities + 600 closures: 88.9 us with one wave a
+// point and all 126 products of the row, 12 now.
+__global__ void __launch_bounds__(512) k_eht_gn9(GradArgs g) {
+  __shared__ double jac[NINV * NP9];
+  __shared__ double part[GRAD_MAXW][64];
+  __shared__ float4 btab[2 * BESSEL_TAB_N];
+  __shared__ float4 btabd[BESSEL_TAB_N];
+  load_bessel_tabs(btab, btabd);
+  const BesselTabBCD bt{btab, btabd};
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int W = __builtin_amdgcn_readfirstlane((int)(blockDim.x >> 6));
+  const int w = blockIdx.x;
+  const int lane = lane_id();
+  const FitDesc& f = *(const FitDesc*)wave_const(g.fd);
+  const float pl = lane < NP9 ? g.P[(size_t)w * g.ldp + lane] : 0.0f;
+  float p[NP9];
+#pragma unroll
+  for (int j = 0; j < NP9; ++j) p[j] = bcast(pl, j);
+  const Sgra9::Inv q = Sgra9::prepare(p);
+  if (wid == 0) inv_jacobian(pl, jac);
+  __syncthreads();
 
   const int nvr = f.ndat - f.ncph;
-  double chi = 0.0;
-  double jtr[NP9], jtj[NJTJ];
+  double s[64];
 #pragma unroll
-  for (int i = 0; i < NP9; ++i) jtr[i] = 0.0;
-#pragma unroll
-  for (int i = 0; i < NJTJ; ++i) jtj[i] = 0.0;
-  for (int i = lane; i < nvr; i += 64) {
-    const float4 d = gptr(f.vis)[i];
-    const Fwd9 fw = sgra9_fwd(q, d.x, d.y, bt);
-    const float amp = __builtin_amdgcn_sqrtf(fmaf(fw.Vx, fw.Vx, fw.Vy * fw.Vy));
-    const float sw = d.w;   // vis holds (d sqrt(w), sqrt(w))
-    const float r = fmaf(-amp, sw, d.z);
-    chi += (double)r * (double)r;
-    // dr/dV = -sqrt(w) V / amp
-    const float s = -sw * __builtin_amdgcn_rcpf(fmaxf(amp, 1e-30f));
-    float rinv[NINV];
-#pragma unroll
-    for (int m = 0; m < NINV; ++m) rinv[m] = 0.0f;
-    sgra9_bwd(q, fw, s * fw.Vx, s * fw.Vy, rinv);
-    gn_accumulate(rinv, r, jac, jtr, jtj);
-  }
-  for (int c = lane; c < f.ncph; c += 64) {
+  for (int i = 0; i < 64; ++i) s[i] = 0.0;
+  // the closures first, which take three times as long, from the last wave on
+  for (int c = (W - 1 - wid) * TILE + lane; c < f.ncph; c += W * TILE) {
     const int4 ix = gptr(f.clo)[c];
     const float4 ow = gptr(f.clow)[c];
     const GLOBAL float4* vis = gptr(f.vis);
@@ -551,7 +683,6 @@ __global__ void __launch_bounds__(64) k_eht_gn9(GradArgs g) {
     const Fwd9 fe = sgra9_fwd(q, de.x, de.y, bt);
     const float sw = __builtin_amdgcn_sqrtf(ow.z);
     const float r = closure_resid(fa, fb, fe, ow) * sw;
-    chi += (double)r * (double)r;
     // r = sqrt(w) (obs - pa - pb + pc)
     const float2 ga = darg(fa, -sw), gb = darg(fb, -sw), ge = darg(fe, sw);
     float rinv[NINV];
@@ -560,36 +691,73 @@ __global__ void __launch_bounds__(64) k_eht_gn9(GradArgs g) {
     sgra9_bwd(q, fa, ga.x, ga.y, rinv);
     sgra9_bwd(q, fb, gb.x, gb.y, rinv);
     sgra9_bwd(q, fe, ge.x, ge.y, rinv);
-    gn_accumulate(rinv, r, jac, jtr, jtj);
+    gn_accumulate(rinv, r, jac, s);
   }
-  chi = wave_sum(chi);
+  for (int i = wid * TILE + lane; i < nvr; i += W * TILE) {
+    const float4 d = gptr(f.vis)[i];
+    const Fwd9 fw = sgra9_fwd(q, d.x, d.y, bt);
+    const float amp = __builtin_amdgcn_sqrtf(fmaf(fw.Vx, fw.Vx, fw.Vy * fw.Vy));
+    const float sw = d.w;   // vis holds (d sqrt(w), sqrt(w))
+    const float r = fmaf(-amp, sw, d.z);
+    // dr/dV = -sqrt(w) V / amp
+    const float k = -sw * __builtin_amdgcn_rcpf(fmaxf(amp, 1e-30f));
+    float rinv[NINV];
 #pragma unroll
-  for (int i = 0; i < NP9; ++i) jtr[i] = wave_sum(jtr[i]);
-#pragma unroll
-  for (int i = 0; i < NJTJ; ++i) jtj[i] = wave_sum(jtj[i]);
-  if (lane == 0) {
-    g.chi2[w] = chi;
-#pragma unroll
-    for (int i = 0; i < NP9; ++i) g.jtr[(size_t)w * NP9 + i] = jtr[i];
-#pragma unroll
-    for (int i = 0; i < NJTJ; ++i) g.jtj[(size_t)w * NJTJ + i] = jtj[i];
+    for (int m = 0; m < NINV; ++m) rinv[m] = 0.0f;
+    sgra9_bwd(q, fw, k * fw.Vx, k * fw.Vy, rinv);
+    gn_accumulate(rinv, r, jac, s);
+  }
+  part[wid][lane] = wave_sums64(s);
+  __syncthreads();
+  if (wid != 0) return;
+  double v = 0.0;
+  for (int i = 0; i < W; ++i) v += part[i][lane];
+  if (lane == 0) g.chi2[w] = v;
+  else if (lane <= NP9) g.jtr[(size_t)w * NP9 + lane - 1] = v;
+  else if (lane < 1 + NP9 + NJTJ) {
+    const int k = lane - 1 - NP9;
+    if (g.full) {
+      // both triangles of the 9 x 9 matrix
+      int i = 0, first = 0;
+      while (k >= first + NP9 - i) first += NP9 - i++;
+      const int j = i + k - first;
+      double* m = g.jtj + (size_t)w * NP9 * NP9;
+      m[i * NP9 + j] = v;
+      m[j * NP9 + i] = v;
+    } else {
+      g.jtj[(size_t)w * NJTJ + k] = v;
+    }
   }
 }
 
+// Waves per point: as many as keep the launch within GRAD_WAVES, 4 per SIMD.
+constexpr int GRAD_WAVES = 4096;
+static int waves_per_point(int n) {
+  int w = GRAD_MAXW;
+  while (w > 1 && (long long)n * w > GRAD_WAVES) w >>= 1;
+  return w;
+}
+
 hipError_t launch_eht_grad9(const FitDesc* fd, const float* P, int n, int ldp, double* chi2, float* grad,
-                            int ring, hipStream_t s) {
+                            int ring, int split, size_t split_lds, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  GradArgs g{fd, P, n, ldp, chi2, grad, nullptr, nullptr};
-  if (ring) k_eht_grad9_ring<<<(n + 3) / 4, 256, 0, s>>>(g);
-  else k_eht_grad9<<<(n + 3) / 4, 256, 0, s>>>(g);
+  GradArgs g{fd, P, n, ldp, chi2, grad, nullptr, nullptr, 0};
+  if (split > 1) {
+    if (grad) k_eht_grad9_split<true><<<n, 64 * split, split_lds, s>>>(g);
+    else k_eht_grad9_split<false><<<n, 64 * split, split_lds, s>>>(g);
+  } else if (ring) {
+    k_eht_grad9_ring<<<(n + 3) / 4, 256, 0, s>>>(g);
+  } else {
+    k_eht_grad9<<<(n + 3) / 4, 256, 0, s>>>(g);
+  }
   return hipGetLastError();
 }
 
 hipError_t launch_eht_gn9(const FitDesc* fd, const float* P, int n, int ldp, double* chi2, double* jtr,
-                          double* jtj, hipStream_t s) {
+                          double* jtj, int full, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  GradArgs g{fd, P, n, ldp, chi2, nullptr, jtr, jtj};
-  k_eht_gn9<<<n, 64, 0, s>>>(g);
+  GradArgs g{fd, P, n, ldp, chi2, nullptr, jtr, jtj, full};
+  k_eht_gn9<<<n, 64 * waves_per_point(n), 0, s>>>(g);
   return hipGetLastError();
 }
 

@@ -241,6 +241,9 @@ int mhre_eht_chi2_grad(void *handle, const float *params, int n, int ldp,
  * triangle of J^T J row by row, jtj[n][45]. */
 int mhre_eht_gn_system(void *handle, const float *params, int n, int ldp,
                        double *chi2, double *jtr, double *jtj, void *stream);
+/* The same with both triangles of J^T J: jtj[n][9][9]. */
+int mhre_eht_gn_matrices(void *handle, const float *params, int n, int ldp,
+                         double *chi2, double *jtr, double *jtj, void *stream);
 int mhre_eht_data_destroy(void *handle);
 /* How the data were packed (no reference counterpart): info[0] = 1 if the
  * gradient uses the single-pass ring kernel, info[1] = its closure-adjoint
