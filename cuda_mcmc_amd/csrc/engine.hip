@@ -1024,6 +1024,7 @@ struct QuadCarry {
   uint32_t nacc[CACHE ? (NQ + 1) / 2 : 1];
   float* sp;
   uint32_t* hw;
+  const float4* par;   // per parameter k: ivar[k], its pdescr (as bits), pmint and pmaxt
   // the last proposal's accept flag, parameter and old value
   int flag, tlast;
   float told;
@@ -1082,7 +1083,7 @@ __device__ inline void quad_store(const FitDesc& f, int ch, bool hist, const Qua
 // n + 3 operations per equation instead of n(n+1)/2 + n.  Its chi^2 is the
 // same sum of squares to float rounding (sqrt(w) r)^2 against r^2 w.
 template <int NQ, bool CACHE, bool ROWS = false>
-__device__ unsigned quad_substeps(const FitDesc& f, int ch, int ibeta, int it, const TraceBuf& tr, float (&x)[NQ],
+__device__ unsigned quad_substeps(const FitDesc& f, int ch, float betaf, int it, const TraceBuf& tr, float (&x)[NQ],
                                   float& chi2c, QuadCarry<NQ, CACHE>& q, const float* rows = nullptr) {
   const int C = f.nchain, P = f.nprm;
   const CONSTANT float* qc = wave_const(f.qcoef);
@@ -1097,7 +1098,7 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, int ibeta, int it, c
   const CONSTANT float* pmint = wave_const(f.pmint);
   const CONSTANT float* pmaxt = wave_const(f.pmaxt);
   const bool burn = it < f.nburn;
-  const double beta = (double)gptr(f.beta)[ibeta];
+  const double beta = (double)betaf;
   const int nadj = __builtin_amdgcn_readfirstlane(f.nadj);
   const int hwn = __builtin_amdgcn_readfirstlane(f.hwords);
   const float rnadj = 1.0f / (float)nadj;
@@ -1108,7 +1109,11 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, int ibeta, int it, c
   for (int s = 0; s < P; ++s) {
     const U4 r = philox4x32_10((uint32_t)ch, (uint32_t)it, (uint32_t)s, 0u, f.key0, f.key1);
     const int k = pick_with_retry(r.x, P, (uint32_t)ch, (uint32_t)it, (uint32_t)s, 0u, f.key0, f.key1);
-    const int t = ivar[k];
+    // CACHE: the parameter's constants with one LDS read (lanes pick different
+    // ones, so each read from memory would be waited for in turn)
+    float4 par = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (CACHE) par = q.par[k];
+    const int t = CACHE ? __float_as_int(par.x) : ivar[k];
     const int pk = k * C + ch;   // 32-bit element offsets: the host bounds nprm * nchain * hwords
     float old = 0.0f;
 #pragma unroll
@@ -1141,8 +1146,8 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, int ibeta, int it, c
     const float z = __builtin_amdgcn_sqrtf(-1.3862943611198906f * __builtin_amdgcn_logf(u01(r.y))) *
                     __builtin_amdgcn_cosf(u01(r.z));
     float pn = fmaf(sd, z, old);
-    if (pdescr[t] == 2) pn = wrap_angle(pn);
-    const bool inprior = !(pn < pmint[t] || pn > pmaxt[t]);
+    if ((CACHE ? __float_as_int(par.y) : pdescr[t]) == 2) pn = wrap_angle(pn);
+    const bool inprior = !(pn < (CACHE ? par.z : pmint[t]) || pn > (CACHE ? par.w : pmaxt[t]));
     int acc = 0;
     double c2 = 0.0;
     if (inprior) {
@@ -1230,7 +1235,7 @@ __device__ unsigned quad_one_chain(const FitDesc& f, int ch, int it, const Trace
   for (int i = 0; i < NQ; ++i) x[i] = pcur[(size_t)ch * NQ + i];
   float chi2c = gptr(f.chi2c)[ch];
   QuadCarry<NQ, false> q;
-  const unsigned nev = quad_substeps<NQ, false>(f, ch, ch / f.nseq, it, tr, x, chi2c, q);
+  const unsigned nev = quad_substeps<NQ, false>(f, ch, gptr(f.beta)[ch / f.nseq], it, tr, x, chi2c, q);
 #pragma unroll
   for (int i = 0; i < NQ; ++i) pcur[(size_t)ch * NQ + i] = x[i];
   gptr(f.chi2c)[ch] = chi2c;
@@ -1433,6 +1438,7 @@ struct __align__(16) QuadLds {
   float rows[ROWS ? NQ * QROW_TS(NQ) : 4];   // the fit's update rows
   float sp[NQ * 64];
   uint32_t hw[NQ * 64];
+  float4 par[NQ];
   LadderLds ladder;
 };
 
@@ -1458,6 +1464,12 @@ __device__ void iter_quad_wave(const FitDesc& f0, int iseq0, int it0, int it1, c
   QuadCarry<NQ, true> q;
   q.sp = lds.sp;
   q.hw = lds.hw;
+  q.par = lds.par;
+  if (lane < f.nprm) {
+    const int t = gptr(f.ivar)[lane];
+    lds.par[lane] = make_float4(__int_as_float(t), __int_as_float(gptr(f.pdescr)[t]), gptr(f.pmint)[t], gptr(f.pmaxt)[t]);
+  }
+  const float beta = slot ? gptr(f.beta)[sl] : 0.0f;
   float x[NQ];
   float c2 = 0.0f;
   int tc = 0;
@@ -1474,8 +1486,8 @@ __device__ void iter_quad_wave(const FitDesc& f0, int iseq0, int it0, int it1, c
     const GLOBAL float4* src = (const GLOBAL float4*)gptr(f.qrow);
     float4* dst = reinterpret_cast<float4*>(lds.rows);
     for (int i = lane; i < n4; i += 64) dst[i] = src[i];
-    ring_fence();
   }
+  ring_fence();
   const double hb = swap_factor(f, sl);
   unsigned nev = 0;
   int nex = 0;
@@ -1483,7 +1495,7 @@ __device__ void iter_quad_wave(const FitDesc& f0, int iseq0, int it0, int it1, c
     const FitDesc& f = fit_again(f0);
     const int B = f.nbeta, S = f.nseq, ch = value_again(ch0);
     const bool burn = it < f.nburn;
-    if (slot) nev += quad_substeps<NQ, true, ROWS>(f, ch, sl, it, tr, x, c2, q, lds.rows);
+    if (slot) nev += quad_substeps<NQ, true, ROWS>(f, ch, beta, it, tr, x, c2, q, lds.rows);
 
     // exchange: as exchange_wave, with slot k of the sequence at lane k * G + g
     if (B > 1) {

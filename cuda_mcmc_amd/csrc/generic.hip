@@ -194,6 +194,16 @@ __device__ inline UserSlot user_slot(char* lds, int P) {
   return u;
 }
 
+// Per varied parameter k: ivar[k], its pdescr (as bits), pmint and pmaxt, in the
+// wave's LDS: a chain's lanes read them one after the other, each proposal anew.
+__device__ inline void user_params(const FitDesc& f, float4* par) {
+  const int k = lane_id();
+  if (k < f.nprm) {
+    const int t = gptr(f.ivar)[k];
+    par[k] = make_float4(__int_as_float(t), __int_as_float(gptr(f.pdescr)[t]), gptr(f.pmint)[t], gptr(f.pmaxt)[t]);
+  }
+}
+
 // Place and number of a wave's lanes of a chain, for work that every wave of
 // the chain does by itself.
 template <int Waves>
@@ -261,23 +271,23 @@ __device__ inline void user_draw(const FitDesc& f, const ChainLanes<Waves>& cl, 
 // current half of u.row.
 template <int Waves, bool OneDatum>
 __device__ unsigned user_substeps(const FitDesc& f, CCalcModel* mc, ChainLanes<Waves>& cl, int ch, int it,
-                                  const TraceBuf& tr, const UserSlot& u, const UserDraws& d, float* row, float& chi2c,
-                                  float* term, LastProposal& last, int* err) {
+                                  const TraceBuf& tr, const UserSlot& u, const UserDraws& d, const float4* par,
+                                  double beta, float* row, float& chi2c, float* term, LastProposal& last, int* err) {
   const int C = f.nchain, P = f.nprm, N = f.nptot;
   const bool burn = it < f.nburn;
-  const double beta = (double)gptr(f.beta)[ch / f.nseq];
   const int nadj = f.nadj;
   const float rnadj = 1.0f / (float)nadj;
   GLOBAL float* prow = gptr(f.pcur) + (size_t)ch * N;
   unsigned nev = 0;
   for (int s = 0; s < P; ++s) {
     const int k = d.k[s];
-    const int t = gptr(f.ivar)[k];
+    const float4 pk = par[k];
+    const int t = __float_as_int(pk.x);
     const float old = row[t], sd = u.stp[k];
     double pd = (double)old + (double)sd * d.z[s];
-    if (gptr(f.pdescr)[t] == 2) pd = pd - 6.283185307179586 * rint(pd / 6.283185307179586);
+    if (__float_as_int(pk.y) == 2) pd = pd - 6.283185307179586 * rint(pd / 6.283185307179586);
     const float pn = (float)pd;
-    const bool inprior = !(pn < gptr(f.pmint)[t] || pn > gptr(f.pmaxt)[t]);
+    const bool inprior = !(pn < pk.z || pn > pk.w);
     wave_sync_lds();   // every lane has read its row and step size
     int acc = 0;
     double c2 = 0.0;
@@ -347,6 +357,7 @@ __global__ void __launch_bounds__(64 * Waves) k_step_user(const FitDesc* fits, c
                                                        int slot_bytes) {
   extern __shared__ __align__(16) char lds[];
   __shared__ double xs[2 * Waves];
+  __shared__ float4 par[Waves][MAXP];
   const int lane = lane_id();
   const int per = Waves == 1 ? 64 / lanes : 1;
   const int c = Waves == 1 ? lane / lanes : 0;
@@ -359,18 +370,21 @@ __global__ void __launch_bounds__(64 * Waves) k_step_user(const FitDesc* fits, c
   const bool live = ch >= 0;   // padding lanes only take part in the counting
   ChainLanes<Waves> cl{Waves == 1 ? lanes : 64 * Waves, Waves == 1 ? lane & (lanes - 1) : (int)threadIdx.x, xs, 0};
   unsigned nev = 0;
+  const int wid = Waves == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  user_params(f, par[wid]);
   if (live) {
-    const int wid = Waves == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const UserSlot u = user_slot(lds + (size_t)(wid * per + c) * slot_bytes, f.nprm);
     const bool hist = it < f.nburn;
     CCalcModel mc = user_model_args(f);
     float chi2c = gptr(f.chi2c)[ch], term;
     LastProposal last{0, 0, 0.0f};
     int err = 0;
+    const double beta = (double)gptr(f.beta)[ch / f.nseq];
     user_load(f, cl, ch, u, hist);
     user_draw(f, cl, ch, it, u.d[0]);
     wave_sync_lds();
-    nev = user_substeps<Waves, false>(f, &mc, cl, ch, it, tr, u, u.d[0], u.row, chi2c, &term, last, &err);
+    nev = user_substeps<Waves, false>(f, &mc, cl, ch, it, tr, u, u.d[0], par[wid], beta, u.row, chi2c, &term, last,
+                                      &err);
     chain_fence<Waves>();   // every wave's state is final and no wave reads the arrays any more
     user_store(f, cl, ch, u, hist);
     if (cl.j == 0) {
@@ -400,6 +414,7 @@ __global__ void __launch_bounds__(128) k_iter_user(const FitDesc* fits, const Wo
   extern __shared__ __align__(16) char lds[];
   __shared__ LadderLds ladder;
   __shared__ SwapDraw swap[2][64];
+  __shared__ float4 par[MAXP];
   const WorkItem w = work[blockIdx.x];
   const FitDesc& f = wave_fit(fits, w.fit);
   pass_clock(clk);
@@ -440,6 +455,8 @@ __global__ void __launch_bounds__(128) k_iter_user(const FitDesc* fits, const Wo
     user_load(f, cl, ch, u, hist);
   }
   const double hb = swap_factor(f, sl);
+  const double beta = live ? (double)gptr(f.beta)[sl] : 0.0;
+  user_params(f, par);
   wave_sync_lds();
   float* row = u.row;
   float* other = u.row + N;
@@ -447,7 +464,8 @@ __global__ void __launch_bounds__(128) k_iter_user(const FitDesc* fits, const Wo
     const int it = it0 + i;
     __syncthreads();   // this iteration's draws are there, the one before's are free
     const bool burn = it < f.nburn;
-    if (live) nev += user_substeps<1, OneDatum>(f, &mc, cl, ch, it, tr, u, u.d[i & 1], row, chi2c, &term, last, &err);
+    if (live) nev += user_substeps<1, OneDatum>(f, &mc, cl, ch, it, tr, u, u.d[i & 1], par, beta, row,
+                                                chi2c, &term, last, &err);
     nprop += P;
     int perm = sl;
     if (nb > 1) {
