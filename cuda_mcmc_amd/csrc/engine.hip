@@ -174,7 +174,11 @@ __device__ double eht_chi2_wave(const EhtView& v, const typename M::Inv& q, floa
     int4 ix = buf_load_i4(cb, l16, (uint32_t)c0 * 16u);
     float4 ow = buf_load_f4(wb, l16, (uint32_t)c0 * 16u);
     const bool any_large = __float_as_uint(r2cur) > r2_thr;
-    const float2 V = M::template vis<BesselTab, HW>(q, d.x, d.y, r2, any_large, bt);
+    // one copy of the model per branch: the table's small-argument form then
+    // is straight-line code up to the phases
+    float2 V;
+    if (!any_large) V = M::template vis<BesselTab, HW>(q, d.x, d.y, r2, false, bt);
+    else V = M::template vis<BesselTab, HW>(q, d.x, d.y, r2, true, bt);
     const float amp = __builtin_amdgcn_sqrtf(fmaf(V.x, V.x, V.y * V.y));
     const float r = fmaf(-amp, d.w, d.z);   // (d - |V|) sqrt(w); zero past the amplitude data
     part = fmaf(r, r, part);
