@@ -1015,39 +1015,54 @@ __global__ void __launch_bounds__(256) k_eval_quad(const FitDesc* fits, const Wo
 }
 
 // What a lane keeps of its chain besides x and chi2c while a launch runs.
-// CACHE (k_iter_quad, many iterations a launch): the adaptation counters n_cnt
-// and sumh of all its parameters, and the accepted proposals of each in 16-bit
-// counts; the step sizes and the current acceptance-history words (the word
-// that holds entry cnt % nadj) sit in the wave's LDS, [NQ][64] each, column =
-// lane.  Lanes pick different parameters, so per-proposal accesses in memory
-// scatter over rows, each lane a cache line of its own; held for the launch,
-// every array moves once per launch instead.
+// CACHE (k_iter_quad, many iterations a launch): sumh of all its parameters, and
+// in place of each n_cnt what the proposals need of it, ent = n_cnt below nadj
+// and nadj + n_cnt % nadj from there on, which goes on by one addition and one
+// wrap.  In the wave's LDS, [NQ][64] each, column = lane: the step sizes, the
+// current acceptance-history words (the word that holds entry n_cnt % nadj),
+// and the launch's burn-in proposals and accepted proposals of each parameter
+// in 16 bits each.  Lanes pick different parameters, so per-proposal accesses in
+// memory scatter over rows, each lane a cache line of its own; held for the
+// launch, every array moves once per launch instead.  What a lane only adds to
+// (ndone) is no register array: picking the element takes selects, and held in
+// registers the counts were spilled to memory in every proposal.  Eight
+// parameters' LDS is as much as lets 4 waves per SIMD be resident.  512 systems of
+// 8 equations, 16 x 32 chains: sampling 24.3 -> 19.8 us an iteration, burn-in
+// 32.1 -> 25.6.
 template <int NQ, bool CACHE>
 struct QuadCarry {
-  int cnt[CACHE ? NQ : 1], sh[CACHE ? NQ : 1];
-  uint32_t nacc[CACHE ? (NQ + 1) / 2 : 1];
+  uint32_t ent[CACHE ? NQ : 1];
+  int sh[CACHE ? NQ : 1];
   float* sp;
   uint32_t* hw;
+  uint32_t* ndone;   // proposals << 16 | accepted
+  const float* beta;   // per lane
   const float4* par;   // per parameter k: ivar[k], its pdescr (as bits), pmint and pmaxt
   // the last proposal's accept flag, parameter and old value
   int flag, tlast;
   float told;
 };
-static_assert(SEQ_ITERS * 8 <= 65535, "a launch's accepted proposals of one parameter fit 16 bits");
+static_assert(SEQ_ITERS * 8 <= 65535, "a launch's proposals of one parameter fit 16 bits");
+
+// n_cnt % nadj from QuadCarry::ent.
+__device__ inline uint32_t hist_entry(uint32_t ent, int nadj) {
+  return ent < (uint32_t)nadj ? ent : ent - (uint32_t)nadj;
+}
 
 // hist: the launch has burn-in iterations.
 template <int NQ>
 __device__ inline void quad_load(const FitDesc& f, int ch, bool hist, QuadCarry<NQ, true>& q) {
   const int C = f.nchain, P = f.nprm, ln = lane_id();
 #pragma unroll
-  for (int i = 0; i < (NQ + 1) / 2; ++i) q.nacc[i] = 0;
-#pragma unroll
   for (int i = 0; i < NQ; ++i) {
-    q.cnt[i] = q.sh[i] = 0;
+    q.ent[i] = 0;
+    q.sh[i] = 0;
+    q.ndone[i * 64 + ln] = 0;
     if (i < P) {
       q.sp[i * 64 + ln] = gptr(f.pstp)[i * C + ch];
       if (hist) {
-        q.cnt[i] = gptr(f.n_cnt)[i * C + ch];
+        const int cnt = gptr(f.n_cnt)[i * C + ch];
+        q.ent[i] = cnt < f.nadj ? (uint32_t)cnt : (uint32_t)f.nadj + (uint32_t)(cnt % f.nadj);
         q.sh[i] = gptr(f.sumh)[i * C + ch];
       }
     }
@@ -1055,7 +1070,7 @@ __device__ inline void quad_load(const FitDesc& f, int ch, bool hist, QuadCarry<
   if (hist) {
 #pragma unroll
     for (int i = 0; i < NQ; ++i)
-      if (i < P) q.hw[i * 64 + ln] = gptr(f.hbits)[(ch * f.hwords + ((q.cnt[i] % f.nadj) >> 5)) * P + i];
+      if (i < P) q.hw[i * 64 + ln] = gptr(f.hbits)[(ch * f.hwords + (int)(hist_entry(q.ent[i], f.nadj) >> 5)) * P + i];
   }
 }
 // Acceptance counts only where a proposal was accepted (a lane left out
@@ -1066,13 +1081,14 @@ __device__ inline void quad_store(const FitDesc& f, int ch, bool hist, const Qua
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
     if (i < P) {
-      const int na = (int)((q.nacc[i / 2] >> (16 * (i & 1))) & 0xffffu);
+      const uint32_t nd = q.ndone[i * 64 + ln];
+      const int na = (int)(nd & 0xffffu);
       if (na) gptr(f.n_acpt)[i * C + ch] += na;
       if (hist) {
-        gptr(f.n_cnt)[i * C + ch] = q.cnt[i];
+        gptr(f.n_cnt)[i * C + ch] += (int)(nd >> 16);
         gptr(f.sumh)[i * C + ch] = q.sh[i];
         gptr(f.pstp)[i * C + ch] = q.sp[i * 64 + ln];
-        gptr(f.hbits)[(ch * f.hwords + ((q.cnt[i] % f.nadj) >> 5)) * P + i] = q.hw[i * 64 + ln];
+        gptr(f.hbits)[(ch * f.hwords + (int)(hist_entry(q.ent[i], f.nadj) >> 5)) * P + i] = q.hw[i * 64 + ln];
       }
     }
   }
@@ -1087,7 +1103,7 @@ __device__ inline void quad_store(const FitDesc& f, int ch, bool hist, const Qua
 // n + 3 operations per equation instead of n(n+1)/2 + n.  Its chi^2 is the
 // same sum of squares to float rounding (sqrt(w) r)^2 against r^2 w.
 template <int NQ, bool CACHE, bool ROWS = false>
-__device__ unsigned quad_substeps(const FitDesc& f, int ch, float betaf, int it, const TraceBuf& tr, float (&x)[NQ],
+__device__ unsigned quad_substeps(const FitDesc& f, int ch, int it, const TraceBuf& tr, float (&x)[NQ],
                                   float& chi2c, QuadCarry<NQ, CACHE>& q, const float* rows = nullptr) {
   const int C = f.nchain, P = f.nprm;
   const CONSTANT float* qc = wave_const(f.qcoef);
@@ -1102,7 +1118,7 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, float betaf, int it,
   const CONSTANT float* pmint = wave_const(f.pmint);
   const CONSTANT float* pmaxt = wave_const(f.pmaxt);
   const bool burn = it < f.nburn;
-  const double beta = (double)betaf;
+  const float betaf = CACHE ? 0.0f : gptr(f.beta)[ch / f.nseq];
   const int nadj = __builtin_amdgcn_readfirstlane(f.nadj);
   const int hwn = __builtin_amdgcn_readfirstlane(f.hwords);
   const float rnadj = 1.0f / (float)nadj;
@@ -1127,19 +1143,20 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, float betaf, int it,
     // cnt % nadj (the oldest one), read before the proposal so that its
     // latency overlaps the chi^2
     int cnt = 0, sh0 = 0, ha = 0;
-    uint32_t hword = 0;
+    uint32_t hword = 0, ent = 0;
     if (burn) {
       if (CACHE) {
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-          cnt = (i == k) ? q.cnt[i] : cnt;
+          ent = (i == k) ? q.ent[i] : ent;
           sh0 = (i == k) ? q.sh[i] : sh0;
         }
+        ha = (int)hist_entry(ent, nadj);
       } else {
         cnt = n_cnt[pk];
         sh0 = sumh[pk];
+        ha = mod_small(cnt, nadj, rnadj);
       }
-      ha = mod_small(cnt, nadj, rnadj);
       hword = CACHE ? q.hw[k * 64 + ln] : hbits[(ch * hwn + (ha >> 5)) * P + k];
     }
     // The Gaussian step in fp32 with the hardware log2 and cosine (which takes
@@ -1163,15 +1180,13 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, float betaf, int it,
         c2 = QuadSys<NQ>::chi2(qc, neq, x);
       }
       ++nev;
-      const double xx = -0.5 * beta * (c2 - (double)chi2c);
+      const double xx = -0.5 * (double)(CACHE ? q.beta[ln] : betaf) * (c2 - (double)chi2c);
       // log u in fp32 (hardware log2): its error, ~1e-7 |log u|, is far inside the tie band
       if ((double)(0.69314718055994531f * __builtin_amdgcn_logf(u01(r.w))) <= xx) {
         acc = 1;
         chi2c = (float)c2;
         if (CACHE) {
-          const uint32_t one = 1u << (16 * (k & 1));
-#pragma unroll
-          for (int i = 0; i < (NQ + 1) / 2; ++i) q.nacc[i] += (k >> 1) == i ? one : 0u;
+          atomicAdd(&q.ndone[k * 64 + ln], 1u);   // the lane's own word: one LDS instruction, nothing to wait for
         } else {
           n_acpt[pk] += 1;
         }
@@ -1207,13 +1222,15 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, float betaf, int it,
         hbits[(ch * hwn + (ha >> 5)) * P + k] = nword;
       }
       const int sh = sh0 + acc - hold;
-      const int den = cnt < nadj ? cnt : nadj;
+      const int den = CACHE ? (int)(ent < (uint32_t)nadj ? ent : (uint32_t)nadj) : cnt < nadj ? cnt : nadj;
       const float nsd = rate_below(sh, den, f.adapt_mid, f.adapt_tie) ? step_shrink(sd) : step_grow(sd);
       if (CACHE) {
         q.sp[k * 64 + ln] = nsd;
+        atomicAdd(&q.ndone[k * 64 + ln], 0x10000u);
+        const uint32_t nent = ent + 1 == 2u * (uint32_t)nadj ? (uint32_t)nadj : ent + 1;
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-          q.cnt[i] = (i == k) ? cnt + 1 : q.cnt[i];
+          q.ent[i] = (i == k) ? nent : q.ent[i];
           q.sh[i] = (i == k) ? sh : q.sh[i];
         }
       } else {
@@ -1239,7 +1256,7 @@ __device__ unsigned quad_one_chain(const FitDesc& f, int ch, int it, const Trace
   for (int i = 0; i < NQ; ++i) x[i] = pcur[(size_t)ch * NQ + i];
   float chi2c = gptr(f.chi2c)[ch];
   QuadCarry<NQ, false> q;
-  const unsigned nev = quad_substeps<NQ, false>(f, ch, gptr(f.beta)[ch / f.nseq], it, tr, x, chi2c, q);
+  const unsigned nev = quad_substeps<NQ, false>(f, ch, it, tr, x, chi2c, q);
 #pragma unroll
   for (int i = 0; i < NQ; ++i) pcur[(size_t)ch * NQ + i] = x[i];
   gptr(f.chi2c)[ch] = chi2c;
@@ -1442,6 +1459,8 @@ struct __align__(16) QuadLds {
   float rows[ROWS ? NQ * QROW_TS(NQ) : 4];   // the fit's update rows
   float sp[NQ * 64];
   uint32_t hw[NQ * 64];
+  uint32_t ndone[NQ * 64];
+  float beta[64];
   float4 par[NQ];
   LadderLds ladder;
 };
@@ -1468,12 +1487,14 @@ __device__ void iter_quad_wave(const FitDesc& f0, int iseq0, int it0, int it1, c
   QuadCarry<NQ, true> q;
   q.sp = lds.sp;
   q.hw = lds.hw;
+  q.ndone = lds.ndone;
   q.par = lds.par;
+  q.beta = lds.beta;
   if (lane < f.nprm) {
     const int t = gptr(f.ivar)[lane];
     lds.par[lane] = make_float4(__int_as_float(t), __int_as_float(gptr(f.pdescr)[t]), gptr(f.pmint)[t], gptr(f.pmaxt)[t]);
   }
-  const float beta = slot ? gptr(f.beta)[sl] : 0.0f;
+  lds.beta[lane] = slot ? gptr(f.beta)[sl] : 0.0f;
   float x[NQ];
   float c2 = 0.0f;
   int tc = 0;
@@ -1499,7 +1520,7 @@ __device__ void iter_quad_wave(const FitDesc& f0, int iseq0, int it0, int it1, c
     const FitDesc& f = fit_again(f0);
     const int B = f.nbeta, S = f.nseq, ch = value_again(ch0);
     const bool burn = it < f.nburn;
-    if (slot) nev += quad_substeps<NQ, true, ROWS>(f, ch, beta, it, tr, x, c2, q, lds.rows);
+    if (slot) nev += quad_substeps<NQ, true, ROWS>(f, ch, it, tr, x, c2, q, lds.rows);
 
     // exchange: as exchange_wave, with slot k of the sequence at lane k * G + g
     if (B > 1) {
@@ -1552,7 +1573,8 @@ __device__ void iter_quad_wave(const FitDesc& f0, int iseq0, int it0, int it1, c
 // proposals).  What bounds it is FP32 issue.  512 systems of 8 equations, 16 x 32
 // chains, an iteration per launch against 64: sampling 37.2 -> 28.1 us an
 // iteration, burn-in (whose per-proposal history and counter accesses kept it
-// waiting on memory) 58.0 -> 35.8 us.
+// waiting on memory) 58.0 -> 35.8 us; with the parameters' constants and the
+// launch's counts in LDS 19.8 and 25.6 us.
 template <int NQ, bool ROWS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ROWS ? 4 : 5)))
 k_iter_quad(const FitDesc* fits, const WorkItem* work, int nwork, RunClock* clk, TraceBuf tr, int it_off, int iters) {
