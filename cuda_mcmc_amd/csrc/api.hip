@@ -501,7 +501,18 @@ bool eht_xfused(const FitHost& h, const MhreOptions& o) {
 // most USER_SEQ_DATA data.  Beyond that, and for longer ladders, k_step_user
 // gives a chain up to 256 lanes: as many as it has data, but no more waves
 // than fill the chip several times over (a wave of fewer chains repeats their
-// bookkeeping on more lanes).
+// bookkeeping on more lanes).  Measured, us an iteration with k_step_user +
+// k_exchange / k_iter_user:
+//   a valley of two parameters, ladders of 32 rungs (2 lanes a chain), 64
+//     sequences: 2 data 16.2 / 4.1, 4: 15.9 / 5.5, 8: 15.9 / 7.4, 32: 31.5 / 18.6;
+//     512 sequences, 8 data: 60.6 / 7.7
+//   the 9-parameter ring+Gaussian as model(), 8 rungs (8 lanes) x 32: 8 data
+//     37.3 / 25.6, 16: 37.2 / 43.9, 28: 39.7 / 78.2; 32 rungs x 32: 8 data 38.9 / 85.0
+// What a model() costs is not known here: four data a lane is where a cheap one
+// still gains twofold and an expensive one loses as much.
+// Waves of k_step_user, 1024 / 2048 / 4096 / 8192 / 16384 at most, the
+// ring+Gaussian, 32 rungs x 128 sequences: 500 visibilities 713 / 398 / 301 / 254
+// / 271, 2000: 2966 / 1561 / 1216 / 954 / 898.
 constexpr int USER_SEQ_DATA = 4;
 constexpr long long USER_WAVES = 8192;
 constexpr int USER_SEQ_LDS = 32 << 10;
