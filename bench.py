@@ -188,7 +188,7 @@ def batched_vs_plain(iters, nfits, log_every=16, session_only=False, streams=2):
             plain_vis += s.stats()["vis_evals"] - e0["vis_evals"]
     plain = plain_vis / tp
     # the same fits one at a time through the reference's per-datum model()
-    # contract (generic model.cuh path, one lane per chain)
+    # contract (generic model.cuh path)
     log("  one session per fit done; now the model.cuh path")
     tg = 0.0
     gen_vis = 0.0

@@ -16,8 +16,11 @@
 //                    through the wave, model visibilities kept in a per-wave
 //                    LDS ring for the closure phases, chi^2 accumulated in fp64
 //                    per lane and reduced across the wave
-//   k_step_quad      the same for systems of quadratic equations, one lane per
-//                    chain (wave-uniform coefficients)
+//   k_step_eht_split the same for sessions of few chains: a work-group per chain
+//   k_iter_quad      the same for systems of quadratic equations, one lane per
+//                    chain (wave-uniform coefficients), many iterations with
+//                    their replica exchange in one launch
+//   k_step_quad      one iteration of them, for ladders of more than 64 rungs
 //   k_exchange       replica_exchange (:533-626); one lane per temperature
 //                    slot, 64 / xlanes sequences per wave
 #include <hip/hip_runtime.h>
