@@ -159,6 +159,8 @@ struct FitHost {
   size_t o_pcur_b = 0, o_chi2c_b = 0, o_tcur_b = 0;   // second state set (xfused)
   int ulanes = 0;                // model.cuh path: lanes per chain (user_lanes)
   bool useq = false;             // model.cuh path: whole sequences per wave (k_iter_user)
+  int ncount = 1;                // copies of its counters (FitDesc::ncount) ...
+  size_t count0 = 0;             // ... and the first one's place among the session's
   bool xfused = false;           // exchange inside the next step launch (FitDesc::xfused)
   bool hwphase = false;          // FitDesc::hwphase
   bool has_datm = false;
@@ -540,6 +542,14 @@ void user_lanes(FitHost& h) {
   h.ulanes = n;
 }
 
+// Copies of a fit's counters (FitDesc::ncount), by the waves that add to them in a launch.
+int count_copies(const FitHost& h) {
+  long long waves = h.nchain;
+  if (h.kind == K_QUAD) waves = h.nchain / 64;
+  if (h.kind == K_USER) waves = h.ulanes < 64 ? (long long)h.nchain * h.ulanes / 64 : h.nchain;
+  return pow2_at_least((int)std::min<long long>(COUNT_MAX, waves / COUNT_WAVES));
+}
+
 // Waves per chain of the ring+Gaussian fits `idx` of a session: 1 (the grid or
 // persistent form), or 4 or 8 (the split form, k_step_eht_split) for sessions
 // whose chains are few enough that a work-group each is resident on the chip
@@ -709,7 +719,8 @@ struct Session {
   char* arena = nullptr;
   size_t arena_bytes = 0;
   FitDesc* d_fits = nullptr;
-  unsigned long long* d_nevals = nullptr;   // [nfits][2]
+  unsigned long long* d_nevals = nullptr;   // every fit's copies of its counters (FitDesc::nevals)
+  size_t ncounts = 0;                       // copies of all fits
   int* d_err = nullptr;
   WorkItem* d_init = nullptr;
   int n_init = 0;
@@ -1274,9 +1285,14 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
   S->arena_bytes = A.bytes;
   HIPCHK(hipMalloc((void**)&S->arena, A.bytes));
   CHK(dev_alloc(S, &S->d_fits, nfits));
-  CHK(dev_alloc(S, &S->d_nevals, 2 * (size_t)nfits));
+  for (FitHost& h : S->fits) {
+    h.ncount = count_copies(h);
+    h.count0 = S->ncounts;
+    S->ncounts += (size_t)h.ncount;
+  }
+  CHK(dev_alloc(S, &S->d_nevals, S->ncounts * COUNT_LINE));
   CHK(dev_alloc(S, &S->d_err, 1));
-  HIPCHK(hipMemsetAsync(S->d_nevals, 0, 2 * sizeof(unsigned long long) * nfits, S->stream));
+  HIPCHK(hipMemsetAsync(S->d_nevals, 0, sizeof(unsigned long long) * S->ncounts * COUNT_LINE, S->stream));
   HIPCHK(hipMemsetAsync(S->d_err, 0, sizeof(int), S->stream));
 
   // decision-trace layout: each fit's [trace_iters][nprm][nchain] decisions and
@@ -1344,7 +1360,8 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
     d.datm = h.has_datm ? at<float>(S, h.o_datm) : nullptr;
     d.chi2m = h.has_datm ? at<float>(S, h.o_chi2m) : nullptr;
     d.mc = at<CCalcModel>(S, h.o_mc);
-    d.nevals = S->d_nevals + 2 * i;
+    d.nevals = S->d_nevals + h.count0 * COUNT_LINE;
+    d.ncount = h.ncount;
     d.errflag = S->d_err;
     d.tr_dec = tr_dec_off[i];
     d.tr_ex = tr_ex_off[i];
@@ -1771,21 +1788,24 @@ int stats(Session* S, MhreStats* st) {
   memset(st, 0, sizeof(*st));
   float ms = 0.0f;
   if (S->iters_done > 0 && hipEventElapsedTime(&ms, S->ev0, S->ev1) == hipSuccess) st->run_ms = ms;
-  std::vector<unsigned long long> ev(2 * S->fits.size());
-  HIPCHK(hipMemcpy(ev.data(), S->d_nevals, ev.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-  for (size_t i = 0; i < S->fits.size(); ++i) {
-    const FitHost& h = S->fits[i];
-    st->chi2_evals += ev[2 * i];
-    st->proposals += ev[2 * i + 1];
+  std::vector<unsigned long long> counts(S->ncounts * COUNT_LINE);
+  HIPCHK(hipMemcpy(counts.data(), S->d_nevals, counts.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
+  for (const FitHost& h : S->fits) {
+    unsigned long long evals = 0;
+    for (int c = 0; c < h.ncount; ++c) {
+      evals += counts[(h.count0 + c) * COUNT_LINE];
+      st->proposals += counts[(h.count0 + c) * COUNT_LINE + 1];
+    }
+    st->chi2_evals += evals;
     if (h.kind == K_SGRA9 || h.kind == K_SGRA13) {
-      st->vis_evals += (double)ev[2 * i] * h.nvis_k;
-      st->cph_evals += (double)ev[2 * i] * h.ncph;
+      st->vis_evals += (double)evals * h.nvis_k;
+      st->cph_evals += (double)evals * h.ncph;
     } else if (h.kind == K_USER && (h.s.imodel == 1 || h.s.imodel == 2) && h.s.idat && h.s.nidat >= 1) {
       // the EHT model.cuh on the generic path: idat = [nvis, ndatm, cpExt]
       const int nv = h.s.idat[0], nc = h.s.ndat - nv;
       const int cpext = h.s.nidat >= 3 ? h.s.idat[2] : 0;
-      st->vis_evals += (double)ev[2 * i] * (nv + (cpext ? 3 * nc : 0));
-      st->cph_evals += (double)ev[2 * i] * nc;
+      st->vis_evals += (double)evals * (nv + (cpext ? 3 * nc : 0));
+      st->cph_evals += (double)evals * nc;
     }
   }
   st->iters_done = S->iters_done;

@@ -68,6 +68,14 @@ __device__ inline double swap_factor(const FitDesc& f, int k) {
   return k < f.nbeta - 1 ? -0.5 * ((double)gptr(f.beta)[k + 1] - (double)gptr(f.beta)[k]) : 0.0;
 }
 
+// Adds to the work-group's copy of the fit's counters; one lane of a wave calls it.
+__device__ inline void add_counts(const FitDesc& f, unsigned nev, unsigned nprop) {
+  if (!f.nevals) return;
+  unsigned long long* c = f.nevals + (size_t)(blockIdx.x & (unsigned)(f.ncount - 1)) * COUNT_LINE;
+  atomicAdd(&c[0], (unsigned long long)nev);
+  atomicAdd(&c[1], (unsigned long long)nprop);
+}
+
 // Adds the wave's performed evaluations and proposals to the fit's counters
 // with one atomic each (every lane of the wave, padding included, calls it).
 __device__ inline void wave_count(const FitDesc& f, unsigned nev, unsigned nprop) {
@@ -77,10 +85,7 @@ __device__ inline void wave_count(const FitDesc& f, unsigned nev, unsigned nprop
     a += (unsigned)__shfl_xor((int)a, m, 64);
     b += (unsigned)__shfl_xor((int)b, m, 64);
   }
-  if (f.nevals && lane_id() == 0) {
-    atomicAdd(&f.nevals[0], (unsigned long long)a);
-    atomicAdd(&f.nevals[1], (unsigned long long)b);
-  }
+  if (lane_id() == 0) add_counts(f, a, b);
 }
 
 // Optional record of the decisions of iterations it0 .. it0+nit-1.

@@ -799,10 +799,7 @@ __device__ __attribute__((always_inline)) void step_one_chain(const FitDesc& f, 
     f.flag[ch] = flag;
     f.ptent[ch] = told;
     f.ptentn[ch] = tlast;
-    if (f.nevals) {
-      atomicAdd(&f.nevals[0], (unsigned long long)nev);
-      atomicAdd(&f.nevals[1], (unsigned long long)P);
-    }
+    add_counts(f, nev, (unsigned)P);
   }
 }
 

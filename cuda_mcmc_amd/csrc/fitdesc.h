@@ -46,6 +46,18 @@ constexpr int QROW_MAXEQ = 8;
 constexpr int QROW_TS(int n) { return (n + 2) * QROW_MAXEQ + 4; }
 constexpr int QROW_FLOATS(int n) { return n * QROW_TS(n) + QROW_MAXEQ; }
 
+// Copies of a fit's counters.  Each wave adds its counts once per launch, and
+// additions to one address from all over the chip take place one after the
+// other, 12.5 ns each.  So a fit whose launches have many waves has several
+// copies, each in a 128-byte line of its own; work-group b adds to copy
+// b % ncount.  The additions of COUNT_WAVES waves (1.6 us) end before a
+// launch does.  us an iteration with one copy / with these: model.cuh
+// chains of one datum on 8 lanes, 70 rungs x 8192 sequences (71680 waves) 1783 /
+// 326, x 1024 300 / 102; 2000 visibilities + 600 closures, 4096 chains 158.6 / 144.5.
+constexpr int COUNT_LINE = 128 / (int)sizeof(unsigned long long);
+constexpr int COUNT_WAVES = 64;
+constexpr int COUNT_MAX = 256;
+
 struct FitDesc {
   // ---- sizes and options
   int model;          // ModelKind
@@ -135,7 +147,9 @@ struct FitDesc {
   CCalcModel* mc;                // device CCalcModel for the user's model()
 
   // ---- counters
-  unsigned long long* nevals;    // [2]: performed chi^2 evaluations, proposals
+  unsigned long long* nevals;    // [ncount][COUNT_LINE]: performed chi^2 evaluations and proposals
+                                 // (the sums over the ncount copies)
+  int ncount;                    // copies of the counters (a power of two)
   int* errflag;                  // first negative model() return code
 };
 
