@@ -68,9 +68,9 @@ __device__ inline double swap_factor(const FitDesc& f, int k) {
   return k < f.nbeta - 1 ? -0.5 * ((double)gptr(f.beta)[k + 1] - (double)gptr(f.beta)[k]) : 0.0;
 }
 
-// Adds to the work-group's copy of the fit's counters; one lane of a wave calls it.
+// Adds to the work-group's copy of the fit's counters (every session has
+// them); one lane of a wave calls it.
 __device__ inline void add_counts(const FitDesc& f, unsigned nev, unsigned nprop) {
-  if (!f.nevals) return;
   unsigned long long* c = f.nevals + (size_t)(blockIdx.x & (unsigned)(f.ncount - 1)) * COUNT_LINE;
   atomicAdd(&c[0], (unsigned long long)nev);
   atomicAdd(&c[1], (unsigned long long)nprop);
