@@ -1020,8 +1020,8 @@ __global__ void __launch_bounds__(256) k_eval_quad(const FitDesc* fits, const Wo
 // and nadj + n_cnt % nadj from there on, which goes on by one addition and one
 // wrap.  In the wave's LDS, [NQ][64] each, column = lane: the step sizes, the
 // current acceptance-history words (the word that holds entry n_cnt % nadj),
-// and the launch's burn-in proposals and accepted proposals of each parameter
-// in 16 bits each.  Lanes pick different parameters, so per-proposal accesses in
+// and the launch's burn-in proposals, accepted proposals and changed history
+// entries of each parameter in one word.  Lanes pick different parameters, so per-proposal accesses in
 // memory scatter over rows, each lane a cache line of its own; held for the
 // launch, every array moves once per launch instead.  What a lane only adds to
 // (ndone) is no register array: picking the element takes selects, and held in
@@ -1035,14 +1035,15 @@ struct QuadCarry {
   int sh[CACHE ? NQ : 1];
   float* sp;
   uint32_t* hw;
-  uint32_t* ndone;   // proposals << 16 | accepted
+  uint32_t* ndone;   // accepted proposals, proposals, changes of the history word, 10 bits each
   const float* beta;   // per lane
   const float4* par;   // per parameter k: ivar[k], its pdescr (as bits), pmint and pmaxt
   // the last proposal's accept flag, parameter and old value
   int flag, tlast;
   float told;
 };
-static_assert(SEQ_ITERS * 8 <= 65535, "a launch's proposals of one parameter fit 16 bits");
+constexpr uint32_t DONE_PROPOSAL = 1u << 10, DONE_CHANGE = 1u << 20, DONE_MASK = 0x3ffu;
+static_assert(SEQ_ITERS * 8 <= (int)DONE_MASK, "a launch's proposals of one parameter fit 10 bits");
 
 // n_cnt % nadj from QuadCarry::ent.
 __device__ inline uint32_t hist_entry(uint32_t ent, int nadj) {
@@ -1073,22 +1074,35 @@ __device__ inline void quad_load(const FitDesc& f, int ch, bool hist, QuadCarry<
       if (i < P) q.hw[i * 64 + ln] = gptr(f.hbits)[(ch * f.hwords + (int)(hist_entry(q.ent[i], f.nadj) >> 5)) * P + i];
   }
 }
-// Acceptance counts only where a proposal was accepted (a lane left out
-// touches no line).
+// Acceptance counts only where a proposal was accepted, history words only
+// where an entry changed: a lane left out touches no line, and a chain's history is a
+// line of its own.  The counts are read side by side first, so that no store waits
+// for the load behind it.  Both matter where a launch holds one iteration:
+// 512 systems of 8 equations, 16 x 32 chains, burn-in in calls of one
+// iteration, 99 -> 84 us a call (with additions in the L2 instead of the loads: 92).
 template <int NQ>
 __device__ inline void quad_store(const FitDesc& f, int ch, bool hist, const QuadCarry<NQ, true>& q) {
   const int C = f.nchain, P = f.nprm, ln = lane_id();
+  int acpt[NQ], cnt[NQ];   // read side by side, then written
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    if (i < P) {
+      acpt[i] = gptr(f.n_acpt)[i * C + ch];
+      if (hist) cnt[i] = gptr(f.n_cnt)[i * C + ch];
+    }
+  }
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
     if (i < P) {
       const uint32_t nd = q.ndone[i * 64 + ln];
-      const int na = (int)(nd & 0xffffu);
-      if (na) gptr(f.n_acpt)[i * C + ch] += na;
-      if (hist) {
-        gptr(f.n_cnt)[i * C + ch] += (int)(nd >> 16);
+      const int na = (int)(nd & DONE_MASK), np = (int)((nd / DONE_PROPOSAL) & DONE_MASK);
+      if (na) gptr(f.n_acpt)[i * C + ch] = acpt[i] + na;
+      if (hist && np) {
+        gptr(f.n_cnt)[i * C + ch] = cnt[i] + np;
         gptr(f.sumh)[i * C + ch] = q.sh[i];
         gptr(f.pstp)[i * C + ch] = q.sp[i * 64 + ln];
-        gptr(f.hbits)[(ch * f.hwords + (int)(hist_entry(q.ent[i], f.nadj) >> 5)) * P + i] = q.hw[i * 64 + ln];
+        if (nd >= DONE_CHANGE)
+          gptr(f.hbits)[(ch * f.hwords + (int)(hist_entry(q.ent[i], f.nadj) >> 5)) * P + i] = q.hw[i * 64 + ln];
       }
     }
   }
@@ -1226,7 +1240,7 @@ __device__ unsigned quad_substeps(const FitDesc& f, int ch, int it, const TraceB
       const float nsd = rate_below(sh, den, f.adapt_mid, f.adapt_tie) ? step_shrink(sd) : step_grow(sd);
       if (CACHE) {
         q.sp[k * 64 + ln] = nsd;
-        atomicAdd(&q.ndone[k * 64 + ln], 0x10000u);
+        atomicAdd(&q.ndone[k * 64 + ln], acc != hold ? DONE_PROPOSAL + DONE_CHANGE : DONE_PROPOSAL);
         const uint32_t nent = ent + 1 == 2u * (uint32_t)nadj ? (uint32_t)nadj : ent + 1;
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
