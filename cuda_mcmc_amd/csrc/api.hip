@@ -963,10 +963,20 @@ StepLaunch exchange_launch(Session* S, const Group& g, int it_off, int close_k) 
   return L;
 }
 
-// The step launches of group g at offset i of its segment.  Kinds whose
-// launches hold whole sequences run iterations i .. i + n - 1 (n = 0: none,
-// an earlier launch has them).
-int launch_steps(Session* S, const Group& g, int i, int n) {
+// The iterations that a launch of whole sequences at offset i of a segment of K
+// holds: from every SEQ_ITERS-th offset on up to SEQ_ITERS, none at the others.
+int seq_iters(int i, int K) { return i % SEQ_ITERS == 0 ? std::min(SEQ_ITERS, K - i) : 0; }
+
+// Whether group g has step launches at offset i of a segment of K.
+bool has_steps(const Group& g, int i, int K) {
+  for (const KindWork& k : g.kinds)
+    if (!k.fused || seq_iters(i, K) > 0) return true;
+  return false;
+}
+
+// The step launches of group g at offset i of its segment of K iterations.
+int launch_steps(Session* S, const Group& g, int i, int K) {
+  const int n = seq_iters(i, K);
   for (const KindWork& k : g.kinds) {
     StepLaunch L = make_launch(S, g, k, i);
     hipError_t e = hipSuccess;
@@ -995,7 +1005,7 @@ int launch_group_exchange(Session* S, const Group& g, int i) {
 // Offset i of group g's segment of K iterations on its stream: the step
 // launches, then the exchange launch of the sequences that need one.
 int launch_iteration(Session* S, const Group& g, int i, int K) {
-  CHK(launch_steps(S, g, i, i % SEQ_ITERS == 0 ? std::min(SEQ_ITERS, K - i) : 0));
+  CHK(launch_steps(S, g, i, K));
   return launch_group_exchange(S, g, i);
 }
 
@@ -1030,7 +1040,8 @@ int join_groups(Session* S) {
   return MHRE_OK;
 }
 
-// Iterations (in segments of BATCH) with HIP events around every launch, on
+// Iterations (in segments of BATCH, so that launches of whole sequences hold as
+// many iterations as those of run) with HIP events around every launch, on
 // each group's stream: average device time per iteration of a group's step
 // launches and of its exchange launches (the per-iteration ones plus the
 // closing launch of each segment), over groups and iterations (launches of
@@ -1038,7 +1049,7 @@ int join_groups(Session* S) {
 // before the host waits, so the gaps between launches are not counted.
 int time_kernels(Session* S, int niter, double* step_ms, double* exch_ms) {
   (void)hipGetLastError();
-  constexpr int BATCH = 32;
+  constexpr int BATCH = SEQ_ITERS;
   const int G = (int)S->groups.size();
   std::vector<hipEvent_t> ev((size_t)3 * BATCH * G + 2 * G, nullptr);
   for (auto& e : ev) HIPCHK(hipEventCreate(&e));
@@ -1056,8 +1067,10 @@ int time_kernels(Session* S, int niter, double* step_ms, double* exch_ms) {
       for (int gi = 0; gi < G; ++gi) {
         const Group& g = S->groups[gi];
         hipEvent_t* e = &ev[(size_t)3 * (i * G + gi)];
-        HIPCHK(hipEventRecord(e[0], g.stream));
-        CHK(launch_steps(S, g, i, 1));
+        if (has_steps(g, i, nb)) {   // else the time between two events alone would count
+          HIPCHK(hipEventRecord(e[0], g.stream));
+          CHK(launch_steps(S, g, i, nb));
+        }
         HIPCHK(hipEventRecord(e[1], g.stream));
         CHK(launch_group_exchange(S, g, i));
         HIPCHK(hipEventRecord(e[2], g.stream));
@@ -1072,7 +1085,8 @@ int time_kernels(Session* S, int niter, double* step_ms, double* exch_ms) {
     for (int gi = 0; gi < G; ++gi) HIPCHK(hipEventSynchronize(ec[2 * gi + 1]));
     for (int i = 0; i < nb * G; ++i) {
       float a = 0.0f, b = 0.0f;
-      HIPCHK(hipEventElapsedTime(&a, ev[(size_t)3 * i], ev[(size_t)3 * i + 1]));
+      if (has_steps(S->groups[i % G], i / G, nb))
+        HIPCHK(hipEventElapsedTime(&a, ev[(size_t)3 * i], ev[(size_t)3 * i + 1]));
       HIPCHK(hipEventElapsedTime(&b, ev[(size_t)3 * i + 1], ev[(size_t)3 * i + 2]));
       st += a;
       ex += b;

@@ -187,7 +187,8 @@ class Session:
         _lib.check(self.L, self.L.mhre_session_run(self.h, int(niter)), "mhre_session_run")
 
     def time_kernels(self, niter):
-        """Run niter iterations with HIP events around every launch; returns
+        """Run niter iterations with HIP events around every launch (the launches
+        that run() makes of them, many iterations each where it does so); returns
         (step_ms, exchange_ms): one sequence group's step and exchange launch
         durations per iteration (groups overlap, so they do not add up to the
         iteration time, which stats()["run_ms"] gives after run())."""

@@ -165,9 +165,10 @@ typedef struct MhreStats {
 int mhre_session_create(const MhreFitSpec *fits, int nfits, const MhreOptions *opt, void **session);
 /* Run niter MH-RE iterations of every fit (asynchronous to the host). */
 int mhre_session_run(void *session, int niter);
-/* Run niter iterations timing every launch with HIP events on the stream of
- * its sequence group; returns the average device time of one group's step
- * launch(es) per iteration and of its exchange launches per iteration (those
+/* Run niter iterations, in the launches that mhre_session_run makes of them
+ * (kinds whose launches hold whole sequences: up to 64 iterations each), timing
+ * every launch with HIP events on the stream of its sequence group; returns
+ * the average device time of one group's step launch(es) per iteration and of its exchange launches per iteration (those
  * that run every iteration, plus each segment's closing launch spread over
  * the segment's iterations), in milliseconds (the launches of different
  * groups overlap, so these do not add up to the iteration time). */
