@@ -151,7 +151,7 @@ def batched_vs_plain(iters, nfits, log_every=16, session_only=False, streams=2):
         if (f + 1) % log_every == 0:
             log("  generated %d/%d fits" % (f + 1, nfits))
     tune_iters = 2
-    mk = lambda d, nb, ns, f: eht_fit(d, nb, ns, nburn=iters + 2 + 6 * tune_iters, niter=0, seed=300 + f)
+    mk = lambda d, nb, ns, f: eht_fit(d, nb, ns, nburn=iters + 2 + 7 * tune_iters, niter=0, seed=300 + f)
     total_vis = 0.0
     with Session([mk(d, nb, ns, f) for f, (d, nb, ns) in enumerate(fits)], persistent=0, streams=streams) as s:
         s.run(1)

@@ -728,7 +728,8 @@ struct Session {
   std::vector<Group> groups;
   MhreOptions opt{};
   int wpb = 4, persistent = 0, grid = 0, ncu = 1;
-  bool split = false;   // ring+Gaussian kinds of few chains run in the split form (KindWork::split)
+  bool split_ok = false;   // the options leave the split form (KindWork::split) to the session
+  bool split = false;      // its kinds that can be split are
   int waves_per_simd = 0, lds_per_cu = 0;   // occupancy cap of the native step launches
   int graph_iters = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1133,23 +1134,25 @@ int time_iterations(Session* S, int niter, double* ms) {
 
 // Picks the launch form of the wave-per-chain step kernels by timing real
 // iterations (they advance the chains like any other iteration): each
-// (waves per work-group, grid or persistent) candidate runs `iters`
-// iterations of every group and the one with the shortest device time per
-// iteration stays.  All forms give bit-identical chains.  A captured graph is
-// dropped and re-captured later.
+// (waves per work-group, grid or persistent) candidate, and in sessions whose
+// chains can be split over waves that form too, runs `iters` iterations of
+// every group and the one with the shortest device time per iteration stays.
+// All forms give bit-identical chains.  A captured graph is dropped and
+// re-captured later.  The pair returned is the fastest of the six forms that
+// it can name, also where the session stays with the split form.
 int autotune(Session* S, int iters, int* best_wpb, int* best_persistent, double* best_ms) {
   static const int cand[6][2] = {{4, 0}, {2, 0}, {1, 0}, {4, 1}, {2, 1}, {1, 1}};
   if (iters <= 0) FAIL(MHRE_EINVAL, "autotune: iters must be positive");
+  auto set_form = [&](int wpb, int persistent, bool split) {
+    S->wpb = wpb;
+    S->persistent = persistent;
+    S->split = split;
+    S->grid = std::max(1, S->ncu * (16 / S->wpb));
+  };
   double best = 1e300;
   int bw = S->wpb, bp = S->persistent;
-  // a session that splits its chains over waves does so in place of the first
-  // candidate, whose work-groups are the widest too
-  const bool split = S->split;
   for (const auto& c : cand) {
-    S->wpb = c[0];
-    S->persistent = c[1];
-    S->split = split && c[0] == 4 && c[1] == 0;
-    S->grid = std::max(1, S->ncu * (16 / S->wpb));
+    set_form(c[0], c[1], false);
     double t = 0.0;
     CHK(time_iterations(S, iters, &t));
     if (t < best) {
@@ -1158,10 +1161,20 @@ int autotune(Session* S, int iters, int* best_wpb, int* best_persistent, double*
       bp = c[1];
     }
   }
-  S->wpb = bw;
-  S->persistent = bp;
-  S->split = split && bw == 4 && bp == 0;
-  S->grid = std::max(1, S->ncu * (16 / S->wpb));
+  bool can_split = false;
+  for (const Group& g : S->groups)
+    for (const KindWork& k : g.kinds) can_split = can_split || (S->split_ok && k.split > 1);
+  bool split = false;
+  if (can_split) {
+    set_form(4, 0, true);   // of kinds that are not split
+    double t = 0.0;
+    CHK(time_iterations(S, iters, &t));
+    if (t < best) {
+      best = t;
+      split = true;
+    }
+  }
+  if (!split) set_form(bw, bp, false);
   drop_graph(S);
   if (best_wpb) *best_wpb = bw;
   if (best_persistent) *best_persistent = bp;
@@ -1204,7 +1217,7 @@ int create(const MhreFitSpec* specs, int nfits, const MhreOptions* opt, Session*
   S->persistent = S->opt.persistent > 0 ? 1 : 0;
   S->waves_per_simd = std::max(0, S->opt.waves_per_simd);
   // a launch form that the caller names is the one that runs
-  S->split = S->opt.waves_per_block == 0 && !S->persistent && S->waves_per_simd == 0;
+  S->split = S->split_ok = S->opt.waves_per_block == 0 && !S->persistent && S->waves_per_simd == 0;
 
   const int it0 = specs[0].it0;
   S->fits.resize(nfits);

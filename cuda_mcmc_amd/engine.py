@@ -199,7 +199,12 @@ class Session:
 
     def autotune(self, iters=8):
         """Pick the step kernels' launch form by timing 6 candidates for `iters`
-        real iterations each; returns (waves_per_block, persistent, step_ms)."""
+        real iterations each, and as a 7th, in a session that may split its
+        chains over waves (fit_info's chain_split), that form; returns
+        (waves_per_block, persistent, step_ms): the fastest of the 6, and the
+        step time of the form that the session stays with (chain_split above 1:
+        the split form, which a session without waves_per_block and persistent
+        takes by itself)."""
         w, p, t = C.c_int(), C.c_int(), C.c_double()
         _lib.check(self.L, self.L.mhre_session_autotune(self.h, int(iters), C.byref(w), C.byref(p), C.byref(t)),
                    "mhre_session_autotune")

@@ -176,8 +176,13 @@ int mhre_session_time_kernels(void *session, int niter, double *step_ms, double 
 /* Choose the step kernels' launch form (waves per work-group 1/2/4, grid or
  * persistent work queue) by timing each candidate on `iters` real
  * iterations; the 6 * iters iterations advance the chains like any others
- * (every form gives bit-identical chains).  Returns the choice and its step
- * time per iteration.  No reference counterpart. */
+ * (every form gives bit-identical chains).  A session that may split its chains
+ * over waves (info[5] of mhre_session_fit_info above 1 for a ring+Gaussian
+ * fit) times that form as a seventh, so 7 * iters iterations.  Returns the
+ * fastest of the six forms, which a later session can be given, and the step
+ * time per iteration of the form that this session stays with: that one, or the
+ * split form (info[5] still above 1), which a later session takes by itself
+ * with waves_per_block = 0 and no persistent queue.  No reference counterpart. */
 int mhre_session_autotune(void *session, int iters, int *waves_per_block, int *persistent,
                           double *step_ms);
 /* Wait for the session's stream. */

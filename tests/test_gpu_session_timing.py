@@ -4,6 +4,9 @@
   also where a launch holds whole sequences for many iterations, is a part of
   run's device time per iteration (1.25 times it for the events between the
   launches), and the iterations advance the chains as run's do.
+* autotune times the six launch forms that it can name, and the split form as
+  a seventh where a session may take it, each time it is called; the form
+  that it returns is one that a session can be given.
 """
 import os
 
@@ -65,3 +68,38 @@ def test_time_kernels_advances_the_chains(streams):
     for a, b in zip(run([(False, 140)]), run([(True, 1), (True, 64), (False, 5), (True, 70)])):
         for k in ("pcur", "chi2c", "pstp", "n_cnt", "n_acpt", "n_hist", "n_exch", "tcur"):
             np.testing.assert_array_equal(getattr(a, k), getattr(b, k), err_msg=k)
+
+
+@pytest.mark.parametrize("opt,candidates", [({}, 7), (dict(streams=3), 7), (dict(waves_per_block=2), 6),
+                                            (dict(persistent=1), 6), (dict(waves_per_simd=2), 6)])
+def test_autotune_candidates(opt, candidates):
+    ref, got, again = _eht()[0], _eht()[0], _eht()[0]
+    with Session([ref]) as s:
+        assert s.fit_info(0)["chain_split"] > 1
+        s.run(4 * candidates + 5)
+        s.download()
+    with Session([got], **opt) as s:
+        before = s.fit_info(0)["chain_split"]
+        assert (before > 1) == (candidates == 7)
+        for n in (1, 2):
+            w, p, t = s.autotune(2)
+            assert w in (1, 2, 4) and p in (0, 1) and t > 0
+            assert s.stats()["iters_done"] == 2 * candidates * n
+            assert s.fit_info(0)["chain_split"] in (1, before)
+        s.run(5)
+        s.download()
+    with Session([again], waves_per_block=w, persistent=p) as s:   # the named form, not the split one
+        assert s.fit_info(0)["chain_split"] == 1
+        s.run(4 * candidates + 5)
+        s.download()
+    for k in ("pcur", "chi2c", "pstp", "n_cnt", "n_acpt", "n_hist", "n_exch", "tcur"):
+        np.testing.assert_array_equal(getattr(ref, k), getattr(got, k), err_msg=k)
+        np.testing.assert_array_equal(getattr(ref, k), getattr(again, k), err_msg=k)
+
+
+def test_autotune_where_nothing_can_be_split():
+    small = [eht_fit(synthdata.ring_gauss_dataset(nvis=128, ncph=0, seed=9), 4, 4, nburn=60, niter=60, seed=1,
+                     record=False)]
+    with Session(small) as s:
+        s.autotune(2)
+        assert s.stats()["iters_done"] == 12
