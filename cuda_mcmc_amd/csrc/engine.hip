@@ -425,14 +425,12 @@ struct WaveChi2 {
 // order, in fp32 over the blocks of 8 tiles (padded with zero terms to a
 // multiple of 8) and then in fp64, so that the chi^2 has the bits of
 // eht_chi2_wave.  Wave 0 adds them all, or beyond SPLIT_TRIPS blocks every
-// wave its share of the blocks (the fp64 sums are then added in another order,
-// which the chi^2, rounded to fp32, does not show).
+// wave adds up its share of the blocks and wave 0 the blocks' sums.
 constexpr int SPLIT_TRIPS = 2;
 constexpr int SPLIT_MAXW = 8;
 template <class M>
 struct SplitLds {
   typename M::Inv q;
-  double xs[SPLIT_MAXW];
   int go;   // 1: model q, 0: the iteration is over
 };
 template <class M>
@@ -564,7 +562,7 @@ struct SplitChi2 {
       __syncthreads();
     }
     const int ntrip = (nt + 7) / 8;
-    const bool all = ntrip > SPLIT_TRIPS;   // every wave adds its blocks
+    const bool all = ntrip > SPLIT_TRIPS;   // every wave adds up its blocks
     double acc = 0.0;
     if (all || wid == 0) {
       for (int k = all ? wid : 0; k < ntrip; k += all ? W : 1) {
@@ -577,15 +575,18 @@ struct SplitChi2 {
 #pragma unroll
           for (int i = 0; i < 8; ++i) part = fmaf(f[i].x, f[i].y, part);
         }
+        // a lane's sum of the block: the visibilities are not read again
+        // before the next proposal's
+        if (all) reinterpret_cast<float*>(vis)[k * TILE + lane] = part;
         acc += (double)part;
       }
+      if (all) {
+        __syncthreads();
+        acc = 0.0;
+        if (wid == 0)
+          for (int k = 0; k < ntrip; ++k) acc += (double)reinterpret_cast<float*>(vis)[k * TILE + lane];
+      }
       acc = wave_sum(acc);
-    }
-    if (all) {
-      if (lane == 0) sh.xs[wid] = acc;
-      __syncthreads();
-      acc = 0.0;
-      for (int w = 0; w < W; ++w) acc += sh.xs[w];
     }
     return acc;
   }
