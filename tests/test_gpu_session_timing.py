@@ -7,6 +7,8 @@
 * autotune times the six launch forms that it can name, and the split form as
   a seventh where a session may take it, each time it is called; the form
   that it returns is one that a session can be given.
+* Under a cap on resident waves the exchange launches of one sequence group run
+  beside the step launch of another.
 """
 import os
 
@@ -103,3 +105,24 @@ def test_autotune_where_nothing_can_be_split():
     with Session(small) as s:
         s.autotune(2)
         assert s.stats()["iters_done"] == 12
+
+
+def test_exchange_launches_run_beside_a_capped_step_launch():
+    """100 rungs x 40 sequences at 2 waves per SIMD: each of two groups has 2000
+    waves of the 2048 that may be resident, so its exchange launch (of ladders
+    over 64 rungs, on one lane) costs no time if it runs under the other
+    group's step launch; one group has two rounds of waves and its exchange
+    after them.  The exchange is about a quarter of the iteration: less than 0.9
+    of one group's time if it is hidden, all of it if it waits."""
+    d = synthdata.ring_gauss_dataset(nvis=2000, ncph=600, seed=3)
+    t = {}
+    for streams in (1, 2):
+        f = eht_fit(d, 100, 40, nburn=4000, niter=0, seed=1, record=False)
+        with Session([f], waves_per_simd=2, streams=streams) as s:
+            s.run(32)
+            t[streams] = 1e30
+            for _ in range(4):
+                s.run(32)
+                s.sync()
+                t[streams] = min(t[streams], s.stats()["run_ms"])
+    assert t[2] <= 0.9 * t[1], t
