@@ -551,20 +551,25 @@ int count_copies(const FitHost& h) {
 }
 
 // Waves per chain of the ring+Gaussian fits `idx` of a session: 1 (the grid or
-// persistent form), or 4 or 8 (the split form, k_step_eht_split) for sessions
-// whose chains are few enough that a work-group each is resident on the chip
-// at once, or in two rounds where there is enough to share.  Of 4 and 8 the
-// one with fewer rounds, then the wider.  Measured, us an iteration with 1 / 4
-// / 8 waves per chain, 9 parameters, ladders of 32 rungs:
-//   323 visibilities + 319 closures:  512 chains 47.1 / 32.3 / 29.2,
-//     1024: 52.5 / 40.1 / 48.3, 2048: 65.8 / 61.7 / 96.4
-//   2000 + 600:  512: 110.8 / 51.8 / 43.1, 1024: 113 / 94.4 / 78.1, 2048: 125.7 / 187 / 155
-//   1000 + 300, 2048: 85.5 / 74.5 / 111;  192, 512: 27.3 / 27.3 / 27.7;  256: 29.3 / 28.0 / 27.9
-// With 13 parameters, 323 + 319, 2048 chains: 87.1 / 89.0 / 144, hence two
-// rounds only from SPLIT_TWO_ROUNDS terms per lane on.
+// persistent form), or 4 or 8 (the split form, k_step_eht_split) for sessions of
+// few chains.  A compute unit holds two work-groups of 8 waves (its
+// registers allow 4 waves per SIMD), or four of 4 where their LDS allows; the
+// times go up in steps of two work-groups per unit.  us an iteration with 1 / 4 / 8
+// waves, 9 parameters, ladders of 32 rungs, by chains per unit:
+//                                    2                  4                  6                  8
+//   256 visibilities (4 terms)       28.8/23.2/23.3     29.5/25.1/40.5     29.7/34.6/59.6     29.7/42.9/78.4
+//   500 + 150 closures (11)          41.1/28.8/27.2     41.5/31.7/48.0     41.6/43.3/70.9     41.5/54.6/94.2
+//   323 + 319 (16)                   50.3/32.9/29.3     50.5/36.1/51.7     50.4/49.9/76.3     50.2/62.6/101
+//   1000 + 300 (23)                  65.9/37.3/33.0     66.7/42.5/59.0     66.6/59.8/87.6     66.3/74.7/116
+//   1700 + 500 (38)                  98.5/47.4/39.5     99.4/66.3/70.6     99.7/91.0/106      98.6/121/140
+//   2000 + 600 (45)                  112/51.8/42.3      113/93.8/76.8      113/139/114        112/185/152
+// (13 parameters: 323 + 319 75.8/49.6/44.8, 76.4/54.4/78.2, 76.8/75.3/116, 76.4/93.8/154.)
+// So 8 waves up to two chains per unit; 4 waves up to four, or six where a lane
+// has at least SPLIT_MANY_TERMS terms; with LDS for only two work-groups (2000 +
+// 600) 8 waves up to four.  Below SPLIT_MIN_TERMS it depends: 192 visibilities
+// 26.9/23.3/23.2, but 100 + 60 25.7/26.5/43.6 at four, and 64 lose.
 constexpr int SPLIT_LDS = 52 << 10;
-constexpr int SPLIT_MIN_TERMS = 4, SPLIT_TWO_ROUNDS = 16;
-constexpr int SPLIT_WAVES_PER_CU = 16;   // its registers allow 4 waves per SIMD
+constexpr int SPLIT_MIN_TERMS = 4, SPLIT_MANY_TERMS = 16;
 
 int eht_split_waves(const std::vector<FitHost>& fits, const std::vector<int>& idx, int ncu, int lds_per_cu) {
   long long chains = 0;
@@ -580,18 +585,11 @@ int eht_split_waves(const std::vector<FitHost>& fits, const std::vector<int>& id
     terms = std::max(terms, h.ntile + np);
   }
   const int lds = eht_split_lds(nt, ne);
-  if (lds > SPLIT_LDS || terms < SPLIT_MIN_TERMS) return 1;
-  int best = 1;
-  long long best_rounds = terms >= SPLIT_TWO_ROUNDS ? 2 : 1;
-  for (int w : {4, 8}) {
-    const long long at_once = (long long)ncu * std::min(lds_per_cu / (lds + EHT_SPLIT_STATIC_LDS), SPLIT_WAVES_PER_CU / w);
-    const long long rounds = at_once > 0 ? (chains + at_once - 1) / at_once : 1000;
-    if (rounds <= best_rounds) {
-      best = w;
-      best_rounds = rounds;
-    }
-  }
-  return best;
+  const int per_cu = lds_per_cu / (lds + EHT_SPLIT_STATIC_LDS);   // work-groups, by LDS
+  if (lds > SPLIT_LDS || terms < SPLIT_MIN_TERMS || per_cu < 2) return 1;
+  if (chains <= 2ll * ncu) return 8;
+  if (per_cu == 2) return chains <= 4ll * ncu ? 8 : 1;
+  return chains <= (terms >= SPLIT_MANY_TERMS ? 6ll : 4ll) * ncu ? 4 : 1;
 }
 
 // Most concurrent sequence groups (streams) of a session.

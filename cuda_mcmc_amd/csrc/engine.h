@@ -130,7 +130,7 @@ hipError_t launch_eval_eht(int model, const FitDesc* fits, const WorkItem* work,
 hipError_t launch_step_eht(int model, const StepLaunch& L, hipStream_t s);
 // LDS of the split step form's model visibilities and term factors.
 constexpr int eht_split_lds(int ntile, int nentry) { return (ntile + nentry) * TILE * (int)sizeof(float2); }
-constexpr int EHT_SPLIT_STATIC_LDS = 12 << 10;   // bound of its other LDS (Bessel table, prologue)
+constexpr int EHT_SPLIT_STATIC_LDS = 11 << 10;   // bound of its other LDS (Bessel table, prologue)
 hipError_t launch_eval_quad(int n, const FitDesc* fits, const WorkItem* work, int nwork, hipStream_t s);
 hipError_t launch_step_quad(int n, const StepLaunch& L, hipStream_t s);
 // L.iters iterations (step + exchange) of whole sequences (ladders of at most
