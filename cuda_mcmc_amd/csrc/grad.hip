@@ -730,8 +730,14 @@ __global__ void __launch_bounds__(512) k_eht_gn9(GradArgs g) {
   }
 }
 
-// Waves per point: as many as keep the launch within GRAD_WAVES, 4 per SIMD.
-constexpr int GRAD_WAVES = 4096;
+// Waves per point: as many as are on the chip at once (256 registers: 2 waves
+// per SIMD, so one work-group of 8 waves per compute unit).  us a call with 1 / 2 / 4 / 8:
+//                       256 points             512                    1024                   2048
+//   323 vis. + 319 clo. 26.4/18.8/16.0/14.1    29.1/22.3/18.6/24.6    32.2/24.6/34.1/44.4    38.7/45.6/61.7/85.7
+//   2000 + 600          55.8/34.7/24.8/21.1    59.1/43.9/29.8/38.2    65.8/47.1/53.9/73.0    83.0/104/104/145
+//   20000 + 6000        445/245/137/94.6       471/323/176/183        523/342/338/362        672/808/650/721
+// and from 4096 points on one wave, 72 us at 323 + 319, 159 at 2000 + 600.
+constexpr int GRAD_WAVES = 2048;
 static int waves_per_point(int n) {
   int w = GRAD_MAXW;
   while (w > 1 && (long long)n * w > GRAD_WAVES) w >>= 1;
