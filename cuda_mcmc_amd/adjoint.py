@@ -98,7 +98,12 @@ class EhtData:
         return P.shape[0], P.shape[1]
 
     def chi2_grad(self, P, need_grad=True):
-        """chi^2 [n] (float64) and, if need_grad, d chi^2/dP [n, nptot] (float32)."""
+        """chi^2 [n] (float64) and, if need_grad, d chi^2/dP [n, nptot] (float32).
+
+        Few points share a point's data among several waves, which adds the same
+        terms in another order: a point's values depend, in the last bits, on
+        how many points the call holds (chi^2 within 1e-6, the gradient within
+        1e-5 of its norm)."""
         n, ldp = self._rows(P)
         chi = torch.empty(n, dtype=torch.float64, device=P.device)
         grad = torch.empty((n, ldp), dtype=torch.float32, device=P.device) if need_grad else None

@@ -504,17 +504,18 @@ bool eht_xfused(const FitHost& h, const MhreOptions& o) {
 // gives a chain up to 256 lanes: as many as it has data, but no more waves
 // than fill the chip several times over (a wave of fewer chains repeats their
 // bookkeeping on more lanes).  Measured, us an iteration with k_step_user +
-// k_exchange / k_iter_user:
+// k_exchange / k_iter_user (runs of 64 and 32 iterations):
 //   a valley of two parameters, ladders of 32 rungs (2 lanes a chain), 64
-//     sequences: 2 data 16.2 / 4.1, 4: 15.9 / 5.5, 8: 15.9 / 7.4, 32: 31.5 / 18.6;
-//     512 sequences, 8 data: 60.6 / 7.7
+//     sequences: 2 data 15.6 / 5.7, 4: 15.5 / 6.5, 8: 15.4 / 6.8, 32: 16.7 / 9.7;
+//     512 sequences, 8 data: 17.8 / 7.3
 //   the 9-parameter ring+Gaussian as model(), 8 rungs (8 lanes) x 32: 8 data
-//     37.3 / 25.6, 16: 37.2 / 43.9, 28: 39.7 / 78.2; 32 rungs x 32: 8 data 38.9 / 85.0
+//     42.8 / 30.0, 16: 42.4 / 48.5, 28: 44.6 / 82.9; 32 rungs x 32: 8 data 44.9 / 88.9
 // What a model() costs is not known here: four data a lane is where a cheap one
 // still gains twofold and an expensive one loses as much.
 // Waves of k_step_user, 1024 / 2048 / 4096 / 8192 / 16384 at most, the
-// ring+Gaussian, 32 rungs x 128 sequences: 500 visibilities 713 / 398 / 301 / 254
-// / 271, 2000: 2966 / 1561 / 1216 / 954 / 898.
+// ring+Gaussian, 32 rungs x 128 sequences: 500 visibilities 728 / 418 / 310 / 269
+// / 291, 2000: 2990 / 1573 / 1223 / 976 / 926; 70 rungs x 64, 100 + 30 data: 434 /
+// 295 / 239 / 225 / 226; 32 x 512, 100 + 30: 428 / 422 / 349 / 399 / 495.
 constexpr int USER_SEQ_DATA = 4;
 constexpr long long USER_WAVES = 8192;
 constexpr int USER_SEQ_LDS = 32 << 10;
@@ -1883,8 +1884,8 @@ struct EhtData {
 // Waves per point of a gradient call of n points: 1 (a wave per point), or a
 // work-group of 4, 8 or 16 while all points' work-groups are on the chip at
 // once, or of at least 8 in two rounds; 16 only where each wave still has two
-// tiles.  Measured, one wave per point -> split, us a call, 2000 visibilities +
-// 600 closures: 1 to 128 points 47 -> 15, 512: 48 -> 19, 1024: 50 -> 30, but
+// tiles.  Kernel time, one wave per point -> split, us, 2000 visibilities + 600
+// closures (a call through autograd takes about 85 us either way, 84 at 32 points): 1 to 128 points 47 -> 15, 512: 48 -> 19, 1024: 50 -> 30, but
 // 2048 (two rounds of 4 waves) 56 -> 80; 10000 + 3000: 1 point 198 -> 28, 256:
 // 206 -> 33, 257 (two rounds): 206 -> 63.
 int grad_split_waves(const EhtData* E, int n) {

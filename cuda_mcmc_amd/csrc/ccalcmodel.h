@@ -10,6 +10,11 @@
 //   ipass  0 .. npass-1
 // where ist = nseq * ibeta + iseq.  Return 0 = no result for this datum,
 // 1 = value, 2 = angle (the residual is wrapped), -1 = error.
+// As in the reference, whose data of one pass are threads of one launch
+// (src/gpu_mcmc.cu:754), the data of a pass run side by side in no order: a
+// model reads what an earlier pass stored in datm, never what another datum
+// stores in the same pass.  mc is the caller's copy: the arrays it points to
+// are shared, a field that model() writes is not kept.
 #pragma once
 
 class CCalcModel {

@@ -29,14 +29,9 @@ __device__ inline int value_again(int v) {
   asm volatile("" : "+v"(v));
   return v;
 }
-__device__ inline float value_again(float v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
 #else
 __device__ inline const FitDesc& fit_again(const FitDesc& f) { return f; }
 __device__ inline int value_again(int v) { return v; }
-__device__ inline float value_again(float v) { return v; }
 #endif
 
 // Step launches: the first thread of the grid hands the segment's first

@@ -1585,7 +1585,9 @@ __device__ void iter_quad_wave(const FitDesc& f0, int iseq0, int it0, int it1, c
 
 // The rows form keeps every equation's residual in registers: 4 waves per
 // SIMD; the full form 5 (with one wave more each, both spill inside the
-// proposals).  What bounds it is FP32 issue.  512 systems of 8 equations, 16 x 32
+// proposals).  As it is, 8 parameters keep up to 45 registers of an iteration's
+// constants (the float64 logarithm's above all) in 172 bytes of scratch a lane,
+// written once a launch and read once an iteration.  What bounds it is FP32 issue.  512 systems of 8 equations, 16 x 32
 // chains, an iteration per launch against 64: sampling 37.2 -> 28.1 us an
 // iteration, burn-in (whose per-proposal history and counter accesses kept it
 // waiting on memory) 58.0 -> 35.8 us; with the parameters' constants and the

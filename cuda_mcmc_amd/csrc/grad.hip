@@ -499,7 +499,7 @@ __global__ void __launch_bounds__(256) k_eht_grad9_ring(GradArgs g) {
 // are formed 64 a wave, each leaving its s = -2 dd w; and tile by tile each
 // visibility gathers S_j from the closures that contain it (FitDesc::vcl, so
 // no two lanes add to one place) and runs its reverse pass.
-// 32 points against 2000 visibilities + 600 closures: 47.4 -> 14.9 us.
+// 32 points against 2000 visibilities + 600 closures: kernel time 47.4 -> 14.2 us.
 template <bool GRAD>
 __global__ void __launch_bounds__(64 * GRAD_SPLIT_MAXW) k_eht_grad9_split(GradArgs g) {
   extern __shared__ __align__(16) char lds[];
@@ -645,9 +645,10 @@ __device__ inline void gn_accumulate(const float* rinv, float r, const double* j
 // J^T J and J^T r of one point a work-group, its data shared by the
 // work-group's 1 to GRAD_MAXW waves (the launch takes as many as few points
 // leave the chip idle).  Bound by float64 arithmetic: per datum 35 products
-// for the row (the nonzero entries of J_inv) and 55 for the sums.
-// 16 points against 2000 visibilities + 600 closures: 88.9 us with one wave a
-// point and all 126 products of the row, 12 now.
+// for the row (the nonzero entries of J_inv) and 55 for the sums, whose 64
+// totals a lane take half of the 256 registers that two waves per SIMD leave
+// (40 more are spilled).  2000 visibilities + 600 closures, with one wave a
+// point and all 126 products of the row -> now: 16 points 79 -> 19 us, 4096 320 -> 159.
 __global__ void __launch_bounds__(512) k_eht_gn9(GradArgs g) {
   __shared__ double jac[NINV * NP9];
   __shared__ double part[GRAD_MAXW][64];

@@ -238,7 +238,9 @@ int mhre_eht_data_create(const float *coor, const float *dat, const float *std2r
  * parameter vectors params[n][ldp] (9 <= ldp <= 32; entries past 9 get 0).
  * Data whose closures lie within the 512-visibility ring window use the
  * single-pass ring kernel; the environment variable MHRE_GRAD_RING=0 selects
- * the per-closure kernel instead (same results to float rounding). */
+ * the per-closure kernel instead (same results to float rounding).  Calls of
+ * few points share a point's data among several waves (the same terms in
+ * another order): a point's last bits depend on n. */
 int mhre_eht_chi2_grad(void *handle, const float *params, int n, int ldp,
                        double *chi2, float *grad, void *stream);
 /* Gauss-Newton normal equations of the weighted residuals r (amplitudes:
